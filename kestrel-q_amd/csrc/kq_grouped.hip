@@ -1157,624 +1157,14 @@ hipError_t pass_any(uint32_t type, uint32_t kdim, const uint8_t *W0, const uint8
 }
 
 /* ------------------------------------------------------------------ */
-/* Batched Q6_K matvec on MFMA: y[b] = W x[b] for 2 .. 4 activation columns
- *
- * The row engine keeps every lane's activations in registers, 32 per batch
- * column; at 4 columns that leaves no room for the weights in flight. Here
- * the columns ride on the token dimension of 16x16x32 matrix steps: they are
- * staged once per workgroup as fp16 hi + lo after an exact power-of-two
- * scaling (an LDS image of kMvCols rows). The four columns' hi and lo parts
- * fill 8 token rows, so one step carries two 16-column sub-blocks of the
- * block: token rows 0..7 hold the first sub-block's activations on k 0..15
- * (zeros on k 16..31) and rows 8..15 the second's on k 16..31. Each product
- * row then belongs to one sub-block, and lane l keeps row l % 16 of a
- * 16-row tile for the four token rows 4 (l / 16) .. + 3: its sub-block's
- * scale applies to all four.
- *
- * Weights: the MFMA operand wants scattered 4-byte pieces of a block per
- * lane, which as global loads would touch 16 rows per instruction. So each
- * wave streams one block of its tile's 16 rows at a time (16 windows of 224
- * bytes from the block's aligned start) with four LDS-DMA loads straight
- * into a ring of NS private LDS slots, NS - 1 blocks ahead of the one it
- * multiplies, and reads the operand pieces from there. Eight waves with a
- * four-slot ring fill the LDS beside the activation image at 2,048 columns;
- * on the 151936 x 2048 LM head at 4 columns this was faster than 4, 6, 10,
- * 12 or 16 waves with the rings that fit them (92.7, 84.2, 77.6, 81.3 and
- * 82.1 us against 70.9-75.6 us). The per-row fp32 sums are compared with
- * the CPU by tolerance; the argmax partials (largest value, lowest row on
- * ties) are exact over them. */
-
-constexpr uint32_t kMvCols = 4;      /* staged activation columns */
-constexpr int kMvWaves = 8;          /* waves per workgroup */
-constexpr uint32_t kMvMaxK = 4096u;
-constexpr uint32_t kMvWin = 224u;    /* bytes of a row's block window (>= 210 + 2) */
-constexpr uint32_t kMvPitch = 240u;  /* slot row pitch: lanes (j, g) hit distinct banks */
+/* one 256-column Q6_K block of 16 rows in LDS: 224-byte windows (a block
+ * from its 4-byte aligned start) at a 240-byte pitch, so lanes (row, k-group)
+ * hit distinct banks */
+constexpr uint32_t kMvWin = 224u;
+constexpr uint32_t kMvPitch = 240u;
 constexpr uint32_t kMvSlot = kTile * kMvPitch;
-constexpr uint32_t kMvUnits = kTile * (kMvWin / 16u); /* 16-byte loads per block: 224 */
+constexpr uint32_t kMvUnits = kTile * (kMvWin / 16u);   /* 16-byte loads per block: 224 */
 constexpr int kMvLoads = (int)((kMvUnits + 63u) / 64u); /* per lane: 4 */
-constexpr uint32_t kMvUnitsPerRow = kMvPitch / 16u; /* 15: 14 window units + 1 gap */
-constexpr int kMvDma = (int)((kMvSlot / 16u + 63u) / 64u); /* DMA loads per block: 4 */
-constexpr uint32_t kMvZero = 256u; /* fp16 zeros: k 8 g + 128 n + 32 q .. + 7 < 256 */
-constexpr uint32_t kMvLdsMax = 160u * 1024u;
-constexpr uint32_t kMvMaxSlots = 4u; /* block slots per wave, at most */
-
-__device__ __forceinline__ void mv_argmax_merge(float &bv, uint32_t &bi, float v, uint32_t i) {
-    if (v > bv || (v == bv && i < bi)) {
-        bv = v;
-        bi = i;
-    }
-}
-
-/* x image pitch in fp16 (a 32-byte skew per column keeps the 16 operand
- * reads of a step on distinct banks) */
-__host__ __device__ __forceinline__ uint32_t mv_xpitch(uint32_t nb) { return nb * 256u + 16u; }
-
-__host__ __device__ __forceinline__ uint32_t mv_lds_bytes(uint32_t nb, uint32_t ns) {
-    return 2u * kMvCols * mv_xpitch(nb) * 2u + kMvCols * 4u + kMvZero * 2u +
-           (uint32_t)kMvWaves * ns * kMvSlot;
-}
-
-/* NS block slots per wave: block it is multiplied from slot it % NS while
- * blocks it + 1 .. it + NS - 1 are in flight */
-template <uint32_t NS>
-__global__ __launch_bounds__(kMvWaves * 64) void matvec_mfma_q6k(
-    const uint8_t *__restrict__ W, uint32_t rows, uint32_t nb, const float *__restrict__ x,
-    uint32_t batch, float *__restrict__ y, uint32_t *status, float *part_v, uint32_t *part_i,
-    uint32_t part_stride) {
-    using F = Fmt<KQ_LAUNCH_Q6_K>;
-    extern __shared__ __align__(16) _Float16 mv_lds[];
-    const uint32_t K = nb * 256u, pitch = mv_xpitch(nb);
-    _Float16 *xh = mv_lds, *xl = mv_lds + kMvCols * pitch;
-    int *sig = (int *)(xl + kMvCols * pitch);
-    /* the zero operand of the token rows off their sub-block (16 bytes past
-     * a 32-byte boundary of the x image, so its broadcast reads sit on the
-     * banks the live rows leave free) */
-    _Float16 *xz = (_Float16 *)(sig + kMvCols);
-    uint8_t *slots = (uint8_t *)(xz + kMvZero);
-
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t j = lane & 15u, g = lane >> 4;
-    const uint32_t gw = blockIdx.x * (uint32_t)kMvWaves + wave;
-    const uint32_t nwaves = gridDim.x * (uint32_t)kMvWaves;
-    const uint32_t rb = nb * F::kBytes;
-    const uint32_t wbytes = rows * rb;
-    const kq_i4v wr = dma_rsrc(W, wbytes);
-    const uint32_t ntiles = (rows + kTile - 1u) / kTile;
-    uint8_t *myslot = slots + wave * NS * kMvSlot;
-    const uint32_t myslot_lds = lds_addr(myslot);
-
-    /* Work item it = block it % nb of tile gw + nwaves * (it / nb), walked
-     * with counters (t, b) and the tile's byte offset tb = 16 t rb (no
-     * division or 32-bit multiply per item; tb is used only while
-     * t < ntiles, where it stays below wbytes). */
-    struct Pos {
-        uint32_t t, b, tb;
-    };
-    const uint32_t tstep = nwaves * kTile * rb;
-    auto advance = [&](Pos &q) {
-        if (++q.b == nb) {
-            q.b = 0u;
-            q.t += nwaves;
-            q.tb += tstep;
-        }
-    };
-    /* A block's DMA: load i, lane l writes slot bytes [16 p, 16 p + 16) with
-     * p = 64 i + l, which is unit p % 15 of row p / 15 (row pitch 240: 14
-     * units of the row's window -- the block's start rounded down to 4
-     * bytes -- and a gap). Gap units and rows past the matrix read the
-     * matrix's first bytes instead (whatever lands there is never a result:
-     * gap bytes are not read, and rows past the matrix are not stored); the
-     * last load runs on the 48 lanes that reach the slot's 3,840 bytes. */
-    uint32_t ld_r[kMvDma], ld_rb[kMvDma], ld_u[kMvDma];
-#pragma unroll
-    for (int i = 0; i < kMvDma; ++i) {
-        const uint32_t p = (uint32_t)i * 64u + lane;
-        const uint32_t r = p / kMvUnitsPerRow, u = p - kMvUnitsPerRow * r;
-        ld_r[i] = (r < kTile && u * 16u < kMvWin) ? r : 0xffffu;
-        ld_u[i] = 16u * u;
-        ld_rb[i] = r * rb;
-    }
-    auto dma_item = [&](const Pos &q, uint32_t slot) {
-        const uint32_t dst = myslot_lds + slot * kMvSlot;
-#pragma unroll
-        for (int i = 0; i < kMvDma; ++i) {
-            const uint32_t row = q.t * kTile + ld_r[i];
-            const uint32_t o = q.tb + ld_rb[i] + q.b * F::kBytes;
-            const uint32_t off =
-                (ld_r[i] < kTile && q.t < ntiles && row < rows) ? (o & ~3u) + ld_u[i] : ld_u[i];
-            if ((uint32_t)i * 64u + 64u <= kMvSlot / 16u) {
-                dma16(wr, off, dst + 1024u * (uint32_t)i);
-            } else if ((uint32_t)i * 64u + lane < kMvSlot / 16u) {
-                dma16(wr, off, dst + 1024u * (uint32_t)i);
-            }
-        }
-    };
-
-    /* the first block is requested before the staging, the next NS - 1
-     * after it (the staging's own loads wait for every load issued before
-     * theirs) */
-    const uint32_t nitems = ntiles > gw ? ((ntiles - gw + nwaves - 1u) / nwaves) * nb : 0u;
-    Pos ld = {gw, 0u, gw * kTile * rb}, pr = ld;
-    if (nitems > 0u) {
-        dma_item(ld, 0u);
-        advance(ld);
-    }
-
-    /* stage column i (one wave each): scale by 2^sig[i], split into hi + lo */
-    bool bad = false;
-    for (uint32_t i = wave; i < kMvCols; i += (uint32_t)kMvWaves) {
-        const bool real = i < batch;
-        float m = 0.0f;
-        bool nf = false;
-        for (uint32_t c = 4u * lane; c < K; c += 256u) {
-            const float4 v = real ? *(const float4 *)(x + (size_t)i * K + c)
-                                  : make_float4(0.f, 0.f, 0.f, 0.f);
-            nf |= !kq_isfinite(v.x) || !kq_isfinite(v.y) || !kq_isfinite(v.z) || !kq_isfinite(v.w);
-            m = fmaxf(m, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
-        }
-        bad |= nf;
-        m = wave_max_abs(m);
-        const bool any_nf = __ballot(nf) != 0ull;
-        int e = 0;
-        if (!any_nf && m > 0.0f) e = 15 - __builtin_amdgcn_frexp_expf(m);
-        for (uint32_t c = 4u * lane; c < K; c += 256u) {
-            const float4 v = real ? *(const float4 *)(x + (size_t)i * K + c)
-                                  : make_float4(0.f, 0.f, 0.f, 0.f);
-            const float a[4] = {v.x, v.y, v.z, v.w};
-            _Float16 hi[4], lo[4];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const float xs = any_nf ? 0.0f : ldexpf(a[q], e);
-                hi[q] = (_Float16)xs;
-                lo[q] = (_Float16)(xs - (float)hi[q]);
-            }
-            *(h4 *)(xh + i * pitch + c) = h4{hi[0], hi[1], hi[2], hi[3]};
-            *(h4 *)(xl + i * pitch + c) = h4{lo[0], lo[1], lo[2], lo[3]};
-        }
-        if (lane == 0u) sig[i] = e;
-    }
-    if (threadIdx.x < kMvZero / 8u) *(h8 *)(xz + 8u * threadIdx.x) = h8{};
-#pragma unroll
-    for (uint32_t sl = 1u; sl < NS; ++sl) {
-        if (sl < nitems) {
-            dma_item(ld, sl);
-            advance(ld);
-        }
-    }
-    kq_lds_barrier();
-    int unscale[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) unscale[k] = -sig[k];
-
-    bool malformed = false, nonfinite = false;
-    float best_v[4];
-    uint32_t best_i[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        best_v[k] = -__builtin_inff();
-        best_i[k] = 0xffffffffu;
-    }
-    /* Lane l supplies token row j = l % 16 of the A operand on k 8 (l / 16)
-     * .. + 7: rows 0..3 are the hi parts of columns 0..3, rows 4..7 their lo
-     * parts, rows 8..15 repeat them for the step's second sub-block. Lanes
-     * whose k range belongs to the other sub-block read zeros. Product rows
-     * 4 (l / 16) .. + 3 in lane l are then: l / 16 = 0 hi and 1 lo of the
-     * first sub-block, 2 hi and 3 lo of the second. */
-    const bool live = (j >> 3) == (g >> 1);
-    const _Float16 *xa = live ? ((j & 4u) ? xl : xh) + (j & 3u) * pitch + 8u * g : xz + 8u * g;
-    const uint32_t xstep = live ? 256u : 0u;
-    const uint32_t hsh = 8u * (g >> 1); /* this lane's scale byte within a pair */
-    const h2 bias = h2{(_Float16)-1056.0f, (_Float16)-1056.0f}; /* 1024 + 32 */
-    f4 acc = {0.f, 0.f, 0.f, 0.f};
-
-    /* item from its slot: 8 two-sub-block steps into acc; at the tile's last
-     * block lanes 0..15 write row t*16 + j of columns 0 .. batch-1. Every LDS
-     * read of the item is issued before its first product. */
-    const uint32_t jrb = j * rb;
-    auto process = [&](const Pos &q, const uint8_t *sp, auto &&refill) {
-        const uint32_t bb = q.b;
-        const uint32_t row = q.t * kTile + j;
-        const uint32_t sh = (q.tb + jrb + bb * F::kBytes) & 3u;
-        const uint8_t *p = sp + j * kMvPitch;
-        auto w32 = [&](uint32_t o) { return *(const uint32_t *)(p + o); };
-        /* columns 128 n + 32 q + 8 g .. + 7 of step (n, q): ql bytes 64 n +
-         * 8 g (q = 0, 2) and + 32 (q = 1, 3), qh bytes 128 + 32 n + 8 g; the
-         * scales at 192 and d at 208 (the window starts up to 3 bytes early) */
-        uint32_t wa[2][3], wbv[2][3], wq[2][3], ws[6];
-#pragma unroll
-        for (uint32_t n = 0; n < 2u; ++n) {
-            const uint32_t oa = 64u * n + 8u * g, oq = 128u + 32u * n + 8u * g;
-#pragma unroll
-            for (uint32_t e = 0; e < 3u; ++e) {
-                wa[n][e] = w32(oa + 4u * e);
-                wbv[n][e] = w32(oa + 32u + 4u * e);
-                wq[n][e] = w32(oq + 4u * e);
-            }
-        }
-#pragma unroll
-        for (uint32_t e = 0; e < 6u; ++e) ws[e] = w32(192u + 4u * e);
-        const _Float16 *pa = xa + xstep * bb;
-        h8 av[2][4];
-#pragma unroll
-        for (uint32_t n = 0; n < 2u; ++n)
-#pragma unroll
-            for (uint32_t qq = 0; qq < 4u; ++qq) av[n][qq] = *(const h8 *)(pa + 128u * n + 32u * qq);
-        /* every read of the slot has landed: its next block can be requested
-         * before the products */
-        wait_lgkm0();
-        refill();
-        __builtin_amdgcn_sched_barrier(0);
-
-        const float d = f16f(kq_align2(ws[5], ws[4], sh)); /* block bytes 208, 209 */
-        malformed |= row < rows && !kq_isfinite(d);
-        uint32_t sc[4];
-#pragma unroll
-        for (uint32_t e = 0; e < 4u; ++e) sc[e] = kq_align2(ws[e + 1u], ws[e], sh) >> hsh;
-#pragma unroll
-        for (uint32_t n = 0; n < 2u; ++n) {
-            const uint32_t A[2] = {kq_align2(wa[n][1], wa[n][0], sh),
-                                   kq_align2(wa[n][2], wa[n][1], sh)};
-            const uint32_t B[2] = {kq_align2(wbv[n][1], wbv[n][0], sh),
-                                   kq_align2(wbv[n][2], wbv[n][1], sh)};
-            const uint32_t H[2] = {kq_align2(wq[n][1], wq[n][0], sh),
-                                   kq_align2(wq[n][2], wq[n][1], sh)};
-            uint32_t c[4][2];
-#pragma unroll
-            for (int w = 0; w < 2; ++w) {
-                c[0][w] = (A[w] & 0x0f0f0f0fu) | ((H[w] << 4) & 0x30303030u);
-                c[1][w] = (B[w] & 0x0f0f0f0fu) | ((H[w] << 2) & 0x30303030u);
-                c[2][w] = ((A[w] >> 4) & 0x0f0f0f0fu) | (H[w] & 0x30303030u);
-                c[3][w] = ((B[w] >> 4) & 0x0f0f0f0fu) | ((H[w] >> 2) & 0x30303030u);
-            }
-            /* the four steps are independent products: all are issued
-             * before any result is scaled, so the matrix core's latency
-             * overlaps the next products and the scaling */
-            f4 tm[4];
-#pragma unroll
-            for (uint32_t qq = 0; qq < 4u; ++qq) {
-                const h2 w0 = bytes_lo(c[qq][0]) + bias, w1 = bytes_hi(c[qq][0]) + bias;
-                const h2 w2 = bytes_lo(c[qq][1]) + bias, w3 = bytes_hi(c[qq][1]) + bias;
-                const h8 bw = h8{w0.x, w0.y, w1.x, w1.y, w2.x, w2.y, w3.x, w3.y};
-                tm[qq] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[n][qq], bw,
-                                                                f4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-            }
-#pragma unroll
-            for (uint32_t qq = 0; qq < 4u; ++qq) {
-                /* sub-block 8 n + 2 qq + (g >> 1): byte (2 qq) & 3 of word
-                 * 2 n + qq / 2, pre-shifted by this lane's half */
-                const int8_t scv = (int8_t)((sc[2u * n + (qq >> 1)] >> (16u * (qq & 1u))) & 0xffu);
-                const float ds = d * (float)scv;
-#pragma unroll
-                for (int k = 0; k < 4; ++k) acc[k] = fmaf(ds, tm[qq][k], acc[k]);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        if (bb + 1u == nb) {
-            /* column k of row j = the four lanes j + 16 G: hi and lo of both
-             * sub-block halves */
-            f4 o;
-#pragma unroll
-            for (int k = 0; k < 4; ++k) o[k] = acc[k] + __shfl_down(acc[k], 32, KQ_WAVE);
-#pragma unroll
-            for (int k = 0; k < 4; ++k) o[k] += __shfl_down(o[k], 16, KQ_WAVE);
-            if (g == 0u && row < rows) {
-#pragma unroll
-                for (uint32_t k = 0; k < 4u; ++k) {
-                    if (k < batch) {
-                        const float v = ldexpf(o[k], unscale[k]);
-                        nonfinite |= !kq_isfinite(v);
-                        y[(size_t)k * rows + row] = v;
-                        mv_argmax_merge(best_v[k], best_i[k], v, row);
-                    }
-                }
-            }
-            acc = f4{0.f, 0.f, 0.f, 0.f};
-        }
-    };
-    /* Before block it: every DMA issued after its own has not necessarily
-     * landed, and there are min(NS - 1, nitems - 1 - it) of them (kMvDma
-     * loads each; the y stores between are not loads). Once its reads are
-     * in registers, its slot takes block it + NS. */
-    uint32_t slot = 0u;
-    for (uint32_t it = 0u; it < nitems; ++it) {
-        const uint32_t after = nitems - 1u - it;
-        wait_after<(uint32_t)kMvDma, NS - 1u>(after);
-        process(pr, myslot + slot * kMvSlot, [&]() {
-            if (it + NS < nitems) {
-                dma_item(ld, slot);
-                advance(ld);
-            }
-        });
-        advance(pr);
-        slot = slot + 1u == NS ? 0u : slot + 1u;
-    }
-    if (bad) kq_flag(status, KQ_DEV_INPUT);
-    if (malformed) kq_flag(status, KQ_DEV_MALFORMED);
-    if (nonfinite) kq_flag(status, KQ_DEV_NUMERIC);
-    if (part_v != nullptr) {
-#pragma unroll
-        for (uint32_t k = 0; k < 4u; ++k) {
-            float bv = best_v[k];
-            uint32_t bi = best_i[k];
-            /* lanes 16..63 hold no real column: only lanes 0..15 merge */
-#pragma unroll
-            for (int o = 8; o > 0; o >>= 1) {
-                const float ov = __shfl_xor(bv, o, KQ_WAVE);
-                const uint32_t oi = __shfl_xor(bi, o, KQ_WAVE);
-                mv_argmax_merge(bv, bi, ov, oi);
-            }
-            if (lane == 0u && k < batch) {
-                part_v[(size_t)k * part_stride + gw] = bv;
-                part_i[(size_t)k * part_stride + gw] = bi;
-                for (uint32_t sl = gw + nwaves; sl < part_stride; sl += nwaves) {
-                    part_v[(size_t)k * part_stride + sl] = -__builtin_inff();
-                    part_i[(size_t)k * part_stride + sl] = 0xffffffffu;
-                }
-            }
-        }
-    }
-}
-
-/* ------------------------------------------------------------------ */
-/* The same product at 2,048 columns on whole tiles shared by a workgroup
- *
- * matvec_mfma_q6k gives every wave its own ring of block slots and its own
- * tiles, so the weights in flight grow with the waves and two waves per
- * SIMD fill the LDS. Here a workgroup of eight waves owns a contiguous run
- * of 16-row tiles; a tile (16 rows x 1,680 contiguous bytes) is copied into
- * a two-slot LDS ring by 1 KiB LDS-DMA instructions spread over the waves,
- * one tile ahead of the one being multiplied, and wave b multiplies Q6_K
- * block b of every row of it. Its activation operand (the block's 256
- * columns of the four columns, hi and lo, laid out as above) is 32
- * registers held for the whole run, so nothing but the tile is read from
- * LDS and two workgroups share a CU (four waves per SIMD). Each wave sums
- * its product rows across lanes and leaves 16 rows x 4 columns in LDS;
- * after the next barrier wave 0 adds the eight blocks in order, unscales,
- * stores and keeps the argmax partials: one per workgroup and column. */
-
-constexpr uint32_t kLtWaves = 8u;                      /* one per 256-column block */
-constexpr uint32_t kLtRow = 8u * 210u;                 /* row bytes at 2,048 columns */
-constexpr uint32_t kLtTile = kTile * kLtRow;           /* 26,880 */
-constexpr uint32_t kLtIns = (kLtTile + 1023u) / 1024u; /* DMA instructions per tile: 27 */
-constexpr uint32_t kLtSlot = kLtIns * 1024u;
-constexpr uint32_t kLtIpw = (kLtIns + kLtWaves - 1u) / kLtWaves; /* per wave, at most 4 */
-
-__global__ __launch_bounds__(kLtWaves * 64) __attribute__((amdgpu_waves_per_eu(4, 4)))
-void lm_q6k_tiles(const uint8_t *__restrict__ W, uint32_t rows, const float *__restrict__ x,
-                  uint32_t batch, float *__restrict__ y, uint32_t *status, float *part_v,
-                  uint32_t *part_i, uint32_t part_stride) {
-    constexpr uint32_t K = 2048u;
-    __shared__ __align__(16) uint8_t ring[2][kLtSlot];
-    __shared__ __align__(16) float part[2][kLtWaves][64];
-    __shared__ float smax[kLtWaves][kMvCols];
-    __shared__ uint32_t snf[kLtWaves][kMvCols];
-
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t b = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); /* block of the row */
-    const uint32_t j = lane & 15u, g = lane >> 4;
-    const uint32_t ntiles = (rows + kTile - 1u) / kTile;
-    const uint32_t lo = (uint32_t)((uint64_t)ntiles * blockIdx.x / gridDim.x);
-    const uint32_t hi = (uint32_t)((uint64_t)ntiles * (blockIdx.x + 1u) / gridDim.x);
-    const kq_i4v wr = dma_rsrc(W, rows * kLtRow);
-
-    /* instruction n = b + 8 q of a tile: lane l copies tile bytes
-     * [16 (64 n + l), + 16) to the same place in the slot; units past the
-     * tile re-read its first bytes (never used) */
-    uint32_t rel[kLtIpw];
-#pragma unroll
-    for (uint32_t q = 0; q < kLtIpw; ++q) {
-        const uint32_t u = (b + kLtWaves * q) * 64u + lane;
-        rel[q] = u * 16u < kLtTile ? u * 16u : 0u;
-    }
-    auto issue = [&](uint32_t t, uint32_t s) {
-        const uint32_t toff = t * kLtTile, dst = lds_addr(&ring[s][0]);
-#pragma unroll
-        for (uint32_t q = 0; q < kLtIpw; ++q) {
-            const uint32_t n = b + kLtWaves * q; /* wave-uniform */
-            if (n < kLtIns) dma16(wr, toff + rel[q], dst + 1024u * n);
-        }
-    };
-    if (lo < hi) issue(lo, 0u);
-
-    /* column k's power of two from its largest magnitude: wave b scans its
-     * block's 256 columns of the four (16 per lane), the workgroup merges */
-    bool bad = false;
-    {
-        const uint32_t k = lane >> 4, c0 = 256u * b + 16u * (lane & 15u);
-        float m = 0.0f;
-        uint32_t nf = 0u;
-        if (k < batch) {
-#pragma unroll
-            for (uint32_t i = 0; i < 4u; ++i) {
-                const float4 v = *(const float4 *)(x + (size_t)k * K + c0 + 4u * i);
-                nf |= (!kq_isfinite(v.x) || !kq_isfinite(v.y) || !kq_isfinite(v.z) ||
-                       !kq_isfinite(v.w)) ? 1u : 0u;
-                m = fmaxf(m, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
-            }
-        }
-#pragma unroll
-        for (int o = 8; o > 0; o >>= 1) {
-            m = fmaxf(m, __shfl_xor(m, o, KQ_WAVE));
-            nf |= __shfl_xor(nf, o, KQ_WAVE);
-        }
-        bad = nf != 0u;
-        if ((lane & 15u) == 0u) {
-            smax[b][k] = m;
-            snf[b][k] = nf;
-        }
-    }
-    __syncthreads();
-    int sig[kMvCols];
-    bool zero[kMvCols];
-#pragma unroll
-    for (uint32_t k = 0; k < kMvCols; ++k) {
-        float m = 0.0f;
-        uint32_t nf = 0u;
-#pragma unroll
-        for (uint32_t w = 0; w < kLtWaves; ++w) {
-            m = fmaxf(m, smax[w][k]);
-            nf |= snf[w][k];
-        }
-        zero[k] = nf != 0u;
-        sig[k] = (nf == 0u && m > 0.0f) ? 15 - __builtin_amdgcn_frexp_expf(m) : 0;
-    }
-
-    /* lane (j, g): token row j of the A operand on k 8 g .. + 7 of step
-     * (n, qq) = columns 256 b + 128 n + 32 qq + 8 g ..; rows 0..3 the hi
-     * parts of columns 0..3, 4..7 their lo parts, 8..15 the same for the
-     * step's second sub-block; lanes off their sub-block hold zeros */
-    h8 av[2][4];
-    {
-        const uint32_t c = j & 3u;
-        const bool live = (j >> 3) == (g >> 1) && c < batch && !zero[c];
-        const bool want_lo = (j & 4u) != 0u;
-        int e = sig[0];
-#pragma unroll
-        for (uint32_t k = 1; k < kMvCols; ++k) e = c == k ? sig[k] : e;
-        const float *xp = x + (size_t)(live ? c : 0u) * K + 256u * b + 8u * g;
-#pragma unroll
-        for (uint32_t n = 0; n < 2u; ++n)
-#pragma unroll
-            for (uint32_t qq = 0; qq < 4u; ++qq) {
-                float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-                if (live) {
-                    const float4 p0 = *(const float4 *)(xp + 128u * n + 32u * qq);
-                    const float4 p1 = *(const float4 *)(xp + 128u * n + 32u * qq + 4u);
-                    v[0] = p0.x; v[1] = p0.y; v[2] = p0.z; v[3] = p0.w;
-                    v[4] = p1.x; v[5] = p1.y; v[6] = p1.z; v[7] = p1.w;
-                }
-                h8 h;
-#pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const float xs = ldexpf(v[i], e);
-                    const _Float16 hv = (_Float16)xs;
-                    h[i] = want_lo ? (_Float16)(xs - (float)hv) : hv;
-                }
-                av[n][qq] = h;
-            }
-    }
-
-    const uint32_t hsh = 8u * (g >> 1); /* this lane's scale byte within a pair */
-    const h2 bias = h2{(_Float16)-1056.0f, (_Float16)-1056.0f}; /* 1024 + 32 */
-    /* row j's block b in a slot: from its 4-byte aligned start, sh bytes in */
-    const uint32_t boff = j * kLtRow + 210u * b;
-    const uint32_t sh = boff & 3u, wbase = boff & ~3u;
-    bool malformed = false, nonfinite = false;
-    float best_v = -__builtin_inff();
-    uint32_t best_i = 0xffffffffu;
-    const uint32_t rk = lane >> 4, rr = lane & 15u; /* wave 0's output: column, row */
-
-    for (uint32_t tau = lo; tau < hi + 1u; ++tau) {
-        wait_vm<0>();
-        kq_lds_barrier();
-        if (tau + 1u < hi) issue(tau + 1u, (tau + 1u - lo) & 1u);
-        if (tau > lo && b == 0u) {
-            /* tile tau - 1: the eight blocks' sums in order */
-            const uint32_t pb = (tau - 1u - lo) & 1u;
-            float s = 0.0f;
-#pragma unroll
-            for (uint32_t w = 0; w < kLtWaves; ++w) s += part[pb][w][lane];
-            const uint32_t row = (tau - 1u) * kTile + rr;
-            if (row < rows && rk < batch) {
-                const float v = ldexpf(s, -sig[rk]);
-                nonfinite |= !kq_isfinite(v);
-                y[(size_t)rk * rows + row] = v;
-                mv_argmax_merge(best_v, best_i, v, row);
-            }
-        }
-        if (tau == hi) break;
-
-        const uint8_t *p = &ring[(tau - lo) & 1u][wbase];
-        auto w32 = [&](uint32_t o) { return *(const uint32_t *)(p + o); };
-        uint32_t wa[2][3], wbv[2][3], wq[2][3], ws[6];
-#pragma unroll
-        for (uint32_t n = 0; n < 2u; ++n) {
-            const uint32_t oa = 64u * n + 8u * g, oq = 128u + 32u * n + 8u * g;
-#pragma unroll
-            for (uint32_t e = 0; e < 3u; ++e) {
-                wa[n][e] = w32(oa + 4u * e);
-                wbv[n][e] = w32(oa + 32u + 4u * e);
-                wq[n][e] = w32(oq + 4u * e);
-            }
-        }
-#pragma unroll
-        for (uint32_t e = 0; e < 6u; ++e) ws[e] = w32(192u + 4u * e);
-        const uint32_t row = tau * kTile + j;
-        const float d = f16f(kq_align2(ws[5], ws[4], sh)); /* block bytes 208, 209 */
-        malformed |= row < rows && !kq_isfinite(d);
-        uint32_t sc[4];
-#pragma unroll
-        for (uint32_t e = 0; e < 4u; ++e) sc[e] = kq_align2(ws[e + 1u], ws[e], sh) >> hsh;
-        f4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (uint32_t n = 0; n < 2u; ++n) {
-            const uint32_t A[2] = {kq_align2(wa[n][1], wa[n][0], sh),
-                                   kq_align2(wa[n][2], wa[n][1], sh)};
-            const uint32_t B[2] = {kq_align2(wbv[n][1], wbv[n][0], sh),
-                                   kq_align2(wbv[n][2], wbv[n][1], sh)};
-            const uint32_t H[2] = {kq_align2(wq[n][1], wq[n][0], sh),
-                                   kq_align2(wq[n][2], wq[n][1], sh)};
-            uint32_t c[4][2];
-#pragma unroll
-            for (int w = 0; w < 2; ++w) {
-                c[0][w] = (A[w] & 0x0f0f0f0fu) | ((H[w] << 4) & 0x30303030u);
-                c[1][w] = (B[w] & 0x0f0f0f0fu) | ((H[w] << 2) & 0x30303030u);
-                c[2][w] = ((A[w] >> 4) & 0x0f0f0f0fu) | (H[w] & 0x30303030u);
-                c[3][w] = ((B[w] >> 4) & 0x0f0f0f0fu) | ((H[w] >> 2) & 0x30303030u);
-            }
-            f4 tm[4];
-#pragma unroll
-            for (uint32_t qq = 0; qq < 4u; ++qq) {
-                const h2 w0 = bytes_lo(c[qq][0]) + bias, w1 = bytes_hi(c[qq][0]) + bias;
-                const h2 w2 = bytes_lo(c[qq][1]) + bias, w3 = bytes_hi(c[qq][1]) + bias;
-                const h8 bw = h8{w0.x, w0.y, w1.x, w1.y, w2.x, w2.y, w3.x, w3.y};
-                tm[qq] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[n][qq], bw,
-                                                                f4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-            }
-#pragma unroll
-            for (uint32_t qq = 0; qq < 4u; ++qq) {
-                const int8_t scv = (int8_t)((sc[2u * n + (qq >> 1)] >> (16u * (qq & 1u))) & 0xffu);
-                const float ds = d * (float)scv;
-#pragma unroll
-                for (int k = 0; k < 4; ++k) acc[k] = fmaf(ds, tm[qq][k], acc[k]);
-            }
-        }
-        /* column k of row j = the four lanes j + 16 G: hi and lo of both
-         * sub-block halves */
-        f4 o;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) o[k] = acc[k] + __shfl_down(acc[k], 32, KQ_WAVE);
-#pragma unroll
-        for (int k = 0; k < 4; ++k) o[k] += __shfl_down(o[k], 16, KQ_WAVE);
-        if (g == 0u) {
-#pragma unroll
-            for (uint32_t k = 0; k < 4u; ++k) part[(tau - lo) & 1u][b][16u * k + j] = o[k];
-        }
-    }
-    /* no LDS-DMA load may outlive the workgroup */
-    wait_vm<0>();
-    if (bad) kq_flag(status, KQ_DEV_INPUT);
-    if (malformed) kq_flag(status, KQ_DEV_MALFORMED);
-    if (nonfinite) kq_flag(status, KQ_DEV_NUMERIC);
-    if (part_v != nullptr && b == 0u) {
-        /* wave 0's lanes 16 k .. 16 k + 15 hold column k's candidates */
-#pragma unroll
-        for (int o = 8; o > 0; o >>= 1) {
-            const float ov = __shfl_xor(best_v, o, KQ_WAVE);
-            const uint32_t oi = __shfl_xor(best_i, o, KQ_WAVE);
-            mv_argmax_merge(best_v, best_i, ov, oi);
-        }
-        if (rr == 0u && rk < batch) {
-            part_v[(size_t)rk * part_stride + blockIdx.x] = best_v;
-            part_i[(size_t)rk * part_stride + blockIdx.x] = best_i;
-            for (uint32_t sl = blockIdx.x + gridDim.x; sl < part_stride; sl += gridDim.x) {
-                part_v[(size_t)rk * part_stride + sl] = -__builtin_inff();
-                part_i[(size_t)rk * part_stride + sl] = 0xffffffffu;
-            }
-        }
-    }
-}
 
 /* ------------------------------------------------------------------ */
 /* grouped Q6_K down pass with its weights streamed through LDS
@@ -1782,7 +1172,7 @@ void lm_q6k_tiles(const uint8_t *__restrict__ W, uint32_t rows, const float *__r
  * The same work split, staging and Tile<Q6_K> steps as grouped_pass, but
  * the block operand pieces (twelve scattered 4-byte windows per lane) are
  * not fetched from global memory: each wave loads one 16-row block of its
- * tile contiguously (as matvec_mfma_q6k does) into a private LDS slot, two
+ * tile contiguously into a private LDS slot, two
  * blocks ahead of the one it multiplies, and the Raw pieces are read from
  * there. Offsets past the matrix read as zeros and stores past the
  * workgroup's outputs are dropped, so no path branches around a load. */
@@ -2139,102 +1529,4 @@ extern "C" hipError_t kq_launch_gemm_q8_0(const void *W, uint32_t rows, uint32_t
     return pass_cols<KQ_LAUNCH_Q8_0, 1>(cols, nullptr, nullptr, (const uint8_t *)W, nullptr, x,
                                         nullptr, nullptr, 0u, tokens, 0u, rows, 0u, ny, 1u, y,
                                         status, s);
-}
-
-/* batched Q6_K matvec on MFMA: rows of 256 .. 4096 columns (whole blocks),
- * 2 .. 4 activation columns, at least 65,536 rows (enough 16-row tiles to
- * fill the device) */
-extern "C" int kq_launch_matvec_mfma_supported(uint32_t type, uint32_t rows, uint32_t cols,
-                                               uint32_t batch) {
-    /* block offsets, and the out-of-range offset past the last row, stay
-     * within 32 bits */
-    const uint64_t bytes = (uint64_t)rows * (cols / 256u) * 210u;
-    return type == KQ_LAUNCH_Q6_K && batch >= 2u && batch <= kMvCols && cols % 256u == 0u &&
-           cols >= 256u && cols <= kMvMaxK && rows >= 65536u && bytes <= 0xfffff000ull;
-}
-
-/* block slots per wave: as many (2 .. kMvMaxSlots) as fit beside the
- * activation image */
-static uint32_t mv_ns(uint32_t nb) {
-    uint32_t ns = kMvMaxSlots;
-    while (ns > 2u && mv_lds_bytes(nb, ns) > kMvLdsMax) --ns;
-    return ns;
-}
-/* f(std::integral_constant<uint32_t, ns>) for ns in 2 .. kMvMaxSlots */
-template <uint32_t NS = 2u, typename Fn>
-static void kq_mv_ns_dispatch(uint32_t ns, Fn &&f) {
-    if constexpr (NS <= kMvMaxSlots) {
-        if (ns == NS) f(std::integral_constant<uint32_t, NS>{});
-        else kq_mv_ns_dispatch<NS + 1u>(ns, f);
-    }
-}
-template <uint32_t NS>
-static hipError_t mv_occupancy(int *n, uint32_t nb) {
-    return hipOccupancyMaxActiveBlocksPerMultiprocessor(n, matvec_mfma_q6k<NS>, kMvWaves * 64,
-                                                         mv_lds_bytes(nb, NS));
-}
-
-/* a resident grid (workgroups that fit at once), capped by the tile count */
-static uint32_t mv_blocks(uint32_t rows, uint32_t nb) {
-    static uint32_t per_cu_cache[kMvMaxK / 256u + 1u];
-    uint32_t &per = per_cu_cache[nb];
-    if (per == 0u) {
-        int dev = 0, cus = 0, n = 0;
-        const uint32_t ns = mv_ns(nb);
-        hipError_t oe = hipErrorInvalidValue;
-        kq_mv_ns_dispatch(ns, [&](auto c) { oe = mv_occupancy<decltype(c)::value>(&n, nb); });
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-            cus < 1)
-            cus = 256;
-        if (oe != hipSuccess || n < 1) n = 1;
-        per = (uint32_t)(n * cus);
-    }
-    const uint32_t tiles = (rows + kTile - 1u) / kTile;
-    uint32_t blocks = (tiles + (uint32_t)kMvWaves - 1u) / (uint32_t)kMvWaves;
-    if (blocks > per) blocks = per;
-    return blocks < 1u ? 1u : blocks;
-}
-
-/* lm_q6k_tiles (2,048 columns): two workgroups per CU */
-static uint32_t lt_blocks() {
-    static uint32_t blocks = 0u;
-    if (blocks == 0u) {
-        int dev = 0, cus = 0;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-            cus < 1)
-            cus = 256;
-        blocks = 2u * (uint32_t)cus;
-    }
-    return blocks;
-}
-
-/* argmax partials per column: one per wave (matvec_mfma_q6k) or per
- * workgroup (lm_q6k_tiles) */
-extern "C" uint32_t kq_launch_matvec_mfma_waves(uint32_t rows, uint32_t cols) {
-    if (cols == 2048u) return lt_blocks();
-    return mv_blocks(rows, cols / 256u) * (uint32_t)kMvWaves;
-}
-
-extern "C" hipError_t kq_launch_matvec_mfma(const void *W, uint32_t rows, uint32_t cols,
-                                            const float *x, uint32_t batch, float *y,
-                                            uint32_t *status, float *part_v, uint32_t *part_i,
-                                            uint32_t part_stride, hipStream_t stream) {
-    const uint32_t nb = cols / 256u;
-    if (nb == 8u) {
-        hipLaunchKernelGGL(lm_q6k_tiles, dim3(lt_blocks()), dim3(kLtWaves * 64), 0, stream,
-                           (const uint8_t *)W, rows, x, batch, y, status, part_v, part_i,
-                           part_stride);
-        return hipGetLastError();
-    }
-    const uint32_t ns = mv_ns(nb);
-    const dim3 grid(mv_blocks(rows, nb)), block(kMvWaves * 64);
-#define KQ_MV(NS)                                                                              \
-    hipLaunchKernelGGL(matvec_mfma_q6k<NS>, grid, block, mv_lds_bytes(nb, NS), stream,         \
-                       (const uint8_t *)W, rows, nb, x, batch, y, status, part_v, part_i,      \
-                       part_stride)
-    kq_mv_ns_dispatch(ns, [&](auto c) { KQ_MV(decltype(c)::value); });
-#undef KQ_MV
-    return hipGetLastError();
 }

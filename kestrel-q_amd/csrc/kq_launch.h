@@ -39,6 +39,18 @@ hipError_t kq_launch_matvec(uint32_t type, const void *W, uint32_t rows, uint32_
                             const float *x, uint32_t batch, float *y, uint32_t *status,
                             float *part_v, uint32_t *part_i, uint32_t part_stride,
                             hipStream_t stream);
+/* y = W x for up to 8 columns on MFMA over whole tiles (kq_mvtiles.hip);
+ * parts: argmax partials per column, one per workgroup; same partials
+ * contract */
+int kq_launch_mv_tiles_supported(uint32_t type, uint32_t rows, uint32_t cols, uint32_t batch);
+uint32_t kq_launch_mv_tiles_parts(uint32_t type, uint32_t rows, uint32_t cols);
+hipError_t kq_launch_mv_tiles(uint32_t type, const void *W, uint32_t rows, uint32_t cols,
+                              const float *x, uint32_t batch, float *y, uint32_t *status,
+                              float *part_v, uint32_t *part_i, uint32_t part_stride,
+                              hipStream_t stream);
+/* how many of `left` activation columns the next launch of a product takes
+ * (1 .. 8), the batch argument of kq_launch_matvec and _waves */
+uint32_t kq_launch_matvec_columns(uint32_t type, uint32_t rows, uint32_t cols, uint32_t left);
 /* y[t] = W x[t] for many tokens, Q8_0 W on MFMA (kq_grouped.hip): row
  * lengths 256, 320, 512, 640, 1024, 2048 or 10240 */
 int kq_launch_gemm_q8_0_supported(uint32_t rows, uint32_t cols);
@@ -61,13 +73,6 @@ hipError_t kq_launch_dense_q8(const void *w0, const void *w1, uint32_t rows, uin
                               uint32_t splits, float *out, uint32_t *status, hipStream_t s);
 hipError_t kq_launch_gemm_q8_0(const void *W, uint32_t rows, uint32_t cols, const float *x,
                                uint32_t tokens, float *y, uint32_t *status, hipStream_t stream);
-/* batched Q6_K matvec on MFMA (kq_grouped.hip), used by kq_launch_matvec
- * where supported; same partials contract */
-int kq_launch_matvec_mfma_supported(uint32_t type, uint32_t rows, uint32_t cols, uint32_t batch);
-uint32_t kq_launch_matvec_mfma_waves(uint32_t rows, uint32_t cols);
-hipError_t kq_launch_matvec_mfma(const void *W, uint32_t rows, uint32_t cols, const float *x,
-                                 uint32_t batch, float *y, uint32_t *status, float *part_v,
-                                 uint32_t *part_i, uint32_t part_stride, hipStream_t stream);
 uint32_t kq_launch_argmax_parts(uint32_t count);
 hipError_t kq_launch_argmax(const float *logits, uint32_t count, uint32_t batch,
                             float *part_v, uint32_t *part_i, uint32_t *ids,

@@ -1,7 +1,8 @@
 /*
  * kq_matvec.hip — dequant-fused matrix-vector products y = W x for GGUF
- * Q4_K, Q5_K, Q6_K, Q8_0, Q5_1 and IQ4_NL rows (batch 1..4, fp32 activations and outputs) and
- * greedy argmax over the results.
+ * Q4_K, Q5_K, Q6_K, Q8_0, Q5_1 and IQ4_NL rows (fp32 activations and outputs: the row engine
+ * for batch 1..4, and the choice between it and kq_mvtiles.hip) and greedy argmax over the
+ * results.
  *
  * Restates the row loop of kq_weight_provider_linear_f32
  * (src/kq_weight_provider.c:464-475) around kq_quantized_row_dot_f32
@@ -721,10 +722,54 @@ extern "C" int kq_launch_matvec_supported(uint32_t type, uint32_t cols, uint32_t
     return be != 0u && cols != 0u && cols % be == 0u && cols <= kMaxCols;
 }
 
+/* launches the row engine takes for a product of at most 4 columns */
+static uint32_t row_launches(uint32_t type, uint32_t cols, uint32_t batch) {
+    uint32_t be, bb, n = 0u;
+    block_geometry(type, be, bb);
+    if (be == 0u || cols % be != 0u) return 0u;
+    if (cols > kWideCols && wide_shape((cols + kWideCols - 1u) / kWideCols, batch)) return 1u;
+    for (uint32_t off = 0u, seg; off < cols; off += seg, ++n) {
+        seg = segment_cols(be, cols - off);
+        if (seg == 0u) return 0u;
+    }
+    return n;
+}
+
+/* The row engine or the matrix-core tiles (kq_mvtiles.hip). The tiles take
+ * about the same time for 1 to 8 columns; the row engine's grows with them.
+ * Measured over 256 .. 40,000 rows of 512 .. 10,240 columns in every format
+ * (row engine against tiles, us):
+ *   - five columns or more are two launches of the row engine: the tiles
+ *     win everywhere (1000 x 2048 Q5_1, 5 columns: 9.2 / 6.4; 10000 x 2560
+ *     Q8_0, 8 columns: 74.8 / 11.7);
+ *   - so they do where fewer columns take several launches, rows of other
+ *     widths than the engine's (4000 x 640 Q8_0, 1 column: 7.6 / 4.8;
+ *     10000 x 10240 Q4_K, 2 columns: 43.7 / 24.4), up to 20,000 rows at one
+ *     column (40000 x 640 Q5_1: 11.8 / 15.2);
+ *   - in one launch, 3 and 4 columns from about 2,048 rows (4000 x 2048
+ *     Q8_0, 4 columns: 7.6 / 5.8; 300 rows: 4.8 / 5.6), Q6_K 2 columns from
+ *     about 4,096 (4000 x 2560: 8.4 / 6.8; 1000 rows: 5.4 / 6.6) up to 4,096
+ *     columns (4000 x 6144: 12.1 / 14.4); the other formats at 2 columns and
+ *     all at one stay (40000 x 2048, 2 columns: Q8_0 16.1 / 18.6, Q4_K
+ *     13.1 / 15.6). */
+static bool use_tiles(uint32_t type, uint32_t rows, uint32_t cols, uint32_t batch) {
+    if (!kq_launch_mv_tiles_supported(type, rows, cols, batch)) return false;
+    if (batch > 4u) return true;
+    if (row_launches(type, cols, batch) > 1u) return batch > 1u || rows <= 20000u;
+    if (batch >= 3u) return rows >= 2048u;
+    return batch == 2u && type == KQ_LAUNCH_Q6_K && rows >= 4096u && cols <= 4096u;
+}
+
+extern "C" uint32_t kq_launch_matvec_columns(uint32_t type, uint32_t rows, uint32_t cols,
+                                             uint32_t left) {
+    const uint32_t all = left > 8u ? 8u : left;
+    if (use_tiles(type, rows, cols, all)) return all;
+    return left > 4u ? 4u : left;
+}
+
 extern "C" uint32_t kq_launch_matvec_waves(uint32_t type, uint32_t rows, uint32_t cols,
                                            uint32_t batch) {
-    if (kq_launch_matvec_mfma_supported(type, rows, cols, batch))
-        return kq_launch_matvec_mfma_waves(rows, cols);
+    if (use_tiles(type, rows, cols, batch)) return kq_launch_mv_tiles_parts(type, rows, cols);
     uint32_t waves = 0u;
     if (dispatch(type, nullptr, rows, cols, nullptr, batch, nullptr, nullptr, nullptr, nullptr,
                  0u, nullptr, &waves) != hipSuccess)
@@ -736,9 +781,9 @@ extern "C" hipError_t kq_launch_matvec(uint32_t type, const void *W, uint32_t ro
                                        uint32_t cols, const float *x, uint32_t batch, float *y,
                                        uint32_t *status, float *part_v, uint32_t *part_i,
                                        uint32_t part_stride, hipStream_t stream) {
-    if (kq_launch_matvec_mfma_supported(type, rows, cols, batch))
-        return kq_launch_matvec_mfma(W, rows, cols, x, batch, y, status, part_v, part_i,
-                                     part_stride, stream);
+    if (use_tiles(type, rows, cols, batch))
+        return kq_launch_mv_tiles(type, W, rows, cols, x, batch, y, status, part_v, part_i,
+                                  part_stride, stream);
     return dispatch(type, W, rows, cols, x, batch, y, status, part_v, part_i, part_stride, stream,
                     nullptr);
 }

@@ -853,13 +853,15 @@ static kq_status validate_matvec(const kq_hip_context *c, uint32_t type_id, cons
     return KQ_STATUS_OK;
 }
 
-/* Enqueue y for up to 8 batch columns, in launches of at most 4. */
+/* Enqueue y for up to 8 batch columns, in launches of as many columns as
+ * the product takes at once. */
 static hipError_t enqueue_matvec(kq_hip_context *c, uint32_t type_id, const void *w,
                                  uint64_t rows, uint64_t cols, const float *x, uint32_t batch,
                                  float *y, float *pv, uint32_t *pi, uint32_t nparts) {
     uint32_t done = 0u;
     while (done < batch) {
-        uint32_t nb = batch - done > 4u ? 4u : batch - done;
+        const uint32_t nb =
+            kq_launch_matvec_columns(type_id, (uint32_t)rows, (uint32_t)cols, batch - done);
         hipError_t e = kq_launch_matvec(type_id, w, (uint32_t)rows, (uint32_t)cols,
                                         x + (size_t)done * cols, nb, y + (size_t)done * rows,
                                         c->d_status, pv ? pv + (size_t)done * nparts : NULL,
@@ -953,9 +955,10 @@ static kq_status lm_head(kq_hip_context *c, uint32_t type_id, const void *w, uin
     if (st != KQ_STATUS_OK) return st;
     /* partials per batch column: the most any launch of the call uses */
     nparts = 0u;
-    for (uint32_t done = 0u; done < batch; done += 4u) {
-        const uint32_t nb = batch - done > 4u ? 4u : batch - done;
-        const uint32_t w_nb = kq_launch_matvec_waves(type_id, (uint32_t)vocab, (uint32_t)cols, nb);
+    for (uint32_t done = 0u, nb; done < batch; done += nb) {
+        uint32_t w_nb;
+        nb = kq_launch_matvec_columns(type_id, (uint32_t)vocab, (uint32_t)cols, batch - done);
+        w_nb = kq_launch_matvec_waves(type_id, (uint32_t)vocab, (uint32_t)cols, nb);
         if (w_nb > nparts) nparts = w_nb;
     }
     if (nparts == 0u)

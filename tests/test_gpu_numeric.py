@@ -449,6 +449,67 @@ def test_matvec_q6k_batched_mfma_fails_closed(ctx, cols):
                  exact=exact.matvec(kq_oracle.Q6_K, w, rows, cols, x))
 
 
+@pytest.mark.parametrize("fmt,rows,cols,batch", [
+    (f, r, c, b) for f in ALL_FMTS for r, c, b in (
+        (1, 256, 5), (33, 768, 8), (17, 2816, 6), (257, 6144, 5), (4099, 2560, 8), (40, 10240, 7))
+] + [(f, r, c, b) for f in ("Q8_0", "Q5_1", "IQ4_NL") for r, c, b in (
+        (31, 320, 1), (129, 3136, 8), (16, 64, 5), (20, 96, 6))])
+def test_matvec_tiles(ctx, fmt, rows, cols, batch):
+    # five columns and more (and rows of odd widths) run on the matrix-core
+    # tiles: ragged last tiles, 1 .. 40 units of 256 columns in one to five
+    # chunks, a last unit of fewer columns, Q6_K rows that start off a dword
+    # (an odd number of 210-byte blocks), and columns whose magnitudes lie
+    # far apart, one of them all zeros; 96 columns of 34- or 18-byte blocks
+    # stay on the row engine
+    t = FMTS[fmt]
+    key = S.stream_key(S.W_MATVEC_Q6K, 93, rows * 64 + batch, cols // 32)
+    w = S.quant_matrix(fmt, key, rows, cols)
+    x = S.normal_f32(key ^ 0x55, batch * cols).reshape(batch, cols)
+    scale = np.array([1.0, 1e-30, 1e6, 1.0, 3e-5, 1e4, 1.0, 1e-12][:batch])
+    x = (x * scale[:, None].astype(np.float32)).astype(np.float32)
+    if batch > 3:
+        x[3] = 0.0
+    dw, dx, dy = ctx.upload(w), ctx.upload(x), ctx.alloc(rows * batch * 4)
+    ctx.matvec(t, dw, rows, cols, dx, batch, dy)
+    got = ctx.download(dy, np.float32, rows * batch).reshape(batch, rows)
+    want = kq_oracle.matvec(t, w, rows, cols, x, threads=oracle_threads())
+    for b in (dw, dx, dy):
+        b.close()
+    if batch > 3:
+        assert (got[3] == 0.0).all()
+    ex = exact.matvec(t, w, rows, cols, x)
+    inv = 1.0 / scale
+    assert_close(got.astype(np.float64) * inv[:, None], want.astype(np.float64) * inv[:, None],
+                 exact=exact.Exact(lambda i: ex(i) * inv[np.asarray(i) // rows],
+                                   lambda i: ex.scale(i) * inv[np.asarray(i) // rows]))
+
+
+@pytest.mark.parametrize("fmt,cols,field", [("Q4_K", 2560, 2), ("Q5_K", 512, 0), ("Q6_K", 768, 208),
+                                            ("Q8_0", 640, 0), ("Q5_1", 320, 2), ("IQ4_NL", 2112, 0)])
+def test_matvec_tiles_fails_closed(ctx, fmt, cols, field):
+    # a non-finite activation in one column, or block scale in the last row's
+    # last block, fails the call; a following good call is unaffected
+    rows, batch, t = 49, 6, FMTS[fmt]
+    bb = kq_hip.GEOMETRY[t][1]
+    w = S.quant_matrix(fmt, S.stream_key(S.W_MATVEC_Q6K, 94, t), rows, cols)
+    x = S.normal_f32(S.stream_key(S.W_MATVEC_Q6K, 95, t), batch * cols).reshape(batch, cols)
+    x_bad, w_bad = x.copy(), w.copy().reshape(-1, bb)
+    x_bad[5, cols - 1] = np.nan
+    w_bad[-1, field:field + 2] = [0x00, 0x7C]  # +Inf
+    dw, dx, dy = ctx.upload(w), ctx.upload(x), ctx.alloc(rows * batch * 4)
+    dxb, dwb = ctx.upload(x_bad), ctx.upload(w_bad.reshape(-1))
+    for a, b, name in ((dw, dxb, "NUMERIC_DOMAIN"), (dwb, dx, "MALFORMED_QUANTIZED_DATA")):
+        with pytest.raises(kq_hip.KqError) as e:
+            ctx.matvec(t, a, rows, cols, b, batch, dy)
+        assert e.value.name == name
+    ctx.matvec(t, dw, rows, cols, dx, batch, dy)
+    got = ctx.download(dy, np.float32, rows * batch).reshape(batch, rows)
+    assert_close(got, kq_oracle.matvec(t, w, rows, cols, x, threads=oracle_threads()),
+                 exact=exact.matvec(t, w, rows, cols, x))
+    for b in (dw, dx, dy, dxb, dwb):
+        b.close()
+
+
 def test_argmax_exact(ctx):
     rng = np.random.default_rng(9)
     v = rng.standard_normal((3, 151936)).astype(np.float32)
