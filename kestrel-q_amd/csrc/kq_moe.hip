@@ -33,6 +33,7 @@
 #include "kq_launch.h"
 #include "kq_rowdot.h"
 #include "kq_stage.h"
+#include "kq_dma.h"
 
 namespace {
 
@@ -1334,6 +1335,528 @@ __global__ __launch_bounds__(1024) void route_select(RouteArgs a) {
     select_one<HIDDEN>(a);
 }
 
+/* ---------------- routing of several tokens by candidates ---------------- */
+/*
+ * The layer needs the CPU's expert ids exactly, and running every logit's
+ * left-to-right chain for every token costs 2 VALU instructions per token,
+ * expert and column (router_chain_sx: 55 us at 512 tokens x 512 experts x
+ * 2048, 273 at 2499 x 2560, and 52 at 7 tokens, where its 8 workgroups leave
+ * the device idle). But only the few experts near the top can be selected:
+ *
+ *   1. route_prep: every token's row is split into fp16 hi + lo for the
+ *      gate/up pass (which needs that anyway), with its 2-norm and its shared
+ *      gate logit; every router row gets its 2-norm and a power-of-two scale.
+ *   2. route_approx: approximate logits a on the matrix cores, hi and lo
+ *      parts of the tokens against the router rounded to fp16.
+ *   3. route_candidates, one wave per token: |a - l| <= B for the CPU's
+ *      logit l, with B below; L, the k-th largest a - B, bounds the k-th
+ *      largest l from below, so every expert whose a + B lies clearly below L
+ *      (certify_sep's margin: its rounded probability is then strictly below
+ *      the k-th one's) is out. The others, 11 of 512 on N(0, 1) activations
+ *      at k = 10, get the CPU's exact chains, and from those the
+ *      exact expf terms: the selection and its order follow where the terms
+ *      are equal (ids ascending, as the CPU orders equal probabilities) or
+ *      apart by more than the spacing of their quotients by the common sum;
+ *      two terms one step apart, equal terms across the selection's edge,
+ *      probabilities that may underflow and anything non-finite do not decide.
+ *   4. route_fallback: the tokens left undecided (3e-5 of random ones) run
+ *      every chain and the reference's route finish.
+ *
+ * The four launches against the chains and the route finish, us: 7 tokens x
+ * 2560 columns 39 / 64, 201 x 2560 42 / 61, 512 x 2048 45 / 70, 2499 x 2560
+ * 92 / 334. A candidate wave is bound by its chain (8 cycles per dependent
+ * add, 8.5 us at 2560) and the loads that lead up to it.
+ *
+ * The bound. With s = |w| |x| (2-norms), sum |w_i x_i| <= s (Cauchy-Schwarz)
+ * and n columns: the CPU's chain errs by at most n u s (1 + n u), u = 2^-24,
+ * products included. The approximation errs by |dw| |x| for the router's
+ * rounding errors dw (their 2-norm is formed, a third of the 2^-11 |w| it
+ * could be), 2^-21 s for the tokens' split, and by its fp32 accumulation: two
+ * steps of 32 products per 32 columns, each at most 32 2^-24 of its own terms
+ * and 2^-23 of the running sum off, at most (2^-18 + n 2^-27) s; n 2^-25 s is
+ * taken. Together |dw| |x| + (2^-21 + 1.5 n 2^-24) s; B takes 1.02 of that,
+ * plus 2^-20 |a| for the binary32 arithmetic on a and B, plus 1e-37 for
+ * underflow.
+ */
+struct RouteManyArgs {
+    const float *router, *sgw, *x;
+    uint32_t experts, top_k, tokens, hidden;
+    void *stage;        /* kq_stage.h */
+    float4 *row;        /* [experts], of the scaled row: 2-norm, 2-norm of its fp16 rounding
+                           errors, its power of two (int bits) */
+    _Float16 *wh;       /* [experts][hidden]: the scaled router in fp16 */
+    float *parts;       /* approximate logits' parts from the third on */
+    uint32_t splits;
+    float *logits, *shared_logit, *probs;
+    uint32_t *ids;
+    float *weights;
+    uint32_t *order;    /* order[t K] holds token t's scaled 2-norm until its selection is written */
+    float *shared_scale;
+    uint32_t *n_left, *left; /* undecided tokens */
+    uint32_t *status;
+};
+
+constexpr uint32_t kCandMaxK = 32;  /* top_k this route takes */
+constexpr uint32_t kCandMax = 64;   /* candidates per token */
+constexpr uint32_t kCandRows = 16;  /* chains a wave runs at a time */
+constexpr uint32_t kCandDepth = 4;  /* 32-column chunks in flight */
+constexpr uint32_t kRouteSplits = 8; /* their bytes stay below 2^31: 6 x 65536 x 1023 x 4 */
+
+/* the approximate logits' part z, [tokens][experts] in the rows' scales */
+__device__ __forceinline__ float *route_part(float *logits, float *probs, float *parts, uint32_t z,
+                                             size_t values) {
+    float *p = parts + (size_t)(z - 2u) * values;
+    p = z == 1u ? probs : p;
+    return z == 0u ? logits : p;
+}
+
+/* sum over the workgroup of 256 threads, in thread 0 */
+__device__ __forceinline__ float block_sum_256(float v, float *part) {
+    v = wave_sum_f32(v);
+    if ((threadIdx.x & 63u) == 0u) part[threadIdx.x >> 6] = v;
+    __syncthreads();
+    return part[0] + part[1] + part[2] + part[3];
+}
+
+/* grid: tokens + experts workgroups of 256 threads */
+__global__ __launch_bounds__(256) void route_prep(RouteManyArgs a) {
+    __shared__ float part[2][4];
+    __shared__ uint32_t s_max[4];
+    const uint32_t tid = threadIdx.x;
+    if (blockIdx.x < a.tokens) {
+        const uint32_t t = blockIdx.x;
+        const float sq = kq::stage_row(a.x, t, a.tokens, a.hidden, a.stage, a.status);
+        const float4 *xq = (const float4 *)(a.x + (size_t)t * a.hidden);
+        const float4 *gq = (const float4 *)a.sgw;
+        float acc = 0.0f;
+        bool bad = false;
+        for (uint32_t q = tid; q < a.hidden / 4u; q += 256u) {
+            const float4 gv = gq[q], xv = xq[q];
+            bad |= !kq_isfinite(gv.x) || !kq_isfinite(gv.y) || !kq_isfinite(gv.z) ||
+                   !kq_isfinite(gv.w);
+            acc = fmaf(gv.x, xv.x, acc);
+            acc = fmaf(gv.y, xv.y, acc);
+            acc = fmaf(gv.z, xv.z, acc);
+            acc = fmaf(gv.w, xv.w, acc);
+        }
+        const float total = block_sum_256(sq, part[0]), sl = block_sum_256(acc, part[1]);
+        if (tid == 0u) {
+            a.order[(size_t)t * a.top_k] = __float_as_uint(sqrtf(total));
+            a.shared_logit[t] = sl;
+        }
+        if (bad) kq_flag(a.status, KQ_DEV_INPUT);
+        return;
+    }
+    const uint32_t e = blockIdx.x - a.tokens;
+    if (e == 0u && tid == 0u) *a.n_left = 0u;
+    const float4 *row = (const float4 *)(a.router + (size_t)e * a.hidden);
+    uint32_t m = 0u;
+    for (uint32_t q = tid; q < a.hidden / 4u; q += 256u) {
+        const float4 v = row[q];
+        m = max(max(m, __float_as_uint(v.x) & 0x7fffffffu), __float_as_uint(v.y) & 0x7fffffffu);
+        m = max(max(m, __float_as_uint(v.z) & 0x7fffffffu), __float_as_uint(v.w) & 0x7fffffffu);
+    }
+    for (int o = 32; o >= 1; o >>= 1) m = max(m, (uint32_t)__shfl_xor(m, o, 64));
+    if ((tid & 63u) == 0u) s_max[tid >> 6] = m;
+    __syncthreads();
+    m = max(max(s_max[0], s_max[1]), max(s_max[2], s_max[3]));
+    const bool bad = m >= 0x7f800000u;
+    const int r = !bad && m != 0u ? 15 - __builtin_amdgcn_frexp_expf(__uint_as_float(m)) : 0;
+    float sq = 0.0f, er = 0.0f;
+    for (uint32_t q = tid; q < a.hidden / 4u; q += 256u) {
+        const float4 v = row[q];
+        const float f[4] = {ldexpf(v.x, r), ldexpf(v.y, r), ldexpf(v.z, r), ldexpf(v.w, r)};
+        typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+        h4 h;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            h[i] = (_Float16)f[i];
+            const float d = f[i] - (float)h[i]; /* exact */
+            sq = fmaf(f[i], f[i], sq);
+            er = fmaf(d, d, er);
+        }
+        *(h4 *)(a.wh + (size_t)e * a.hidden + 4u * q) = h;
+    }
+    const float total = block_sum_256(sq, part[0]), errs = block_sum_256(er, part[1]);
+    if (tid == 0u) {
+        a.row[e] = float4{bad ? __builtin_inff() : sqrtf(total), sqrtf(errs), __int_as_float(r), 0.0f};
+        if (bad) kq_flag(a.status, KQ_DEV_INPUT);
+    }
+}
+
+/* Approximate logits of 64 tokens x TN experts per workgroup, over one of
+ * `splits` runs of columns (grid z; route_candidates adds their parts). The
+ * split rows come 64 columns at a time through an LDS ring, each row's 128
+ * bytes by eight lanes of a 16-byte LDS-DMA load, two chunks ahead of the one
+ * being multiplied (fragments straight from memory ran at a third of the
+ * rate: 16 rows an instruction). A row's 16-byte units are permuted by its
+ * low bits, so the 16 rows of a fragment read hit distinct banks. */
+template <uint32_t TN, uint32_t NW>
+__global__ __launch_bounds__(NW * 64u) void route_approx(RouteManyArgs a) {
+    typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    constexpr uint32_t TM = 64u, ROWS = 2u * TM + TN; /* xh, xl, w rows of a chunk */
+    constexpr uint32_t IPW = ROWS / 8u / NW;          /* loads per wave and chunk */
+    static_assert(ROWS % (8u * NW) == 0u, "whole instructions per wave");
+    constexpr uint32_t SLOT = ROWS * 128u, RING = 3u;
+    /* a wave's part: WM tokens x 32 experts */
+    constexpr uint32_t WN = TN / 32u, WM = TM * WN / NW, MF = WM / 16u;
+    __shared__ __align__(16) uint8_t ring[RING][SLOT];
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t j = lane & 15u, g = lane >> 4;
+    const uint32_t t0 = blockIdx.x * TM, e0 = blockIdx.y * TN;
+    const uint32_t H = a.hidden, nch = H / 64u;
+    const uint32_t c_lo = nch * blockIdx.z / gridDim.z, c_hi = nch * (blockIdx.z + 1u) / gridDim.z;
+    const kq::StagedX sx = kq::staged_at(a.stage, a.tokens, H);
+    const kq_i4v bh = dma_rsrc(sx.xh, a.tokens * H * 2u), bl = dma_rsrc(sx.xl, a.tokens * H * 2u);
+    const kq_i4v bw = dma_rsrc(a.wh, a.experts * H * 2u);
+    /* instruction n = w IPW + q: rows 8 n .. 8 n + 7 of [xh | xl | w]; rows
+     * past the tokens or experts read as zeros (or whatever the slot held:
+     * they reach no stored product) */
+    uint32_t off[IPW];
+    kq_i4v rs[IPW];
+#pragma unroll
+    for (uint32_t q = 0; q < IPW; ++q) {
+        const uint32_t r0 = (w * IPW + q) * 8u, r = r0 + (lane >> 3), u = (lane & 7u) ^ (r & 7u);
+        const uint32_t t = t0 + (r & (TM - 1u)), e = e0 + r - 2u * TM;
+        const bool in = r < 2u * TM ? t < a.tokens : e < a.experts;
+        off[q] = in ? (r < 2u * TM ? t : e) * H * 2u + 16u * u : 0x80000000u;
+        kq_i4v v = bw;
+        if (r0 < 2u * TM) v = bl;
+        if (r0 < TM) v = bh;
+        rs[q] = kq_i4v{__builtin_amdgcn_readfirstlane(v.x), __builtin_amdgcn_readfirstlane(v.y),
+                       __builtin_amdgcn_readfirstlane(v.z), __builtin_amdgcn_readfirstlane(v.w)};
+    }
+    auto issue = [&](uint32_t c, uint32_t slot) {
+        const uint32_t dst = __builtin_amdgcn_readfirstlane(lds_addr(&ring[slot][0]) + w * IPW * 1024u);
+#pragma unroll
+        for (uint32_t q = 0; q < IPW; ++q) dma16(rs[q], off[q] + 128u * c, dst + 1024u * q);
+    };
+    const uint32_t m0 = (w / WN) * WM, n0 = 2u * TM + (w % WN) * 32u; /* this wave's rows */
+    f4 acc[MF][2];
+#pragma unroll
+    for (uint32_t m = 0; m < MF; ++m) acc[m][0] = acc[m][1] = f4{0.f, 0.f, 0.f, 0.f};
+    if (c_lo < c_hi) issue(c_lo, 0u);
+    if (c_lo + 1u < c_hi) issue(c_lo + 1u, 1u);
+    uint32_t slot = 0u, next = 2u;
+    for (uint32_t c = c_lo; c < c_hi; ++c) {
+        if (c + 1u < c_hi)
+            wait_vm<(int)IPW>();
+        else
+            wait_vm<0>();
+        kq_lds_barrier();
+        if (c + 2u < c_hi) issue(c + 2u, next);
+        next = next == RING - 1u ? 0u : next + 1u;
+        const uint8_t *p = &ring[slot][0];
+        slot = slot == RING - 1u ? 0u : slot + 1u;
+#pragma unroll
+        for (uint32_t k = 0; k < 2u; ++k) {
+            auto frag = [&](uint32_t row0) {
+                const uint32_t r = row0 + j;
+                return *(const h8 *)(p + r * 128u + 16u * ((4u * k + g) ^ (r & 7u)));
+            };
+            const h8 b0 = frag(n0), b1 = frag(n0 + 16u);
+#pragma unroll
+            for (uint32_t m = 0; m < MF; ++m) {
+                const h8 ah = frag(m0 + 16u * m), al = frag(TM + m0 + 16u * m);
+                acc[m][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, b0, acc[m][0], 0, 0, 0);
+                acc[m][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, b1, acc[m][1], 0, 0, 0);
+                acc[m][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, b0, acc[m][0], 0, 0, 0);
+                acc[m][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, b1, acc[m][1], 0, 0, 0);
+            }
+        }
+    }
+    wait_vm<0>();
+    float *out = route_part(a.logits, a.probs, a.parts, blockIdx.z, (size_t)a.tokens * a.experts);
+#pragma unroll
+    for (uint32_t m = 0; m < MF; ++m)
+#pragma unroll
+        for (uint32_t n = 0; n < 2u; ++n)
+#pragma unroll
+            for (uint32_t q = 0; q < 4u; ++q) {
+                const uint32_t t = t0 + m0 + 16u * m + 4u * g + q;
+                const uint32_t e = e0 + (w % WN) * 32u + 16u * n + j;
+                if (t < a.tokens && e < a.experts) out[(size_t)t * a.experts + e] = acc[m][n][q];
+            }
+}
+
+/* int keys in the order of the floats (no NaN) */
+__device__ __forceinline__ int float_key(float f) {
+    const int i = __float_as_int(f);
+    return i ^ ((i >> 31) & 0x7fffffff);
+}
+
+/* One wave per token, four per workgroup; S: experts per lane (E <= 64 S). */
+template <uint32_t S>
+__global__ __launch_bounds__(256) void route_candidates(RouteManyArgs a) {
+    constexpr uint32_t PITCH = 9u; /* float4 per row of products: conflict-free */
+    __shared__ __align__(16) float4 prods[4][2u * kCandRows * PITCH];
+    __shared__ uint32_t cand[4][kCandMax];
+    __shared__ float exact_l[4][kCandMax];
+    __shared__ float srt_ex[4][kCandMax], srt_l[4][kCandMax];
+    __shared__ uint32_t srt_id[4][kCandMax];
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t t = blockIdx.x * 4u + w;
+    if (t >= a.tokens) return; /* no workgroup barrier below */
+    auto wave_sync = []() {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    auto undecided = [&]() {
+        if (lane == 0u) a.left[atomicAdd(a.n_left, 1u)] = t;
+    };
+    const uint32_t K = a.top_k, H = a.hidden;
+    const kq::StagedX sx = kq::staged_at(a.stage, a.tokens, H);
+    const int sig = sx.sig[t];
+    const float xn = __uint_as_float(a.order[(size_t)t * K]);
+    const float cb = 1.02f * (0x1p-21f + 1.5f * 0x1p-24f * (float)H);
+    constexpr int kNone = (int)0x80000000;
+    float av[S], bv[S];
+    int key[S];
+    bool bad = false;
+    float top = -__builtin_inff();
+    /* every part's logits requested at once: parts past the last read as
+     * zeros (a loop over the parts would wait for memory once a part) */
+    const uint32_t nv = a.tokens * a.experts * 4u;
+    const KqBuf p0 = kq_buf(a.logits, nv), p1 = kq_buf(a.probs, a.splits > 1u ? nv : 0u),
+                p2 = kq_buf(a.parts, a.splits > 2u ? (a.splits - 2u) * nv : 0u);
+    float part[S][kRouteSplits];
+#pragma unroll
+    for (uint32_t s = 0; s < S; ++s) {
+        const uint32_t e = lane + 64u * s;
+        const uint32_t o = e < a.experts ? (t * a.experts + e) * 4u : 0x80000000u;
+        part[s][0] = __uint_as_float(kq_ld32(p0, o, 0u));
+        part[s][1] = __uint_as_float(kq_ld32(p1, o, 0u));
+#pragma unroll
+        for (uint32_t z = 2; z < kRouteSplits; ++z)
+            part[s][z] = __uint_as_float(kq_ld32(p2, z < a.splits ? o + (z - 2u) * nv : 0x80000000u, 0u));
+    }
+#pragma unroll
+    for (uint32_t s = 0; s < S; ++s) {
+        const uint32_t e = lane + 64u * s;
+        av[s] = -__builtin_inff();
+        bv[s] = 0.0f;
+        key[s] = kNone;
+        if (e < a.experts) {
+            const float4 row = a.row[e];
+            const int sc = -(sig + __float_as_int(row.z));
+            float sum = part[s][0];
+#pragma unroll
+            for (uint32_t z = 1; z < kRouteSplits; ++z) sum += part[s][z];
+            av[s] = ldexpf(sum, sc);
+            /* scaled norms below 2^21 each: no overflow before the scale */
+            const float prod = ldexpf(xn * row.x, sc);
+            bv[s] = cb * prod + 1.02f * ldexpf(xn * row.y, sc) + 0x1p-20f * fabsf(av[s]) + 1e-37f;
+            bad |= !kq_isfinite(av[s]) || !(prod < 0x1p120f);
+            key[s] = float_key(av[s] - bv[s]);
+            top = fmaxf(top, av[s]);
+        }
+    }
+    if (sig == kq::kBadRow || __ballot(bad) != 0ull) {
+        undecided();
+        return;
+    }
+    top = wave_max(top);
+    /* L: the K-th largest lower bound, with multiplicity */
+    int kth = kNone;
+    {
+        int c[S];
+#pragma unroll
+        for (uint32_t s = 0; s < S; ++s) c[s] = key[s];
+        uint32_t taken = 0;
+        while (taken < K) {
+            int m = c[0];
+#pragma unroll
+            for (uint32_t s = 1; s < S; ++s) m = max(m, c[s]);
+            kth = wave_imax(m);
+#pragma unroll
+            for (uint32_t s = 0; s < S; ++s) {
+                const bool hit = c[s] == kth;
+                taken += (uint32_t)__popcll(__ballot(hit));
+                c[s] = hit ? kNone : c[s];
+            }
+        }
+    }
+    const float L = __int_as_float(kth ^ ((kth >> 31) & 0x7fffffff));
+    uint32_t n = 0;
+#pragma unroll
+    for (uint32_t s = 0; s < S; ++s) {
+        const uint32_t e = lane + 64u * s;
+        const float ub = av[s] + bv[s];
+        const float margin = 0x1p-19f * (4.0f + fabsf(L - top) + fabsf(ub - top));
+        const bool in = e < a.experts && !(L - ub > margin);
+        const uint64_t m = __ballot(in);
+        const uint32_t at = n + bits_below(m);
+        if (in && at < kCandMax) cand[w][at] = e;
+        n += (uint32_t)__popcll(m);
+    }
+    if (n > kCandMax || !(L - top > -74.0f)) {
+        undecided();
+        return;
+    }
+    wave_sync();
+    /* the candidates' chains, kCandRows at a time, in chunks of 32 columns:
+     * lane 8 rr + q forms the rounded products of columns 4q .. 4q + 3 of rows
+     * rr and rr + 8 into LDS, and lanes r, r + 16, .. add row r's 32 products
+     * in order. A chunk's products are written and requested back while the
+     * chunk before is added: a lone wave would pay the LDS round trip for
+     * every one otherwise. */
+    const uint32_t q = lane & 7u, rr = lane >> 3;
+    float4 *pr = prods[w];
+    const uint32_t nch = H / 32u; /* a multiple of kCandDepth */
+    const KqBuf bx = kq_buf(a.x, a.tokens * H * 4u), br = kq_buf(a.router, a.experts * H * 4u);
+    const uint32_t xo = (t * H + 4u * q) * 4u;
+#pragma unroll 1
+    for (uint32_t p0 = 0; p0 < n; p0 += kCandRows) {
+        const uint32_t r0 = p0 + rr, r1 = r0 + 8u;
+        const uint32_t o0 = (cand[w][r0 < n ? r0 : 0u] * H + 4u * q) * 4u;
+        const uint32_t o1 = (cand[w][r1 < n ? r1 : 0u] * H + 4u * q) * 4u;
+        float4 w0[kCandDepth], w1[kCandDepth], xv[kCandDepth], va[8], vb[8];
+        /* (no branch around a load: chunks past the row read as zeros) */
+        auto load = [&](uint32_t c, uint32_t d) {
+            const uint32_t o = c < nch ? 128u * c : 0x80000000u;
+            xv[d] = __builtin_bit_cast(float4, kq_ld128(bx, xo + o, 0u));
+            w0[d] = __builtin_bit_cast(float4, kq_ld128(br, o0 + o, 0u));
+            w1[d] = __builtin_bit_cast(float4, kq_ld128(br, o1 + o, 0u));
+        };
+        auto turn = [&](uint32_t d, uint32_t buf, float4 (&v)[8]) {
+            float4 *b = pr + buf * (kCandRows * PITCH);
+            const float4 x4 = xv[d];
+            b[rr * PITCH + q] = float4{w0[d].x * x4.x, w0[d].y * x4.y, w0[d].z * x4.z, w0[d].w * x4.w};
+            b[(rr + 8u) * PITCH + q] = float4{w1[d].x * x4.x, w1[d].y * x4.y, w1[d].z * x4.z, w1[d].w * x4.w};
+            wave_sync();
+#pragma unroll
+            for (uint32_t i = 0; i < 8u; ++i) v[i] = b[(lane & 15u) * PITCH + i];
+            wave_sync();
+        };
+#pragma unroll
+        for (uint32_t d = 0; d < kCandDepth; ++d) load(d, d);
+        float acc = 0.0f;
+        turn(0u, 0u, va);
+        load(kCandDepth, 0u);
+#pragma unroll 1
+        for (uint32_t c0 = 0; c0 < nch; c0 += kCandDepth) {
+#pragma unroll
+            for (uint32_t d = 0; d < kCandDepth; ++d) {
+                const uint32_t d1 = (d + 1u) % kCandDepth;
+                if ((d & 1u) != 0u)
+                    turn(d1, 0u, va);
+                else
+                    turn(d1, 1u, vb);
+                load(c0 + d + 1u + kCandDepth, d1);
+#pragma unroll
+                for (uint32_t i = 0; i < 8u; ++i) add4(acc, (d & 1u) ? vb[i] : va[i]);
+            }
+        }
+        if (lane < kCandRows && p0 + lane < n) exact_l[w][p0 + lane] = acc;
+    }
+    wave_sync();
+    const bool have = lane < n;
+    const float l = have ? exact_l[w][lane] : -__builtin_inff();
+    const uint32_t id = have ? cand[w][lane] : 0xffffffffu;
+    const float m = wave_max(l);
+    const float ex = have ? kq_expf(l - m) : -1.0f;
+    uint32_t rank = 0;
+    for (uint32_t i = 0; i < n; ++i) {
+        const float ei = rdl_f32(ex, i);
+        const uint32_t ii = (uint32_t)__builtin_amdgcn_readlane((int)id, (int)i);
+        rank += (uint32_t)(ei > ex || (ei == ex && ii < id));
+    }
+    if (have) {
+        srt_ex[w][rank] = ex;
+        srt_l[w][rank] = l;
+        srt_id[w][rank] = id;
+    }
+    wave_sync();
+    const bool sel = lane < K;
+    const float se = sel ? srt_ex[w][lane] : 0.0f;
+    const uint32_t si = sel ? srt_id[w][lane] : 0xffffffffu;
+    const float ne = lane + 1u < n ? srt_ex[w][lane + 1u] : 0.0f;
+    /* quotients by one sum differ after rounding when they are a unit in
+     * the last place (at most 2^-23 of them) apart */
+    const bool apart = lane + 1u >= n || se - ne > 1.02f * 0x1p-23f * se;
+    const bool ok = !sel || (kq_isfinite(srt_l[w][lane]) && srt_l[w][lane] - m > -75.0f &&
+                             (apart || (lane + 1u < K && se == ne)));
+    if (__ballot(!ok) != 0ull || __ballot(have && !kq_isfinite(l)) != 0ull) {
+        undecided();
+        return;
+    }
+    float sum = 0.0f;
+    uint32_t by_id = 0;
+    for (uint32_t i = 0; i < K; ++i) {
+        sum += rdl_f32(se, i);
+        by_id += (uint32_t)((uint32_t)__builtin_amdgcn_readlane((int)si, (int)i) < si);
+    }
+    if (sel) {
+        const size_t o = (size_t)t * K;
+        a.ids[o + lane] = si;
+        a.weights[o + lane] = se / sum;
+        a.order[o + by_id] = lane;
+    }
+    if (lane == 0u) a.shared_scale[t] = kq_sigmoid(a.shared_logit[t]);
+}
+
+/* the undecided tokens: every chain, then the reference's route finish */
+template <uint32_t HIDDEN>
+__global__ __launch_bounds__(1024) void route_fallback(RouteManyArgs a) {
+    const uint32_t n = *a.n_left;
+    for (uint32_t i = blockIdx.x; i < n; i += gridDim.x) {
+        const uint32_t t = a.left[i];
+        exact_all_rows<HIDDEN>(a.router, a.sgw, a.x + (size_t)t * HIDDEN, a.experts,
+                               a.logits + (size_t)t * a.experts, a.shared_logit + t, a.status);
+        route_finish_body(t, a.logits, a.shared_logit, a.experts, a.top_k, a.probs, a.ids,
+                          a.weights, a.order, a.shared_scale, a.status);
+        __syncthreads();
+    }
+}
+
+/* 64 x 256 tiles read the fewest bytes a product; with fewer than 40 of them
+ * 64 x 64 ones spread over more CUs */
+bool route_wide_tiles(uint32_t tokens, uint32_t experts) {
+    return ((tokens + 63u) / 64u) * ((experts + 255u) / 256u) >= 40u;
+}
+
+/* column runs: enough workgroups for the device, at least two chunks each,
+ * as many parts as there is room for (logits, probs and `room` more) */
+uint32_t route_splits(uint32_t tokens, uint32_t experts, uint32_t hidden, uint64_t room) {
+    const uint32_t tn = route_wide_tiles(tokens, experts) ? 256u : 64u;
+    const uint32_t tiles = ((tokens + 63u) / 64u) * ((experts + tn - 1u) / tn);
+    uint32_t z = (256u + tiles - 1u) / tiles;
+    if (z > hidden / 128u) z = hidden / 128u;
+    if (z > 2u + room) z = 2u + (uint32_t)room;
+    return z > kRouteSplits ? kRouteSplits : z;
+}
+
+hipError_t launch_route_many(const RouteManyArgs &a, hipStream_t s) {
+    hipLaunchKernelGGL(route_prep, dim3(a.tokens + a.experts), dim3(256), 0, s, a);
+    const dim3 ag((a.tokens + 63u) / 64u, (a.experts + 255u) / 256u, a.splits);
+    if (route_wide_tiles(a.tokens, a.experts))
+        hipLaunchKernelGGL((route_approx<256u, 8u>), ag, dim3(512), 0, s, a);
+    else
+        hipLaunchKernelGGL((route_approx<64u, 4u>), dim3(ag.x, (a.experts + 63u) / 64u, ag.z),
+                           dim3(256), 0, s, a);
+    const dim3 grid((a.tokens + 3u) / 4u);
+    if (a.experts <= 64u)
+        hipLaunchKernelGGL(route_candidates<1>, grid, dim3(256), 0, s, a);
+    else if (a.experts <= 512u)
+        hipLaunchKernelGGL(route_candidates<8>, grid, dim3(256), 0, s, a);
+    else
+        hipLaunchKernelGGL(route_candidates<16>, grid, dim3(256), 0, s, a);
+    const dim3 fg(a.tokens < 64u ? a.tokens : 64u);
+    switch (a.hidden) {
+    case 256: hipLaunchKernelGGL(route_fallback<256u>, fg, dim3(1024), 0, s, a); break;
+    case 512: hipLaunchKernelGGL(route_fallback<512u>, fg, dim3(1024), 0, s, a); break;
+    case 1024: hipLaunchKernelGGL(route_fallback<1024u>, fg, dim3(1024), 0, s, a); break;
+    case 2048: hipLaunchKernelGGL(route_fallback<2048u>, fg, dim3(1024), 0, s, a); break;
+    case 2560: hipLaunchKernelGGL(route_fallback<2560u>, fg, dim3(1024), 0, s, a); break;
+    default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
 /* ---------------------- expert gate/up + SwiGLU ---------------------- */
 /* Rows longer than one wave covers (or of a width the row engine has no
  * instance for) are cut into column segments, widest first, one launch
@@ -2120,6 +2643,36 @@ extern "C" hipError_t kq_launch_moe_route(const kq_launch_moe_dims *d, const flo
         }
     }
 #undef KQ_ROUTER_DECODE
+    /* several tokens, only the ids exactly, and a gate/up pass that reads the
+     * split activations (KQ_ROUTE_ONE's hidden sizes): by candidates */
+    if (tokens > 1u && certify && stage != nullptr && d->top_k <= kCandMaxK) {
+        RouteManyArgs a;
+        a.router = router;
+        a.sgw = shared_gate_weight;
+        a.x = hidden;
+        a.experts = d->experts;
+        a.top_k = d->top_k;
+        a.tokens = tokens;
+        a.hidden = d->hidden;
+        a.stage = stage;
+        a.row = (float4 *)ws->bound;
+        a.wh = (_Float16 *)ws->router_t;
+        /* act is the gate/up pass's output: free for the parts until then */
+        const uint64_t ai = d->inter > d->shared_inter ? d->inter : d->shared_inter;
+        a.parts = ws->act;
+        a.splits = route_splits(tokens, d->experts, d->hidden, (d->top_k + 1u) * ai / d->experts);
+        a.logits = ws->logits;
+        a.shared_logit = ws->shared_logit;
+        a.probs = ws->probs;
+        a.ids = ws->ids;
+        a.weights = ws->weights;
+        a.order = ws->order;
+        a.shared_scale = ws->shared_scale;
+        a.n_left = ws->pos;     /* the permutation writes pos and perm_tok later */
+        a.left = ws->perm_tok;
+        a.status = status;
+        return launch_route_many(a, s);
+    }
     /* several tokens: the chains read the router in place and the route
      * finish forms the shared gate's logit */
     const bool in_place = !fused && d->hidden % kSxCols == 0u;

@@ -40,9 +40,10 @@ __device__ __forceinline__ StagedX staged_at(void *base, uint32_t tokens, uint32
 /* Token t's row of X [tokens][k] (k a multiple of 256) scaled by 2^sig,
  * its largest magnitude in [2^14, 2^15), split hi + lo, with its 32-column
  * sums. The whole workgroup takes part (blockDim.x a multiple of 64, at
- * most 1024): each pass gives every wave all or none of its lanes. */
-__device__ __forceinline__ void stage_row(const float *__restrict__ X, uint32_t t, uint32_t tokens,
-                                          uint32_t k, void *staged, uint32_t *status) {
+ * most 1024): each pass gives every wave all or none of its lanes. Returns
+ * this thread's share of the scaled row's sum of squares. */
+__device__ __forceinline__ float stage_row(const float *__restrict__ X, uint32_t t, uint32_t tokens,
+                                           uint32_t k, void *staged, uint32_t *status) {
     typedef _Float16 h4 __attribute__((ext_vector_type(4)));
     __shared__ float s_max[16];
     __shared__ uint32_t s_bad[16];
@@ -74,6 +75,7 @@ __device__ __forceinline__ void stage_row(const float *__restrict__ X, uint32_t 
     int sig = 0;
     if (!bad && m > 0.0f) sig = 15 - __builtin_amdgcn_frexp_expf(m);
     if (bad) sig = kBadRow;
+    float squares = 0.0f;
     for (uint32_t i = threadIdx.x; i < ng; i += blockDim.x) {
         const float4 v = row[i];
         const float a[4] = {v.x, v.y, v.z, v.w};
@@ -85,6 +87,7 @@ __device__ __forceinline__ void stage_row(const float *__restrict__ X, uint32_t 
             hi[c] = (_Float16)xs;
             lo[c] = (_Float16)(xs - (float)hi[c]);
             part += xs;
+            squares = fmaf(xs, xs, squares);
         }
         *(h4 *)(sx.xh + (size_t)t * k + 4u * i) = h4{hi[0], hi[1], hi[2], hi[3]};
         *(h4 *)(sx.xl + (size_t)t * k + 4u * i) = h4{lo[0], lo[1], lo[2], lo[3]};
@@ -106,6 +109,7 @@ __device__ __forceinline__ void stage_row(const float *__restrict__ X, uint32_t 
         sx.sig[t] = sig;
         if (bad) kq_flag(status, KQ_DEV_INPUT);
     }
+    return squares;
 }
 
 }  // namespace kq
