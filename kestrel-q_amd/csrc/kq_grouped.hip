@@ -44,6 +44,7 @@
  * weight bytes are contiguous and share one scale.
  */
 #include "kq_launch.h"
+#include "kq_stage.h"
 #include "kq_device.h"
 #include "kq_dma.h"
 
@@ -791,10 +792,11 @@ __global__ __launch_bounds__(NW * 64) void grouped_pass(
 constexpr uint32_t kPermChunk = 256; /* tokens per rank pass */
 
 /* The Q4_K gate/up pass's work list (kq_grouped_gu.hip, gu_items): one
- * item per kItemRows-token chunk of an expert, routed experts in id order,
+ * item per item_rows-token chunk of an expert, routed experts in id order,
  * then the shared expert's chunks; [0] the count, items from [4] on as
  * (expert | kItemShared, first | count << 24). */
-constexpr uint32_t kItemRows = 16;
+constexpr uint32_t kItemRows = 16;     /* of the 16-token passes */
+constexpr uint32_t kWideItemRows = 64; /* of kq_gemm.hip */
 constexpr uint32_t kItemShared = 0x80000000u;
 
 __global__ __launch_bounds__(1024) void moe_permute(const uint32_t *__restrict__ ids,
@@ -804,8 +806,8 @@ __global__ __launch_bounds__(1024) void moe_permute(const uint32_t *__restrict__
                                                     uint32_t *__restrict__ pos,
                                                     uint32_t *__restrict__ pair_slot,
                                                     uint32_t *status, uint32_t *items,
-                                                    uint32_t with_shared, uint32_t *zero,
-                                                    uint32_t nzero) {
+                                                    uint32_t with_shared, uint32_t item_rows,
+                                                    uint32_t *zero, uint32_t nzero) {
     __shared__ uint32_t cnt[1024];
     __shared__ uint32_t base[1024];
     __shared__ uint32_t bits[1024][kPermChunk / 32u];
@@ -851,7 +853,7 @@ __global__ __launch_bounds__(1024) void moe_permute(const uint32_t *__restrict__
          * the chunks per expert */
         __shared__ uint32_t csum[16];
         const uint32_t c = tid < experts ? cnt[tid] : 0u;
-        const uint32_t nc = (c + kItemRows - 1u) / kItemRows;
+        const uint32_t nc = (c + item_rows - 1u) / item_rows;
         uint32_t incl = nc;
 #pragma unroll
         for (uint32_t o = 1; o < 64u; o <<= 1) {
@@ -869,12 +871,12 @@ __global__ __launch_bounds__(1024) void moe_permute(const uint32_t *__restrict__
         const uint32_t o0 = base[tid];
         for (uint32_t k = 0; k < nc; ++k) {
             list[2u * (ib + k)] = tid;
-            list[2u * (ib + k) + 1u] = (o0 + kItemRows * k) | (min(c - kItemRows * k, kItemRows) << 24);
+            list[2u * (ib + k) + 1u] = (o0 + item_rows * k) | (min(c - item_rows * k, item_rows) << 24);
         }
-        const uint32_t nsh = with_shared ? (tokens + kItemRows - 1u) / kItemRows : 0u;
+        const uint32_t nsh = with_shared ? (tokens + item_rows - 1u) / item_rows : 0u;
         for (uint32_t k = tid; k < nsh; k += 1024u) {
             list[2u * (total + k)] = kItemShared | k;
-            list[2u * (total + k) + 1u] = (kItemRows * k) | (min(tokens - kItemRows * k, kItemRows) << 24);
+            list[2u * (total + k) + 1u] = (item_rows * k) | (min(tokens - item_rows * k, item_rows) << 24);
         }
         if (tid == 0u) items[0] = total + nsh;
     }
@@ -1354,7 +1356,7 @@ extern "C" hipError_t kq_launch_moe_permute(const uint32_t *ids, uint32_t tokens
                                             uint32_t *pair_slot, uint32_t *status,
                                             hipStream_t s) {
     hipLaunchKernelGGL(moe_permute, dim3(1), dim3(1024), 0, s, ids, tokens, top_k, experts,
-                       offsets, pair_token, pos, pair_slot, status, nullptr, 0u, nullptr, 0u);
+                       offsets, pair_token, pos, pair_slot, status, nullptr, 0u, kItemRows, nullptr, 0u);
     return hipGetLastError();
 }
 
@@ -1366,6 +1368,69 @@ extern "C" void *kq_launch_moe_grouped_stage(const kq_launch_moe_dims *d,
                                              const kq_launch_moe_weights *w,
                                              const kq_launch_moe_ws *ws) {
     return gu_lds_routed(d, w) ? (void *)ws->outp : nullptr;
+}
+
+static hipError_t launch_combine(const kq_launch_moe_dims *d, const kq_launch_moe_ws *ws,
+                                 uint32_t tokens, float *out, uint32_t *status, hipStream_t s) {
+    hipLaunchKernelGGL(moe_combine, dim3((d->hidden / 4u + 255u) / 256u, tokens), dim3(256), 0, s,
+                       ws->outp, ws->pos, ws->order, ws->weights, ws->shared_scale, tokens,
+                       d->top_k, d->hidden, out, status);
+    return hipGetLastError();
+}
+
+/* Tokens per expert on average from which the 64-token products (kq_gemm.hip)
+ * are the faster ones. Whole layer, 512 experts, 10 per token, 16-token passes
+ * against them: 2560 x 640 Q4_K / Q5_1 at 16 tokens per expert (820 tokens)
+ * 805 and 848 us, at 19.5 928 and 885, at 49 1979 and 1417; Q5_K / Q8_0 at 16
+ * 872 and 910, at 19.5 1084 and 949. The mixed-tile passes of 2048 x 512 Q4_K /
+ * Q6_K keep up for longer: at 27 692 and 780, at 49 1072 and 996, level near
+ * 39. */
+static const uint32_t kWideTokens = 20u, kWideTokensMixed = 44u;
+
+static bool wide_supported(const kq_launch_moe_dims *d, const kq_launch_moe_weights *w,
+                           uint32_t tokens, bool lds_shared, bool mixed) {
+    const uint32_t npos = tokens * d->top_k + tokens;
+    if (!gu_lds_routed(d, w) ||
+        (uint64_t)tokens * d->top_k < (uint64_t)d->experts * (mixed ? kWideTokensMixed : kWideTokens) ||
+        !kq_launch_gm_gate_up_supported(w->gate_type, d->inter, d->hidden, tokens) ||
+        !kq_launch_gm_matrix_supported(w->down_type, d->hidden, d->inter, npos))
+        return false;
+    if (lds_shared) return w->shared_down_type == w->down_type;
+    return w->shared_gate_type == KQ_LAUNCH_Q8_0 && w->shared_down_type == KQ_LAUNCH_Q8_0 &&
+           kq_launch_gm_matrix_supported(KQ_LAUNCH_Q8_0, d->inter, d->hidden, tokens) &&
+           kq_launch_gm_matrix_supported(KQ_LAUNCH_Q8_0, d->hidden, d->inter, npos);
+}
+
+/* gate/up and down of every position into ws->outp */
+static hipError_t launch_wide(const kq_launch_moe_dims *d, const kq_launch_moe_weights *w,
+                              uint32_t tokens, const kq_launch_moe_ws *ws, bool lds_shared,
+                              uint32_t *status, hipStream_t s) {
+    const size_t tk = (size_t)tokens * d->top_k, npos = tk + tokens;
+    hipError_t e = kq_launch_gm_gate_up(w->gate_type, w->gate, w->up, w->shared_gate, w->shared_up,
+                                        d->inter, d->hidden, ws->outp, tokens, d->top_k,
+                                        ws->perm_tok, ws->gitems, ws->act, status, s);
+    if (e == hipSuccess && !lds_shared) {
+        /* the Q8_0 shared expert from the same split (kq_stage.h), its
+         * gate and up products in dstage, free until the down split */
+        const kq::StagedX st = kq::staged_at(ws->outp, tokens, d->hidden);
+        e = kq_launch_gm_dense(KQ_LAUNCH_Q8_0, w->shared_gate, w->shared_up, d->inter, d->hidden,
+                               st.xh, st.xl, st.sig, tokens, (float *)ws->dstage, status, s);
+        if (e == hipSuccess)
+            e = kq_launch_dense_swiglu((const float *)ws->dstage, 1u, tokens, d->inter,
+                                       ws->act + tk * d->inter, status, s);
+    }
+    _Float16 *xh = (_Float16 *)ws->dstage, *xl = xh + npos * d->inter;
+    int *sig = (int *)(xl + npos * d->inter);
+    if (e == hipSuccess)
+        e = kq_launch_dense_split(ws->act, (uint32_t)npos, d->inter, xh, xl, sig, 0, status, s);
+    if (e == hipSuccess)
+        e = kq_launch_gm_down(w->down_type, w->down, w->shared_down, d->hidden, d->inter, xh, xl,
+                              sig, tokens, d->top_k, ws->gitems, ws->outp, status, s);
+    if (e == hipSuccess && !lds_shared)
+        e = kq_launch_gm_dense(KQ_LAUNCH_Q8_0, w->shared_down, nullptr, d->hidden, d->inter,
+                               xh + tk * d->inter, xl + tk * d->inter, sig + tk, tokens,
+                               ws->outp + tk * d->hidden, status, s);
+    return e;
 }
 
 extern "C" hipError_t kq_launch_moe_grouped(const kq_launch_moe_dims *d,
@@ -1386,11 +1451,13 @@ extern "C" hipError_t kq_launch_moe_grouped(const kq_launch_moe_dims *d,
     const bool fused_split = lds_shared && d->hidden == 2048u && d->inter == 512u &&
                              w->down_type == KQ_LAUNCH_Q6_K &&
                              w->shared_down_type == KQ_LAUNCH_Q6_K;
-    uint32_t *posmax = fused_split ? (uint32_t *)ws->dstage : nullptr;
+    /* many tokens per expert: 64 of them against each decoded weight */
+    const bool wide = wide_supported(d, w, tokens, lds_shared, fused_split);
+    uint32_t *posmax = fused_split && !wide ? (uint32_t *)ws->dstage : nullptr;
     hipLaunchKernelGGL(moe_permute, dim3(1), dim3(1024), 0, s, ws->ids, tokens, d->top_k,
                        d->experts, ws->offsets, ws->perm_tok, ws->pos, nullptr, status,
                        lds_routed ? (uint32_t *)ws->gitems : nullptr, lds_shared ? 1u : 0u,
-                       posmax, posmax != nullptr ? tokens * (d->top_k + 1u) : 0u);
+                       wide ? kWideItemRows : kItemRows, posmax, posmax != nullptr ? tokens * (d->top_k + 1u) : 0u);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     const uint8_t *g = (const uint8_t *)w->gate, *u = (const uint8_t *)w->up;
@@ -1402,6 +1469,11 @@ extern "C" hipError_t kq_launch_moe_grouped(const kq_launch_moe_dims *d,
     if (lds_routed && !staged) {
         e = kq_launch_gu_stage(hidden, tokens, d->hidden, ws->outp, status, s);
         if (e != hipSuccess) return e;
+    }
+    if (wide) {
+        e = launch_wide(d, w, tokens, ws, lds_shared, status, s);
+        if (e != hipSuccess) return e;
+        return launch_combine(d, ws, tokens, out, status, s);
     }
     if (lds_routed) {
         e = kq_launch_gu_lds(w->gate_type, d->hidden, g, u, sg, su, ws->outp, ws->offsets,
@@ -1507,10 +1579,7 @@ extern "C" hipError_t kq_launch_moe_grouped(const kq_launch_moe_dims *d,
         }
     }
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(moe_combine, dim3((d->hidden / 4u + 255u) / 256u, tokens), dim3(256), 0, s,
-                       ws->outp, ws->pos, ws->order, ws->weights, ws->shared_scale, tokens,
-                       d->top_k, d->hidden, out, status);
-    return hipGetLastError();
+    return launch_combine(d, ws, tokens, out, status, s);
 }
 
 /* y[t] = W x[t] for every token: a Q8_0 matrix against many activation

@@ -224,6 +224,26 @@ hipError_t kq_launch_dn_lds(uint32_t inter, uint32_t hidden, const void *down,
                             uint32_t top_k, const void *items, void *staged,
                             const uint32_t *posmax, float *out, uint32_t *status,
                             hipStream_t s);
+/* prefill products for many tokens per expert (kq_gemm.hip): up to 64 tokens
+ * of an expert per item (items as kq_launch_gu_lds's, of 64 tokens). Gate/up
+ * in Q4_K or Q5_K from the staged split, positions in permuted order; down in
+ * Q5_1, Q6_K or Q8_0 from the positions' split (xh, xl [tokens * (top_k + 1)]
+ * [k], sig); dense: one matrix (w1 null) or two against every row, out
+ * [tokens][rows] or [tokens][2 rows]. */
+int kq_launch_gm_gate_up_supported(uint32_t type, uint32_t rows, uint32_t k, uint32_t tokens);
+int kq_launch_gm_matrix_supported(uint32_t type, uint32_t rows, uint32_t k, uint32_t src_rows);
+hipError_t kq_launch_gm_gate_up(uint32_t type, const void *gate, const void *up,
+                                const void *shared_gate, const void *shared_up, uint32_t rows,
+                                uint32_t k, const void *staged, uint32_t tokens, uint32_t top_k,
+                                const uint32_t *perm_tok, const void *items, float *act,
+                                uint32_t *status, hipStream_t s);
+hipError_t kq_launch_gm_down(uint32_t type, const void *down, const void *shared_down,
+                             uint32_t rows, uint32_t k, const void *xh, const void *xl,
+                             const int *sig, uint32_t tokens, uint32_t top_k, const void *items,
+                             float *out, uint32_t *status, hipStream_t s);
+hipError_t kq_launch_gm_dense(uint32_t type, const void *w0, const void *w1, uint32_t rows,
+                              uint32_t k, const void *xh, const void *xl, const int *sig,
+                              uint32_t tokens, float *out, uint32_t *status, hipStream_t s);
 /* where the Q4_K / Q5_K gate/up pass reads its per-token activation split (ws's
  * outp), or NULL when these weights take another pass; the route can form
  * it (kq_launch_moe_route's stage), and staged tells the grouped path so */

@@ -44,50 +44,15 @@
 #include "kq_launch.h"
 #include "kq_device.h"
 #include "kq_dma.h"
+#include "kq_mfma.h"
 
 namespace {
 
-typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-typedef float f4 __attribute__((ext_vector_type(4)));
+using namespace kq::mf;
 
 constexpr uint32_t kT = 16;      /* rows per tile */
-constexpr uint32_t kUnit = 256;  /* columns per unit */
 constexpr uint32_t kCols = 8;    /* activation columns */
 constexpr uint32_t kMaxPd = 4;   /* chunks in flight, at most */
-
-__device__ __forceinline__ h2 as_h2(uint32_t u) { return __builtin_bit_cast(h2, u); }
-/* bytes 0, 1 / 2, 3 of m as fp16 1024 + byte */
-__device__ __forceinline__ h2 bytes_lo(uint32_t m) {
-    return as_h2(__builtin_amdgcn_perm(0x64646464u, m, 0x04010400u));
-}
-__device__ __forceinline__ h2 bytes_hi(uint32_t m) {
-    return as_h2(__builtin_amdgcn_perm(0x64646464u, m, 0x04030402u));
-}
-/* and as the subnormals byte 2^-24 */
-__device__ __forceinline__ h2 tiny_lo(uint32_t m) {
-    return as_h2(__builtin_amdgcn_perm(0u, m, 0x04010400u));
-}
-__device__ __forceinline__ h2 tiny_hi(uint32_t m) {
-    return as_h2(__builtin_amdgcn_perm(0u, m, 0x04030402u));
-}
-__device__ __forceinline__ h2 fma2(h2 a, h2 b, h2 c) { return __builtin_elementwise_fma(a, b, c); }
-__device__ __forceinline__ h2 splat(float v) { return h2{(_Float16)v, (_Float16)v}; }
-__device__ __forceinline__ h8 cat(h2 a, h2 b, h2 c, h2 d) {
-    return h8{a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y};
-}
-__device__ __forceinline__ float half_bits(uint32_t h) { return kq_f16_to_f32_hw(h); }
-/* bits 0..3 of x (x < 16) to bit 4 of bytes 0..3 */
-__device__ __forceinline__ uint32_t spread4(uint32_t x) {
-    return (kq_mul_u24(x, 0x00204081u) & 0x01010101u) << 4;
-}
-__device__ __forceinline__ f4 mfma32(h8 a, h8 b, f4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ f4 mfma16(h4 a, h4 b, f4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x16f16(a, b, c, 0, 0, 0);
-}
 
 /* eight halves as four packed registers from here on: without the asm the
  * compiler keeps the unpacked values and packs them again at every use */
@@ -101,22 +66,6 @@ __device__ __forceinline__ uint32_t ror8(uint32_t x) {
 }
 __device__ __forceinline__ float ror8(float x) { return __uint_as_float(ror8(__float_as_uint(x))); }
 __device__ __forceinline__ uint32_t mag(float x) { return __float_as_uint(x) & 0x7fffffffu; }
-
-constexpr bool is_k(uint32_t f) { return f == KQ_LAUNCH_Q4_K || f == KQ_LAUNCH_Q5_K; }
-
-/* bytes of 256 columns */
-constexpr uint32_t unit_bytes(uint32_t f) {
-    return f == KQ_LAUNCH_Q4_K ? 144u
-           : f == KQ_LAUNCH_Q5_K ? 176u
-           : f == KQ_LAUNCH_Q6_K ? 210u
-           : f == KQ_LAUNCH_Q8_0 ? 272u
-           : f == KQ_LAUNCH_Q5_1 ? 192u
-           : f == KQ_LAUNCH_IQ4_NL ? 144u : 0u;
-}
-/* columns per block */
-constexpr uint32_t block_cols(uint32_t f) {
-    return is_k(f) || f == KQ_LAUNCH_Q6_K ? 256u : 32u;
-}
 
 /* The column of its unit that lane k-group g's element e of operand step s
  * stands for. A step's k order is free as long as both operands agree; it
@@ -163,47 +112,17 @@ __device__ __forceinline__ f4 unit_product(const uint8_t *p, uint32_t off, uint3
         }
         const float d = half_bits(hd.x), dmin = half_bits(hd.x >> 16);
         malformed |= real && (!kq_isfinite(d) || !kq_isfinite(dmin));
-        uint32_t s0, s1, m0u, m1u;
-        kq_k_scale_pair(g, hd.y, hd.z, hd.w, &s0, &m0u, &s1, &m1u);
-        /* a code byte under a zero high byte is the subnormal q 2^-24 (16 q
-         * for Q4_K's high nibbles, left in place); one fused multiply-add
-         * makes it (q - c) s 2^-14 with c the middle of the codes' range:
-         * exact, at most 1008 2^-14. The codes' mean thus stays out of the
-         * long sums; c s comes back beside the mins. */
-        constexpr float kMid = Q5 ? 16.0f : 8.0f;
-        const h2 S0 = splat((float)s0 * 1024.0f), S1 = splat((float)s1 * (Q5 ? 1024.0f : 64.0f));
-        const h2 C0 = splat((float)s0 * (-kMid * 0x1p-14f)), C1 = splat((float)s1 * (-kMid * 0x1p-14f));
-        /* scales and mins 4g .. 4g + 3 for g < 2, zero for the others */
-        const uint32_t k0 = 0u - (uint32_t)(g == 0u), k01 = 0u - (uint32_t)(g < 2u);
-        const uint32_t mq = ((hd.z & 0x3f3f3f3fu) & k0) |
-                            ((((hd.w >> 4) & 0x0f0f0f0fu) | ((hd.z >> 2) & 0x30303030u)) & ~k0);
-        const uint32_t sq = ((hd.y & 0x3f3f3f3fu) & k0) |
-                            (((hd.w & 0x0f0f0f0fu) | ((hd.y >> 2) & 0x30303030u)) & ~k0);
-        const h2 neg = splat(-1024.0f);
-        auto ints = [&](uint32_t q) {
-            return __builtin_bit_cast(h4, make_uint2(__builtin_bit_cast(uint32_t, bytes_lo(q) + neg) & k01,
-                                                     __builtin_bit_cast(uint32_t, bytes_hi(q) + neg) & k01));
-        };
+        constexpr float kMid = k_mid(FMT);
+        /* k-group g: sub-blocks 2g (steps 0..3) and 2g + 1 (steps 4..7) */
+        const KPair<FMT, true> sc(hd, g);
 #pragma unroll
-        for (uint32_t s = 0; s < 8u; ++s) {
-            const uint4 &qd = (s & 2u) ? qb : qa;
-            const uint32_t r0 = (s & 1u) ? qd.z : qd.x, r1 = (s & 1u) ? qd.w : qd.y;
-            uint32_t m0, m1;
-            if constexpr (Q5) {
-                const uint4 &hq = (s & 2u) ? hb : ha;
-                const uint32_t h0 = (s & 1u) ? hq.z : hq.x, h1 = (s & 1u) ? hq.w : hq.y;
-                const uint32_t sh = s < 4u ? 2u * g : 2u * g + 1u;
-                m0 = ((s < 4u ? r0 : r0 >> 4) & 0x0f0f0f0fu) | (((h0 >> sh) & 0x01010101u) << 4);
-                m1 = ((s < 4u ? r1 : r1 >> 4) & 0x0f0f0f0fu) | (((h1 >> sh) & 0x01010101u) << 4);
-            } else {
-                m0 = s < 4u ? kq_and_0f(r0) : kq_and_f0(r0);
-                m1 = s < 4u ? kq_and_0f(r1) : kq_and_f0(r1);
-            }
-            const h2 S = s < 4u ? S0 : S1, C = s < 4u ? C0 : C1;
-            acc = mfma32(A[s], cat(fma2(tiny_lo(m0), S, C), fma2(tiny_hi(m0), S, C),
-                                   fma2(tiny_lo(m1), S, C), fma2(tiny_hi(m1), S, C)), acc);
-        }
-        const f4 mm = mfma16(sums, ints(mq), zero), ss = mfma16(sums, ints(sq), zero);
+        for (uint32_t s = 0; s < 8u; ++s)
+            acc = mfma32(A[s], sc.weights(s >> 2, g, dword_of(qa, qb, s & 3u, 0u), dword_of(qa, qb, s & 3u, 1u),
+                                          dword_of(ha, hb, s & 3u, 0u), dword_of(ha, hb, s & 3u, 1u)),
+                         acc);
+        const uint32_t k01 = 0u - (uint32_t)(g < 2u);
+        const f4 mm = mfma16(sums, byte_halves(k_mins(hd, g) & k01), zero);
+        const f4 ss = mfma16(sums, byte_halves(k_scales(hd, g) & k01), zero);
         /* the sums carry 2^-5 */
         const float dw = d * 0x1p14f, dc = d * (kMid * 32.0f), dm = dmin * 32.0f;
 #pragma unroll

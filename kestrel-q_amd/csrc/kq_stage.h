@@ -24,7 +24,7 @@ struct StagedX {
     int *sig;
 };
 
-__device__ __forceinline__ StagedX staged_at(void *base, uint32_t tokens, uint32_t k) {
+__host__ __device__ __forceinline__ StagedX staged_at(void *base, uint32_t tokens, uint32_t k) {
     StagedX s;
     uint8_t *p = (uint8_t *)base;
     s.xh = (_Float16 *)p;

@@ -687,6 +687,27 @@ def test_moe_prefill_grouped_formats(ctx, H, E, K, I, T, g, d, sg, sd):
         b.close()
 
 
+# 20 and more tokens per expert on average (44 at 2048 x 512): up to 64 of them against each
+# decoded weight. Items of one to four 16-token fragments, an expert's second
+# item, the last of its tokens alone in one; row tiles that the rows do not
+# fill; every down format; a shared expert in the item list and beside it.
+@pytest.mark.parametrize("H,E,K,I,T,g,d,sg,sd", [
+    (2560, 16, 4, 640, 83, "Q4_K", "Q5_1", "Q8_0", "Q8_0"),
+    (2560, 8, 4, 640, 67, "Q5_K", "Q8_0", "Q8_0", "Q8_0"),
+    (2048, 16, 4, 512, 180, "Q4_K", "Q6_K", "Q4_K", "Q6_K"),
+    (512, 3, 1, 512, 197, "Q4_K", "Q6_K", "Q4_K", "Q6_K"),
+    (256, 5, 2, 640, 129, "Q5_K", "Q5_1", "Q5_K", "Q5_1"),
+    (256, 4, 2, 512, 41, "Q4_K", "Q8_0", "Q4_K", "Q8_0"),
+    (1024, 4, 4, 640, 65, "Q4_K", "Q5_1", "Q4_K", "Q5_1"),
+], ids=["2560-q5_1", "2560-q5k-q8_0", "2048-q6_k", "512-q6_k", "256-q5k-q5_1", "256-q8_0",
+        "all-65"])
+def test_moe_prefill_many_per_expert(ctx, H, E, K, I, T, g, d, sg, sd):
+    seed = S.W_MOE + 7000 + H + I + T
+    out, ids, ref, tr, ex = run_layer(ctx, H, E, K, I, T, g, d, sg, sd, seed)
+    assert np.array_equal(ids, tr["selected_ids"])
+    assert_close(out, ref, exact=ex)
+
+
 def test_moe_reference_model_prefill_512(ctx):
     # The reference model's MoE layer (2560 / 512 experts / top-10 / 640,
     # Q4_K gate/up, Q5_1 down, Q8_0 shared) over 512 tokens: the grouped
