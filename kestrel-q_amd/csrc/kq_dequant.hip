@@ -20,13 +20,14 @@
 namespace {
 
 constexpr int kThreads = 256;
-constexpr uint64_t kMaxBlocks = 256 * 16;
+constexpr uint64_t kMaxBlocks = 256 * 64;
 
 /* 4 floats at byte offset o of the output buffer; stores at or past its
  * end are dropped by the hardware */
-__device__ __forceinline__ void store4(KqBuf ob, uint32_t o, float a, float b, float c, float d) {
+template <int AUX>
+__device__ __forceinline__ void store4(KqBufA<AUX> ob, uint32_t o, float a, float b, float c, float d) {
     kq_u32x4 v = {__float_as_uint(a), __float_as_uint(b), __float_as_uint(c), __float_as_uint(d)};
-    __builtin_amdgcn_raw_buffer_store_b128(v, ob.r, (int)o, 0, 0);
+    __builtin_amdgcn_raw_buffer_store_b128(v, ob.r, (int)o, 0, AUX);
 }
 
 /*
@@ -63,7 +64,8 @@ struct DeqQ4K {
         r.q = kq_ld32(b, o + qoff, 0u);
         return r;
     }
-    __device__ void emit(const Raw &r, uint32_t s, bool valid, KqBuf out, bool &bad) const {
+    template <int AUX>
+    __device__ void emit(const Raw &r, uint32_t s, bool valid, KqBufA<AUX> out, bool &bad) const {
         const float d = kq_f16_to_f32(r.hd.x & 0xffffu);
         const float dmin = kq_f16_to_f32(r.hd.x >> 16);
         bad |= valid && (!kq_isfinite(d) || !kq_isfinite(dmin));
@@ -107,7 +109,8 @@ struct DeqQ5K {
         r.h = kq_ld32(b, o + hoff, 0u);
         return r;
     }
-    __device__ void emit(const Raw &r, uint32_t s, bool valid, KqBuf out, bool &bad) const {
+    template <int AUX>
+    __device__ void emit(const Raw &r, uint32_t s, bool valid, KqBufA<AUX> out, bool &bad) const {
         const float d = kq_f16_to_f32(r.hd.x & 0xffffu);
         const float dmin = kq_f16_to_f32(r.hd.x >> 16);
         bad |= valid && (!kq_isfinite(d) || !kq_isfinite(dmin));
@@ -154,7 +157,8 @@ struct DeqQ6K {
         r.d = kq_ld16(b, o + 208u, 0u);
         return r;
     }
-    __device__ void emit(const Raw &r, uint32_t s, bool valid, KqBuf out, bool &bad) const {
+    template <int AUX>
+    __device__ void emit(const Raw &r, uint32_t s, bool valid, KqBufA<AUX> out, bool &bad) const {
         const float d = kq_f16_to_f32(r.d);
         bad |= valid && !kq_isfinite(d);
         const uint32_t ql = kq_align2(r.ql.y, r.ql.x, r.sh);
@@ -190,7 +194,8 @@ struct DeqQ8 {
         r.d = kq_ld16(b, o, 0u);
         return r;
     }
-    __device__ void emit(const Raw &r, uint32_t s, bool valid, KqBuf out, bool &bad) const {
+    template <int AUX>
+    __device__ void emit(const Raw &r, uint32_t s, bool valid, KqBufA<AUX> out, bool &bad) const {
         const uint32_t blk = 8u * s + (lane >> 3);
         const float d = kq_f16_to_f32(r.d);
         bad |= valid && !kq_isfinite(d);
@@ -232,7 +237,8 @@ struct DeqQ51 {
         r.q = kq_ld32(b, p + 8u + 4u * k, 0u);
         return r;
     }
-    __device__ void emit(const Raw &r, uint32_t s, bool valid, KqBuf out, bool &bad) const {
+    template <int AUX>
+    __device__ void emit(const Raw &r, uint32_t s, bool valid, KqBufA<AUX> out, bool &bad) const {
         const uint32_t blk = 8u * s + (lane >> 3);
         const float d = kq_f16_to_f32(r.dm & 0xffffu);
         const float m = kq_f16_to_f32(r.dm >> 16);
@@ -278,7 +284,8 @@ struct DeqIQ4NL {
         r.d = kq_ld16(b, p, 0u);
         return r;
     }
-    __device__ void emit(const Raw &r, uint32_t s, bool valid, KqBuf out, bool &bad) const {
+    template <int AUX>
+    __device__ void emit(const Raw &r, uint32_t s, bool valid, KqBufA<AUX> out, bool &bad) const {
         const uint32_t blk = 8u * s + (lane >> 3);
         const float d = kq_f16_to_f32(r.d);
         bad |= valid && !kq_isfinite(d);
@@ -301,7 +308,15 @@ struct DeqIQ4NL {
  * that no dword of the last block straddles it. */
 constexpr uint32_t kUnroll = 4u;
 
-template <class D>
+/* The write stream bounds this (five to nine bytes out per byte in). An output
+ * that the L2s (8 x 4 MB) cannot hold anyway is stored non-temporally: a
+ * plain store first takes a line there and evicts another. Q6_K, 2^18 blocks
+ * (323 MB moved) 79 -> 47 us (4.1 -> 6.9 TB/s), 100000 blocks 29.5 -> 19.1,
+ * 32768 (33 MB out) 8.4 -> 7.0; 8192 4.2 and 4.2, so smaller outputs stay in
+ * the caches for whoever reads them next. */
+constexpr uint64_t kNtBytes = UINT64_C(1) << 25;
+
+template <class D, int AUX>
 __global__ __launch_bounds__(kThreads) void dequant_blocks(const uint8_t *__restrict__ packed,
                                                            uint32_t blocks,
                                                            float *__restrict__ out,
@@ -312,7 +327,7 @@ __global__ __launch_bounds__(kThreads) void dequant_blocks(const uint8_t *__rest
     const uint32_t steps = (blocks + D::kPerStep - 1u) / D::kPerStep;
     const KqBuf b = kq_buf(packed, (blocks * D::kBytes + 3u) & ~3u);
     /* outputs of blocks past the end fall outside this buffer */
-    const KqBuf ob = kq_buf(out, blocks * D::kOut * 4u);
+    const KqBufA<AUX> ob = kq_buf<AUX>(out, blocks * D::kOut * 4u);
     D dec;
     dec.setup(lane);
     bool bad = false;
@@ -371,7 +386,8 @@ hipError_t launch_blocks(const uint8_t *p, uint64_t blocks, float *out, uint32_t
     for (uint64_t done = 0; done < blocks; done += kChunk) {
         const uint64_t n = blocks - done < kChunk ? blocks - done : kChunk;
         const uint64_t steps = (n + D::kPerStep - 1u) / D::kPerStep;
-        hipLaunchKernelGGL(dequant_blocks<D>, dim3(grid_for((steps + kUnroll - 1u) / kUnroll)),
+        const auto kernel = blocks * kOut * 4u >= kNtBytes ? dequant_blocks<D, kKqNt> : dequant_blocks<D, 0>;
+        hipLaunchKernelGGL(kernel, dim3(grid_for((steps + kUnroll - 1u) / kUnroll)),
                            dim3(kThreads), 0, stream, p + done * D::kBytes, (uint32_t)n,
                            out + done * kOut, status);
         const hipError_t e = hipGetLastError();

@@ -87,6 +87,18 @@ def test_dequant_ragged_block_counts(ctx, fmt):
         assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), (fmt, n)
 
 
+@pytest.mark.parametrize("fmt", ALL_FMTS)
+def test_dequant_around_nontemporal_outputs(ctx, fmt):
+    # outputs of 32 MiB and more are stored non-temporally
+    gen, qk, bb = S.BLOCK_GEN[fmt]
+    at = (1 << 25) // (4 * qk)
+    for n in (at - 1, at, at + 3):
+        packed = gen(S.stream_key(S.W_DEQUANT, 61, FMTS[fmt], n), n).reshape(-1)
+        got = gpu_dequant(ctx, FMTS[fmt], packed)
+        want = kq_oracle.dequantize(FMTS[fmt], packed)
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
 def test_dequant_subnormal_and_edge_scales(ctx):
     # Q4_K blocks whose d/dmin are fp16 subnormals, zero, negative zero and
     # the largest finite half; Q6_K/Q8_0 with subnormal d.
