@@ -751,7 +751,13 @@ static uint32_t row_launches(uint32_t type, uint32_t cols, uint32_t batch) {
  *     about 4,096 (4000 x 2560: 8.4 / 6.8; 1000 rows: 5.4 / 6.6) up to 4,096
  *     columns (4000 x 6144: 12.1 / 14.4); the other formats at 2 columns and
  *     all at one stay (40000 x 2048, 2 columns: Q8_0 16.1 / 18.6, Q4_K
- *     13.1 / 15.6). */
+ *     13.1 / 15.6).
+ * The 151936 x 2048 Q6_K head at 2 .. 4 columns is the one place where an
+ * earlier kernel, made for 4 columns of that width, was a little faster (whole
+ * call 61.3, 60.9, 62.4 against 64.1, 62.2, 64.9; level at 70001 rows, 25.4 ..
+ * 35.9 against 22.6 .. 23.0 at 40000): its step held two sub-blocks of 4
+ * columns where a tile's holds one of 8. 5 columns took it 106, 8 112; a tile
+ * pass takes 63 and 65. */
 static bool use_tiles(uint32_t type, uint32_t rows, uint32_t cols, uint32_t batch) {
     if (!kq_launch_mv_tiles_supported(type, rows, cols, batch)) return false;
     if (batch > 4u) return true;
