@@ -43,7 +43,7 @@ hipError_t kq_launch_matvec(uint32_t type, const void *W, uint32_t rows, uint32_
  * parts: argmax partials per column, one per workgroup; same partials
  * contract */
 int kq_launch_mv_tiles_supported(uint32_t type, uint32_t rows, uint32_t cols, uint32_t batch);
-uint32_t kq_launch_mv_tiles_parts(uint32_t type, uint32_t rows, uint32_t cols);
+uint32_t kq_launch_mv_tiles_parts(uint32_t type, uint32_t rows, uint32_t cols, uint32_t batch);
 hipError_t kq_launch_mv_tiles(uint32_t type, const void *W, uint32_t rows, uint32_t cols,
                               const float *x, uint32_t batch, float *y, uint32_t *status,
                               float *part_v, uint32_t *part_i, uint32_t part_stride,

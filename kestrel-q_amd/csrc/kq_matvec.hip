@@ -775,7 +775,7 @@ extern "C" uint32_t kq_launch_matvec_columns(uint32_t type, uint32_t rows, uint3
 
 extern "C" uint32_t kq_launch_matvec_waves(uint32_t type, uint32_t rows, uint32_t cols,
                                            uint32_t batch) {
-    if (use_tiles(type, rows, cols, batch)) return kq_launch_mv_tiles_parts(type, rows, cols);
+    if (use_tiles(type, rows, cols, batch)) return kq_launch_mv_tiles_parts(type, rows, cols, batch);
     uint32_t waves = 0u;
     if (dispatch(type, nullptr, rows, cols, nullptr, batch, nullptr, nullptr, nullptr, nullptr,
                  0u, nullptr, &waves) != hipSuccess)

@@ -81,14 +81,20 @@ __device__ __forceinline__ uint32_t k_scales(const uint4 hd, uint32_t h) {
     return ((hd.y & 0x3f3f3f3fu) & k0) |
            (((hd.w & 0x0f0f0f0fu) | ((hd.y >> 2) & 0x30303030u)) & ~k0);
 }
+/* the scales of the sub-blocks that have a min, 0 of the others */
+__device__ __forceinline__ uint32_t k_centres(const uint4 hd, uint32_t h) {
+    const uint32_t some = ((k_mins(hd, h) + 0x7f7f7f7fu) & 0x80808080u) >> 7;
+    return k_scales(hd, h) & ((some << 8) - some);
+}
 
 /* The scales of sub-blocks 2 pair and 2 pair + 1 of a Q4_K or Q5_K block, the
  * low and the high nibbles of bytes 32 pair .. + 31. A code byte under a zero
  * high byte is the subnormal q 2^-24 (16 q for Q4_K's high nibbles, left in
  * place); one fused multiply-add makes it (q - c) s 2^-14: exact. CENTRED: c
  * is the middle of the codes' range (at most 1008 2^-14), their mean stays out
- * of the long sums and c s comes back beside the mins; otherwise c is 0 (at
- * most 1953 2^-14). */
+ * of the long sums and c s comes back beside the mins (k_centres); otherwise,
+ * and in sub-blocks without a min, whose zero codes are zero weights, c is 0
+ * (at most 1953 2^-14). */
 template <uint32_t FMT, bool CENTRED>
 struct KPair {
     h2 S[2], C[2];
@@ -99,8 +105,8 @@ struct KPair {
         kq_k_scale_pair(pair, hd.y, hd.z, hd.w, &s0, &m0, &s1, &m1);
         S[0] = splat((float)s0 * 1024.0f);
         S[1] = splat((float)s1 * (FMT == KQ_LAUNCH_Q5_K ? 1024.0f : 64.0f));
-        C[0] = splat(CENTRED ? (float)s0 * c : 0.0f);
-        C[1] = splat(CENTRED ? (float)s1 * c : 0.0f);
+        C[0] = splat(CENTRED && m0 != 0u ? (float)s0 * c : 0.0f);
+        C[1] = splat(CENTRED && m1 != 0u ? (float)s1 * c : 0.0f);
     }
     /* the weights of eight columns of sub-block 2 pair + high: r0, r1 their
      * qs bytes, h0, h1 their qh bytes (Q5_K) */

@@ -1,6 +1,7 @@
 /*
- * kq_mvtiles.hip — y = W x for 2 to 8 activation columns on the matrix
- * cores: GGUF Q4_K, Q5_K, Q6_K, Q8_0, Q5_1 and IQ4_NL rows.
+ * kq_mvtiles.hip — y = W x on the matrix cores: GGUF Q4_K, Q5_K, Q6_K, Q8_0,
+ * Q5_1 and IQ4_NL rows, 2 to 8 activation columns (and one column of widths
+ * that the row engine takes in several launches).
  *
  * Restates the row loop of kq_weight_provider_linear_f32
  * (src/kq_weight_provider.c:464-475) for several activation vectors.
@@ -10,36 +11,44 @@
  * that reads the weights again. Here the weights are read and decoded once
  * for up to eight columns:
  *
- *   - One 16x16x32 fp16 step multiplies 16 weight rows by 16 operand rows:
- *     rows 0..7 hold the hi parts of the eight columns, rows 8..15 their lo
- *     parts (x = hi + lo to ~23 bits after an exact power-of-two scaling per
- *     column and 256-column unit), so one step serves all the columns.
+ *   - One 16x16x32 fp16 step multiplies 16 weight rows by 16 operand rows,
+ *     which hold the columns in parts (Rows, below): four columns in four
+ *     parts each, the binary32 values exactly; eight columns in two parts
+ *     (~23 bits) where the row engine rounds its columns too, or in four on
+ *     two operands where it does not. The values are scaled by a power of two
+ *     per column and 256-column unit.
  *   - A workgroup walks a contiguous run of 16-row tiles. A row is cut into
  *     units of 256 columns; wave w multiplies unit c nw + w of every row in
- *     the tile's c-th of NC chunks. Its activation operand, 32 registers a
- *     unit, is built once and stays in registers for the whole run.
+ *     the tile's c-th of NC chunks. Its activation operands, 32 registers a
+ *     unit each, are built once and stay in registers for the whole run.
  *   - A chunk (16 rows x nw units) is copied into an LDS ring by 16-byte
  *     LDS-DMA loads spread over the waves, PD chunks ahead of the one being
  *     multiplied. Rows sit at an odd pitch of 16-byte units, so the 16 rows
  *     a step reads hit distinct banks.
- *   - Each wave adds its hi and lo product rows and leaves 8 columns x 16
- *     rows in LDS; after the next barrier 128 threads add the waves in
+ *   - Each wave adds its parts' product rows and leaves its columns x 16 rows
+ *     in LDS; after the next barrier 16 threads a column add the waves in
  *     order, store, and keep the argmax partials: one per workgroup and
  *     column.
  *
- * Codes enter fp16 exactly. Q4_K and Q5_K fold the 6-bit sub-block scale
- * into the weight (at most 1953, exact) and take their mins off with one
- * small step against the columns' sub-block sums; Q6_K takes one 16x16x16
- * step per 16-column sub-block, the 32-weight formats one 16x16x32 step per
- * block, scaled in fp32.
+ * A scale of 256 columns loses what lies far below the unit's largest value.
+ * Columns that hold such values (least_value(), least_group()) are found while
+ * the operand is built, and the workgroups then multiply the rows in binary32
+ * on the vector ALU (10240 x 2560 Q8_0, 8 columns: 99 us; row engine 74).
+ *
+ * Codes enter fp16 exactly. Q4_K and Q5_K fold the 6-bit sub-block scale into
+ * the weight, taken from the middle of the codes' range (at most 1008, exact),
+ * and add the mins and the middle with two small steps against the columns'
+ * sub-block sums; Q6_K takes one 16x16x16 step per 16-column sub-block, the
+ * 32-weight formats one 16x16x32 step per block, scaled in fp32.
  *
  * Bound: HBM for matrices that fill the device, the first loads' latency
- * and the operand's build below that. Against the row engine (and, for Q6_K
- * heads of 2 to 4 columns, the per-format matrix-core kernels that this one
- * replaced at equal times): 10240 x 2560 Q8_0 at 8 columns 76.7 -> 11.8 us
- * (2.4 TB/s), the 248320 x 2560 Q8_0 head at 5 columns 269 -> 140 us
- * (4.8 TB/s). Error against binary64 sums 0.8-1.5e-7 of the result in every
- * format (row engine 1.7-5.7e-7).
+ * and the operand's build below that. Against the row engine: 10240 x 2560
+ * Q8_0 at 8 columns 76.7 -> 11.9 us (2.4 TB/s), the 248320 x 2560 Q8_0 head
+ * at 5 columns 273 -> 136 us (5.0 TB/s). Two operands keep one workgroup per
+ * CU: 40000 x 2048 at 8 columns, Q5_K 23 us (row engine 53), Q5_1 37
+ * (46). Error against binary64 sums of normal
+ * activations 0.7-1.3e-7 of the result in every format (row engine
+ * 1.7-5.7e-7).
  */
 #include "kq_launch.h"
 #include "kq_device.h"
@@ -52,6 +61,7 @@ using namespace kq::mf;
 
 constexpr uint32_t kT = 16;      /* rows per tile */
 constexpr uint32_t kCols = 8;    /* activation columns */
+constexpr int kTiny = 24;        /* the last two parts carry 2^24 */
 constexpr uint32_t kMaxPd = 4;   /* chunks in flight, at most */
 
 /* eight halves as four packed registers from here on: without the asm the
@@ -60,12 +70,75 @@ __device__ __forceinline__ h8 pinned(uint32_t x, uint32_t y, uint32_t z, uint32_
     asm volatile("" : "+v"(x), "+v"(y), "+v"(z), "+v"(w));
     return __builtin_bit_cast(h8, kq_u32x4{x, y, z, w});
 }
-/* the value of lane l ^ 8 (a rotation by 8 within the row of 16 lanes) */
-__device__ __forceinline__ uint32_t ror8(uint32_t x) {
-    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x128, 0xf, 0xf, true);
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp(uint32_t x) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xf, 0xf, true);
 }
+/* the value of lane l ^ 8 (a rotation by 8 within the row of 16 lanes) */
+__device__ __forceinline__ uint32_t ror8(uint32_t x) { return dpp<0x128>(x); }
 __device__ __forceinline__ float ror8(float x) { return __uint_as_float(ror8(__float_as_uint(x))); }
+/* of lanes l ^ 1 and l ^ 2 */
+__device__ __forceinline__ uint32_t quad1(uint32_t x) { return dpp<0xb1>(x); }
+__device__ __forceinline__ uint32_t quad2(uint32_t x) { return dpp<0x4e>(x); }
+__device__ __forceinline__ float quad1(float x) { return __uint_as_float(quad1(__float_as_uint(x))); }
+__device__ __forceinline__ float quad2(float x) { return __uint_as_float(quad2(__float_as_uint(x))); }
 __device__ __forceinline__ uint32_t mag(float x) { return __float_as_uint(x) & 0x7fffffffu; }
+
+/* maximum over the four lanes (i, 0 .. 3), or over (i, g) and (i, g ^ 1) */
+__device__ __forceinline__ uint32_t max16(uint32_t v) {
+    const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    return max((uint32_t)r[0], (uint32_t)r[1]);
+}
+__device__ __forceinline__ uint32_t max_groups(uint32_t v) {
+    v = max16(v);
+    const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    return max((uint32_t)r[0], (uint32_t)r[1]);
+}
+
+/* Two binary32 values (at most 2^15) as N halves each, v = p0 + p1 + 2^-24 (p2 +
+ * p3). N = 4: exact where |v| is 0 or at least 2^-25, whose last bit is 2^-48;
+ * below that the error is at most 2^-49. N = 2: to 2^-23 |v| or 2^-25, the
+ * larger. (The differences are exact.) */
+template <int N>
+__device__ __forceinline__ void split(float a, float b, h2 (&p)[N]) {
+    typedef float f2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+        p[n] = __builtin_convertvector((f2{a, b}), h2);
+        a = fmaf((float)p[n].x, -1.0f, a);
+        b = fmaf((float)p[n].y, -1.0f, b);
+        if (n == 1) {
+            a *= 0x1p24f;
+            b *= 0x1p24f;
+        }
+    }
+}
+
+/* How the 16 operand rows hold the columns.
+ *   kQuad: 4 columns, rows 4c .. 4c + 3 the parts of column c.
+ *   kEight: 8 columns on two operands: rows 0 .. 7 parts 0 (first operand) and
+ *     1 (second), rows 8 .. 15 parts 2 and 3.
+ *   kPair: 8 columns, rows 0 .. 7 part 0, rows 8 .. 15 part 1, nothing more.
+ * The row engine multiplies Q4_K, Q6_K and Q8_0 with 23-bit integers in a
+ * scale per 16 columns, the other formats with the binary32 values; more than
+ * four columns of the former take kPair, of the latter kEight. */
+enum Rows : uint32_t { kQuad, kPair, kEight };
+constexpr bool is_binary32(uint32_t f) {
+    return f == KQ_LAUNCH_Q5_K || f == KQ_LAUNCH_Q5_1 || f == KQ_LAUNCH_IQ4_NL;
+}
+constexpr uint32_t columns_of(Rows m) { return m == kQuad ? 4u : 8u; }
+constexpr uint32_t operands_of(Rows m) { return m == kEight ? 2u : 1u; }
+
+/* What the operands take, in the scaled values (largest in [2^14, 2^15)). Four
+ * parts hold a value as binary32 does down to least_value(), two the values of
+ * 8 columns as a scale per 16 does if one of them reaches least_group(); so do
+ * four parts the sums of such columns, which are scaled down again. Anything
+ * smaller but zeros goes to the binary32 rows. */
+constexpr float least_value() { return 0x1p-25f; }
+template <uint32_t FMT, Rows M>
+constexpr float least_group() {
+    return M == kPair ? 0x1p-2f : is_k(FMT) ? 0x1p-20f : FMT == KQ_LAUNCH_Q5_1 ? 0x1p-16f : 0.0f;
+}
 
 /* The column of its unit that lane k-group g's element e of operand step s
  * stands for. A step's k order is free as long as both operands agree; it
@@ -83,22 +156,43 @@ __device__ __forceinline__ uint32_t column_of(uint32_t g, uint32_t s, uint32_t e
 }
 
 /* what a unit's min term needs of the columns: their sub-block sums times
- * 2^-5, sums 4g .. 4g + 3 on k-groups 0 and 1 (Q4_K, Q5_K); their block sums
+ * 2^-5, sums 4g .. 4g + 3 on k-groups 0 and 1 (Q4_K, Q5_K; kPair: their parts
+ * 2 and 3 times 2^-13 on k-groups 2 and 3, against mins times 2^-11); their block sums
  * times 2^-9 on k-groups 0 and 1 (against m) and times 16 2^-9 on 2 and 3
  * (against d, for the codes' middle 16) (Q5_1) */
 constexpr bool has_min(uint32_t f) { return is_k(f) || f == KQ_LAUNCH_Q5_1; }
 
-/* One unit of row j of the tile times the activation operand: returns
- * lane (j, g)'s products of operand rows 4g .. 4g + 3 in the operand's
- * scale. p: the unit's first byte in LDS (p - off is 4-byte aligned, off 0
+/* IQ4_NL: the values of four nibbles (src/kq_numeric.c) plus 128 */
+__device__ __forceinline__ uint32_t iq4_codes(uint32_t n) {
+    const uint32_t lo = __builtin_amdgcn_perm(0x766a5d4fu, 0x3f2d1801u, n & 0x07070707u);
+    const uint32_t hi = __builtin_amdgcn_perm(0xf1d9c5b5u, 0xa6998d81u, n & 0x07070707u);
+    const uint32_t b3 = (n >> 3) & 0x01010101u, m = (b3 << 8) - b3;
+    return (hi & m) | (lo & ~m);
+}
+
+/* One unit of row j of the tile times the activation operands: returns
+ * lane (j, g)'s products of operand rows 4g .. 4g + 3, summed over the G
+ * operands, in the operand's scale. p: the unit's first byte in LDS (p - off is 4-byte aligned, off 0
  * or 2); live: steps that hold columns (8 but for
  * a row's last unit); real: row j exists. */
-template <uint32_t FMT>
+template <uint32_t FMT, Rows M, uint32_t G>
 __device__ __forceinline__ f4 unit_product(const uint8_t *p, uint32_t off, uint32_t g,
-                                           uint32_t live, bool real, const h8 (&A)[8], h4 sums,
-                                           bool &malformed) {
+                                           uint32_t live, bool real, const h8 (&A)[G][8],
+                                           const h4 (&sums)[G], bool &malformed) {
     const f4 zero = {0.f, 0.f, 0.f, 0.f};
+    /* the operands' products apart: chained, Q5_1 errs by a tenth more */
+    auto step = [&](uint32_t s, h8 b) {
+        f4 t = mfma32(A[0][s], b, zero);
+        if constexpr (G == 2u) t += mfma32(A[1][s], b, zero);
+        return t;
+    };
+    auto min_step = [&](h4 b) {
+        f4 t = mfma16(sums[0], b, zero);
+        if constexpr (G == 2u) t += mfma16(sums[1], b, zero);
+        return t;
+    };
     f4 acc = zero;
+    static_assert(G == 1u || is_binary32(FMT), "two operands hold binary32 values");
     if constexpr (is_k(FMT)) {
         constexpr bool Q5 = FMT == KQ_LAUNCH_Q5_K;
         constexpr uint32_t QS = Q5 ? 48u : 16u;
@@ -115,14 +209,28 @@ __device__ __forceinline__ f4 unit_product(const uint8_t *p, uint32_t off, uint3
         constexpr float kMid = k_mid(FMT);
         /* k-group g: sub-blocks 2g (steps 0..3) and 2g + 1 (steps 4..7) */
         const KPair<FMT, true> sc(hd, g);
+        f4 t[G];
 #pragma unroll
-        for (uint32_t s = 0; s < 8u; ++s)
-            acc = mfma32(A[s], sc.weights(s >> 2, g, dword_of(qa, qb, s & 3u, 0u), dword_of(qa, qb, s & 3u, 1u),
-                                          dword_of(ha, hb, s & 3u, 0u), dword_of(ha, hb, s & 3u, 1u)),
-                         acc);
-        const uint32_t k01 = 0u - (uint32_t)(g < 2u);
-        const f4 mm = mfma16(sums, byte_halves(k_mins(hd, g) & k01), zero);
-        const f4 ss = mfma16(sums, byte_halves(k_scales(hd, g) & k01), zero);
+        for (uint32_t o = 0; o < G; ++o) t[o] = zero;
+#pragma unroll
+        for (uint32_t s = 0; s < 8u; ++s) {
+            const h8 b = sc.weights(s >> 2, g, dword_of(qa, qb, s & 3u, 0u), dword_of(qa, qb, s & 3u, 1u),
+                                    dword_of(ha, hb, s & 3u, 0u), dword_of(ha, hb, s & 3u, 1u));
+#pragma unroll
+            for (uint32_t o = 0; o < G; ++o) t[o] = mfma32(A[o][s], b, t[o]);
+        }
+        acc = t[0];
+        if constexpr (G == 2u) acc += t[1];
+        auto halves = [&](uint32_t b) {
+            if constexpr (M == kPair) {
+                const _Float16 f = g < 2u ? (_Float16)1.0f : (_Float16)0x1p-11f;
+                return byte_halves(b) * h4{f, f, f, f};
+            } else {
+                return byte_halves(g < 2u ? b : 0u);
+            }
+        };
+        const f4 mm = min_step(halves(k_mins(hd, g & 1u)));
+        const f4 ss = min_step(halves(k_centres(hd, g & 1u)));
         /* the sums carry 2^-5 */
         const float dw = d * 0x1p14f, dc = d * (kMid * 32.0f), dm = dmin * 32.0f;
 #pragma unroll
@@ -151,10 +259,10 @@ __device__ __forceinline__ f4 unit_product(const uint8_t *p, uint32_t off, uint3
 #pragma unroll
                 for (uint32_t k = 0; k < 4u; ++k) {
                     const uint32_t i = 8u * n + 4u * h + k;
-                    const h8 &as = A[i >> 1];
+                    const h2 w0 = bytes_lo(c[k]) + bias, w1 = bytes_hi(c[k]) + bias;
+                    const h8 &as = A[0][i >> 1];
                     const h4 a4 = (i & 1u) ? h4{as[4], as[5], as[6], as[7]}
                                            : h4{as[0], as[1], as[2], as[3]};
-                    const h2 w0 = bytes_lo(c[k]) + bias, w1 = bytes_hi(c[k]) + bias;
                     const f4 t = mfma16(a4, h4{w0.x, w0.y, w1.x, w1.y}, zero);
                     const uint32_t sub = 2u * k + h; /* of this half's eight */
                     const int8_t s8 = (int8_t)((sc[sub >> 2] >> (8u * (sub & 3u))) & 0xffu);
@@ -169,8 +277,9 @@ __device__ __forceinline__ f4 unit_product(const uint8_t *p, uint32_t off, uint3
         const uint32_t *w = (const uint32_t *)p;
         uint32_t mins[4] = {0u, 0u, 0u, 0u};
         const uint32_t shn = g >= 2u ? 4u : 0u; /* Q5_1, IQ4_NL: this lane's nibbles */
-        /* Q5_1 codes enter as q - 16; 16 d joins the min */
-        const h2 bias = splat(FMT == KQ_LAUNCH_Q5_1 ? -1040.0f : -1152.0f);
+        /* Q5_1 codes enter as q - 16 and 16 d joins the min; as q where there is
+         * none, whose zero codes are zero weights */
+        h2 bias = splat(FMT == KQ_LAUNCH_Q5_1 ? -1040.0f : -1152.0f);
 #pragma unroll
         for (uint32_t s = 0; s < 8u; ++s) {
             uint32_t c0, c1;
@@ -201,8 +310,10 @@ __device__ __forceinline__ f4 unit_product(const uint8_t *p, uint32_t off, uint3
                 malformed |= real && s < live && (!kq_isfinite(d) || !kq_isfinite(half_bits(dm >> 16)));
                 /* min term: m of blocks 4g .. 4g + 3 (g < 2), then d of
                  * blocks 4 (g - 2) .. */
+                const bool zero_min = (dm & 0x7fff0000u) == 0u;
+                bias = splat(zero_min ? -1024.0f : -1040.0f);
                 if (s < live)
-                    mins[s & 3u] = (s >> 2) == (g & 1u) ? (g < 2u ? dm >> 16 : dm & 0xffffu)
+                    mins[s & 3u] = (s >> 2) == (g & 1u) ? (g < 2u ? dm >> 16 : zero_min ? 0u : dm & 0xffffu)
                                                         : mins[s & 3u];
             } else {
                 /* block s at byte 18 s: this lane's eight nibbles at
@@ -220,31 +331,78 @@ __device__ __forceinline__ f4 unit_product(const uint8_t *p, uint32_t off, uint3
                     q1 = b[2u + 2u * (g & 1u)];
                 }
                 malformed |= real && s < live && !kq_isfinite(d);
-                /* the 16 values (src/kq_numeric.c, IQ4_NL) plus 128 */
-                auto look = [](uint32_t n) {
-                    const uint32_t lo = __builtin_amdgcn_perm(0x766a5d4fu, 0x3f2d1801u, n & 0x07070707u);
-                    const uint32_t hi = __builtin_amdgcn_perm(0xf1d9c5b5u, 0xa6998d81u, n & 0x07070707u);
-                    const uint32_t b3 = (n >> 3) & 0x01010101u, m = (b3 << 8) - b3;
-                    return (hi & m) | (lo & ~m);
-                };
-                c0 = look((q0 >> shn) & 0x0f0f0f0fu);
-                c1 = look((q1 >> shn) & 0x0f0f0f0fu);
+                c0 = iq4_codes((q0 >> shn) & 0x0f0f0f0fu);
+                c1 = iq4_codes((q1 >> shn) & 0x0f0f0f0fu);
             }
             if (s >= live) d = 0.0f;
-            const f4 t = mfma32(A[s], cat(bytes_lo(c0) + bias, bytes_hi(c0) + bias,
-                                          bytes_lo(c1) + bias, bytes_hi(c1) + bias), zero);
+            const f4 t = step(s, cat(bytes_lo(c0) + bias, bytes_hi(c0) + bias, bytes_lo(c1) + bias,
+                                     bytes_hi(c1) + bias));
 #pragma unroll
             for (int k = 0; k < 4; ++k) acc[k] = fmaf(d, t[k], acc[k]);
         }
         if constexpr (FMT == KQ_LAUNCH_Q5_1) {
             const h4 bm = __builtin_bit_cast(
                 h4, make_uint2((mins[0] & 0xffffu) | (mins[1] << 16), (mins[2] & 0xffffu) | (mins[3] << 16)));
-            const f4 mm = mfma16(sums, bm, zero);
+            const f4 mm = min_step(bm);
 #pragma unroll
             for (int k = 0; k < 4; ++k) acc[k] = fmaf(0x1p9f, mm[k], acc[k]);
         }
         return acc;
     }
+}
+
+/* the decoded weights of columns c .. c + 3 of a row (c a multiple of 4), as
+ * the CPU decodes them (src/kq_numeric.c) */
+template <uint32_t FMT>
+__device__ __forceinline__ void weights_at(const uint8_t *row, uint32_t c, float (&w)[4], bool &malformed) {
+    auto half = [&](const uint8_t *p) {
+        const float v = half_bits((uint32_t)p[0] | ((uint32_t)p[1] << 8));
+        malformed |= !kq_isfinite(v);
+        return v;
+    };
+    auto dword = [](const uint8_t *p) {
+        uint32_t v;
+        __builtin_memcpy(&v, p, 4);
+        return v;
+    };
+    constexpr uint32_t BC = block_cols(FMT);
+    const uint8_t *b = row + c / BC * (unit_bytes(FMT) / (kUnit / BC));
+    const uint32_t i = c % BC, sub = i >> 5, l = i & 31u;
+    uint32_t q; /* four codes */
+    float d, m = 0.0f, zero = 0.0f;
+    if constexpr (is_k(FMT)) {
+        const uint8_t *s = b + 4u;
+        const uint32_t sc = sub < 4u ? s[sub] & 63u : (s[sub + 4u] & 15u) | (s[sub - 4u] >> 6 << 4);
+        const uint32_t mn = sub < 4u ? s[sub + 4u] & 63u : (s[sub + 4u] >> 4) | (s[sub] >> 6 << 4);
+        q = (dword(b + (FMT == KQ_LAUNCH_Q5_K ? 48u : 16u) + 32u * (sub >> 1) + l) >> (4u * (sub & 1u))) &
+            0x0f0f0f0fu;
+        if constexpr (FMT == KQ_LAUNCH_Q5_K) q |= ((dword(b + 16u + l) >> sub) & 0x01010101u) << 4;
+        d = half(b) * (float)sc;
+        m = -(half(b + 2) * (float)mn);
+    } else if constexpr (FMT == KQ_LAUNCH_Q6_K) {
+        const uint32_t n = i >> 7, k = sub & 3u;
+        q = ((dword(b + 64u * n + 32u * (k & 1u) + l) >> (2u * (k & 2u))) & 0x0f0f0f0fu) |
+            (((dword(b + 128u + 32u * n + l) >> (2u * k)) & 0x03030303u) << 4);
+        zero = 32.0f;
+        d = half(b + 208) * (float)(int8_t)b[192u + 8u * n + 2u * k + (l >> 4)];
+    } else if constexpr (FMT == KQ_LAUNCH_Q8_0) {
+        q = dword(b + 2u + l) ^ 0x80808080u;
+        zero = 128.0f;
+        d = half(b);
+    } else {
+        const uint32_t nib = (dword(b + (FMT == KQ_LAUNCH_Q5_1 ? 8u : 2u) + (l & 15u)) >> (l >= 16u ? 4u : 0u)) &
+                             0x0f0f0f0fu;
+        d = half(b);
+        if constexpr (FMT == KQ_LAUNCH_Q5_1) {
+            q = nib | spread4((dword(b + 4u) >> l) & 15u);
+            m = half(b + 2);
+        } else {
+            q = iq4_codes(nib);
+            zero = 128.0f;
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) w[e] = d * ((float)((q >> (8 * e)) & 0xffu) - zero) + m;
 }
 
 /* larger value wins, equal values keep the lower row */
@@ -266,7 +424,17 @@ struct MvtArgs {
     uint32_t *part_i;
     uint32_t part_stride;
     uint32_t pitch, slot, pd; /* LDS: 16-byte units per row, bytes per chunk slot; slots - 1 */
+    uint32_t tiles, more;     /* tiles = grid size * tiles + more */
 };
+
+/* The kernel's arguments, loaded where they are used: what only the rare or last
+ * parts of the kernel read stays out of the scalar registers before them (21
+ * of those were spilled otherwise, some in the loop). */
+__device__ __forceinline__ const MvtArgs *late_args() {
+    auto p = (const __attribute__((address_space(4))) MvtArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return (const MvtArgs *)p;
+}
 
 /* LDS-DMA instructions per wave and chunk: a chunk's 16 rows take at most
  * nw unit_bytes / 16 + 2 units each, 64 units an instruction, nw waves */
@@ -275,17 +443,18 @@ constexpr uint32_t ipw() {
     return (unit_bytes(FMT) + 32u + 63u) / 64u;
 }
 
-/* Register budget: 10 waves of up to 168 registers for one or two units a
- * wave, 8 of up to 256 for more. */
-constexpr uint32_t kWideNc = 3u;
-template <uint32_t NC>
+/* Register budget: 10 waves of up to 168 registers while a wave holds at most
+ * two operands of 32, 8 of up to 256 above. */
+constexpr uint32_t kNarrow = 2u;
+template <uint32_t NC, Rows M>
 constexpr int max_threads() {
-    return NC < kWideNc ? 640 : 512;
+    return NC * operands_of(M) <= kNarrow ? 640 : 512;
 }
 
 /* PART: the row's last unit holds fewer than 256 columns */
-template <uint32_t FMT, uint32_t NC, bool PART>
-__global__ __launch_bounds__((max_threads<NC>())) void mv_tiles(MvtArgs a) {
+template <uint32_t FMT, uint32_t NC, bool PART, Rows M>
+__global__ __launch_bounds__((max_threads<NC, M>())) void mv_tiles(MvtArgs a) {
+    constexpr uint32_t KC = columns_of(M), G = operands_of(M);
     constexpr uint32_t UB = unit_bytes(FMT), IPW = ipw<FMT>();
     extern __shared__ __align__(16) uint8_t lds[];
     const uint32_t nw = blockDim.x >> 6;
@@ -293,14 +462,16 @@ __global__ __launch_bounds__((max_threads<NC>())) void mv_tiles(MvtArgs a) {
     const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t j = lane & 15u, g = lane >> 4;
     /* ring, landing place of the padding loads, partial sums by tile parity
-     * [2][nw][8][16], the units' powers of two [NC][nw][8] */
+     * [2][nw][KC][16], the units' powers of two [NC][nw][KC], which waves hold
+     * values out of the operand's reach */
     uint8_t *ring = lds, *trash = ring + (a.pd + 1u) * a.slot;
     float *part = (float *)(trash + 1024u);
-    int *sigs = (int *)(part + 2u * nw * 128u);
+    int *sigs = (int *)(part + 2u * nw * (KC * 16u));
+    uint32_t *deeps = (uint32_t *)(sigs + NC * nw * KC);
 
-    const uint32_t ntiles = (a.rows + kT - 1u) / kT;
-    const uint32_t lo = (uint32_t)((uint64_t)ntiles * blockIdx.x / gridDim.x);
-    const uint32_t hi = (uint32_t)((uint64_t)ntiles * (blockIdx.x + 1u) / gridDim.x);
+    /* the first `more` workgroups walk one tile more than the others */
+    const uint32_t lo = a.tiles * blockIdx.x + min(blockIdx.x, a.more);
+    const uint32_t hi = lo + a.tiles + (blockIdx.x < a.more ? 1u : 0u);
     const uint32_t n_ent = (hi - lo) * NC;
     const kq_i4v wr = dma_rsrc(a.W, a.w_bytes);
     const uint32_t nu = (a.cols + kUnit - 1u) / kUnit;
@@ -334,124 +505,229 @@ __global__ __launch_bounds__((max_threads<NC>())) void mv_tiles(MvtArgs a) {
     /* the first chunk now, the others once the operand's activations have
      * arrived: loads return in order, and behind a full ring the activations
      * would wait for it */
-    if (n_ent != 0u) issue();
+    issue();
 
-    /* the activation operand of this wave's units: lane (i, g) holds operand
-     * row i, hi (i < 8) or lo of column i & 7. Lanes i and i + 8 split the
-     * column's values between them (elements 0..3 and 4..7 of each step)
-     * and trade their lo and hi halves: each value is scaled and split once
-     * (768 -> 350 VALU instructions a unit, which the smallest products
-     * feel). */
-    h8 A[NC][8];
-    h4 sums[NC];
-    bool bad = false;
+    /* the activation operands of this wave's units: lane (i, g) holds operand
+     * row i of k-group g. The lanes that hold parts of one column (kQuad: four
+     * neighbours; else lanes i and i + 8) divide its values between them and
+     * trade their parts, so each value is scaled and split once (768 -> 350
+     * VALU instructions a unit of kPair, which the smallest products feel).
+     * kQuad: steps 2 q and 2 q + 1 on lane q of the four; else elements 4 q ..
+     * 4 q + 3 of every step on lane i + 8 q. */
+    h8 A[NC][G][8];
+    h4 sums[NC][G];
+    bool bad = false, deep = false;
     {
-        const uint32_t i = lane & 15u, col = i & 7u, half = i >> 3;
+        constexpr uint32_t NV = M == kQuad ? 4u : 8u; /* float4 a lane loads and splits */
+        constexpr int NP = M == kPair ? 2 : 4;        /* parts */
+        const uint32_t i = lane & 15u;
+        const uint32_t col = M == kQuad ? i >> 2 : i & 7u, q = M == kQuad ? i & 3u : i >> 3;
+        const bool q0 = (q & 1u) != 0u, q1 = (q & 2u) != 0u;
         /* columns past the row, and columns past the batch, read as zeros */
         const KqBuf bx = kq_buf(a.x, a.batch * a.cols * 4u);
-        auto load = [&](uint32_t c, uint4 (&v)[8]) {
+        auto load = [&](uint32_t c, uint4 (&v)[NV]) {
             const uint32_t u = c * nw + w, xo = (col * a.cols + kUnit * u) * 4u;
             const uint32_t left = u < nu && col < a.batch ? a.cols - kUnit * u : 0u;
 #pragma unroll
-            for (uint32_t s = 0; s < 8u; ++s) {
-                const uint32_t at = half ? column_of<FMT>(g, s, 4u) : column_of<FMT>(g, s, 0u);
-                v[s] = kq_ld128(bx, at < left ? xo + 4u * at : 0x80000000u, 0u);
+            for (uint32_t k = 0; k < NV; ++k) {
+                const uint32_t at = M == kQuad ? column_of<FMT>(g, 2u * q + (k >> 1), 4u * (k & 1u))
+                                    : q0       ? column_of<FMT>(g, k, 4u)
+                                               : column_of<FMT>(g, k, 0u);
+                v[k] = kq_ld128(bx, at < left ? xo + 4u * at : 0x80000000u, 0u);
             }
         };
-        uint4 vn[8];
+        uint4 vn[NV];
         load(0u, vn);
 #pragma unroll
         for (uint32_t c = 0; c < NC; ++c) {
-            float4 v[8];
+            float4 v[NV];
 #pragma unroll
-            for (uint32_t s = 0; s < 8u; ++s) v[s] = __builtin_bit_cast(float4, vn[s]);
+            for (uint32_t k = 0; k < NV; ++k) v[k] = __builtin_bit_cast(float4, vn[k]);
             if (c + 1u < NC) load(c + 1u, vn);
-            uint32_t m = 0u; /* largest magnitude, as bits */
+            /* largest magnitude, and less one the smallest but zero of the
+             * values and of the groups' largest, as bits */
+            uint32_t m = 0u, value1 = 0xffffffffu, group1 = 0xffffffffu, gm[NV];
 #pragma unroll
-            for (uint32_t s = 0; s < 8u; ++s) {
-                m = max(max(m, mag(v[s].x)), mag(v[s].y));
-                m = max(max(m, mag(v[s].z)), mag(v[s].w));
+            for (uint32_t k = 0; k < NV; ++k) {
+                const uint32_t mx = mag(v[k].x), my = mag(v[k].y), mz = mag(v[k].z), mw = mag(v[k].w);
+                gm[k] = max(max(mx, my), max(mz, mw));
+                if constexpr (M != kPair) {
+                    value1 = min(min(value1, mx - 1u), my - 1u);
+                    value1 = min(min(value1, mz - 1u), mw - 1u);
+                }
             }
-            m = max(m, ror8(m));
-            m = max(m, (uint32_t)__shfl_xor(m, 16, KQ_WAVE));
-            m = max(m, (uint32_t)__shfl_xor(m, 32, KQ_WAVE));
+            if constexpr (least_group<FMT, M>() != 0.0f) {
+                /* a group: half a step; Q6_K, four elements of two k-groups */
+#pragma unroll
+                for (uint32_t k = 0; k < NV; ++k) {
+                    if constexpr (M == kQuad) {
+                        if (k & 1u) group1 = min(group1, max(gm[k - 1u], gm[k]) - 1u);
+                    } else {
+                        gm[k] = FMT == KQ_LAUNCH_Q6_K ? max16(gm[k]) : max(gm[k], ror8(gm[k]));
+                        group1 = min(group1, gm[k] - 1u);
+                    }
+                }
+            }
+#pragma unroll
+            for (uint32_t k = 0; k < NV; ++k) m = max(m, gm[k]);
+            m = max(m, M == kQuad ? quad1(m) : ror8(m));
+            if constexpr (M == kQuad) m = max(m, quad2(m));
+            m = max_groups(m);
             /* largest magnitude into [2^14, 2^15); a column with a
              * non-finite value contributes zeros (the call fails) */
             const bool nf = m >= 0x7f800000u;
             bad |= nf;
             const int sig = !nf && m != 0u ? 15 - __builtin_amdgcn_frexp_expf(__uint_as_float(m)) : 0;
-            if (g == 0u && i < kCols) sigs[(c * nw + w) * kCols + i] = sig;
-            float run[2] = {0.0f, 0.0f}, blo[4], bhi[4];
+            auto below = [&](float scaled) { return max(mag(ldexpf(scaled, -sig)), 1u) - 1u; };
+            deep |= !nf && (value1 < below(least_value()) || group1 < below(least_group<FMT, M>()));
+            if (g == 0u && (M == kQuad ? q == 0u : i < KC)) sigs[(c * nw + w) * KC + col] = sig;
+            float run[2] = {0.0f, 0.0f}, by_step[NV]; /* sums over this lane's values */
+            uint32_t own[4][4]; /* kQuad: a step's [part][dword] */
 #pragma unroll
-            for (uint32_t s = 0; s < 8u; ++s) {
-                if (nf) v[s] = float4{0.f, 0.f, 0.f, 0.f};
-                const float xs[4] = {ldexpf(v[s].x, sig), ldexpf(v[s].y, sig), ldexpf(v[s].z, sig),
-                                     ldexpf(v[s].w, sig)};
-                h4 hv, lv;
+            for (uint32_t k = 0; k < NV; ++k) {
+                if (nf) v[k] = float4{0.f, 0.f, 0.f, 0.f};
+                const float xs[4] = {ldexpf(v[k].x, sig), ldexpf(v[k].y, sig), ldexpf(v[k].z, sig),
+                                     ldexpf(v[k].w, sig)};
+                h2 pa[NP], pb[NP];
+                split<NP>(xs[0], xs[1], pa);
+                split<NP>(xs[2], xs[3], pb);
+                auto lo_of = [&](int n) { return __builtin_bit_cast(uint32_t, pa[n]); };
+                auto hi_of = [&](int n) { return __builtin_bit_cast(uint32_t, pb[n]); };
+                const float s4 = (xs[0] + xs[1]) + (xs[2] + xs[3]);
+                if constexpr (M == kQuad) {
+                    run[k >> 1] += s4;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    hv[e] = (_Float16)xs[e];
-                    lv[e] = (_Float16)(xs[e] - (float)hv[e]);
-                }
-                const kq_u32x2 hb = __builtin_bit_cast(kq_u32x2, hv), lb = __builtin_bit_cast(kq_u32x2, lv);
-                const uint32_t r0 = ror8(half ? hb.x : lb.x), r1 = ror8(half ? hb.y : lb.y);
-                A[c][s] = pinned(half ? r0 : hb.x, half ? r1 : hb.y, half ? lb.x : r0, half ? lb.y : r1);
-                if constexpr (has_min(FMT)) {
-                    const float p = (xs[0] + xs[1]) + (xs[2] + xs[3]);
-                    run[s >> 2] += p;
-                    (s < 4u ? blo : bhi)[s & 3u] = p;
+                    for (int n = 0; n < NP; ++n) {
+                        own[n][2u * (k & 1u)] = lo_of(n);
+                        own[n][2u * (k & 1u) + 1u] = hi_of(n);
+                    }
+                    if ((k & 1u) == 0u) continue;
+                    /* four lanes' parts of a step each to each lane's part of four steps */
+                    uint32_t f[4][4]; /* [lane][dword] */
+#pragma unroll
+                    for (int d = 0; d < 4; ++d) {
+                        uint32_t l[2][2];
+#pragma unroll
+                        for (uint32_t n = 0; n < 2u; ++n) {
+                            const uint32_t even = own[2u * n][d], odd = own[2u * n + 1u][d];
+                            const uint32_t r = quad1(q0 ? even : odd);
+                            l[n][0] = q0 ? r : even;
+                            l[n][1] = q0 ? odd : r;
+                        }
+#pragma unroll
+                        for (uint32_t b = 0; b < 2u; ++b) {
+                            const uint32_t r = quad2(q1 ? l[0][b] : l[1][b]);
+                            f[b][d] = q1 ? r : l[0][b];
+                            f[2u + b][d] = q1 ? l[1][b] : r;
+                        }
+                    }
+#pragma unroll
+                    for (uint32_t b = 0; b < 4u; ++b)
+                        A[c][0][2u * b + (k >> 1)] = pinned(f[b][0], f[b][1], f[b][2], f[b][3]);
+                } else {
+                    /* operand o: part o on rows 0 .. 7, part G + o on 8 .. 15 */
+#pragma unroll
+                    for (uint32_t o = 0; o < G; ++o) {
+                        const uint32_t mx = lo_of(o), my = hi_of(o), tx = lo_of(G + o), ty = hi_of(G + o);
+                        const uint32_t r0 = ror8(q0 ? mx : tx), r1 = ror8(q0 ? my : ty);
+                        A[c][o][k] = pinned(q0 ? r0 : mx, q0 ? r1 : my, q0 ? tx : r0, q0 ? ty : r1);
+                    }
+                    if constexpr (has_min(FMT)) {
+                        run[k >> 2] += s4;
+                        by_step[k] = s4;
+                    }
                 }
             }
             float sm[4] = {0.0f, 0.0f, 0.0f, 0.0f};
             if constexpr (is_k(FMT)) {
-                /* lane (i, g) holds sub-blocks 2g and 2g + 1 */
-                run[0] += ror8(run[0]);
-                run[1] += ror8(run[1]);
+                /* each lane of k-group g: sub-blocks 2g and 2g + 1 */
+                if constexpr (M == kQuad) {
+                    float half = run[0] + run[1];
+                    half += quad1(half);
+                    const float other = quad2(half);
+                    run[0] = q1 ? other : half;
+                    run[1] = q1 ? half : other;
+                } else {
+                    run[0] += ror8(run[0]);
+                    run[1] += ror8(run[1]);
+                }
                 const int src = (int)(i + 32u * (g & 1u));
                 sm[0] = __shfl(run[0], src, KQ_WAVE);
                 sm[1] = __shfl(run[1], src, KQ_WAVE);
                 sm[2] = __shfl(run[0], src + 16, KQ_WAVE);
                 sm[3] = __shfl(run[1], src + 16, KQ_WAVE);
             } else if constexpr (FMT == KQ_LAUNCH_Q5_1) {
+                auto over_groups = [](float b) {
+                    b += __shfl_xor(b, 16, KQ_WAVE);
+                    return b + __shfl_xor(b, 32, KQ_WAVE);
+                };
+                if constexpr (M == kQuad) {
+                    /* blocks 2 q and 2 q + 1, from lane q of the four */
+                    const uint32_t b0 = __float_as_uint(over_groups(run[0]));
+                    const uint32_t b1 = __float_as_uint(over_groups(run[1]));
+                    const bool up = (g & 1u) != 0u;
+                    sm[0] = __uint_as_float(up ? dpp<0xaa>(b0) : dpp<0x00>(b0));
+                    sm[1] = __uint_as_float(up ? dpp<0xaa>(b1) : dpp<0x00>(b1));
+                    sm[2] = __uint_as_float(up ? dpp<0xff>(b0) : dpp<0x55>(b0));
+                    sm[3] = __uint_as_float(up ? dpp<0xff>(b1) : dpp<0x55>(b1));
+                } else {
 #pragma unroll
-                for (uint32_t e = 0; e < 4u; ++e) {
-                    blo[e] += ror8(blo[e]);
-                    bhi[e] += ror8(bhi[e]);
-                    blo[e] += __shfl_xor(blo[e], 16, KQ_WAVE);
-                    bhi[e] += __shfl_xor(bhi[e], 16, KQ_WAVE);
-                    blo[e] += __shfl_xor(blo[e], 32, KQ_WAVE);
-                    bhi[e] += __shfl_xor(bhi[e], 32, KQ_WAVE);
-                    sm[e] = (g & 1u) != 0u ? bhi[e] : blo[e];
+                    for (uint32_t e = 0; e < 4u; ++e) {
+                        const float b0 = over_groups(by_step[e] + ror8(by_step[e]));
+                        const float b1 = over_groups(by_step[e + 4u] + ror8(by_step[e + 4u]));
+                        sm[e] = (g & 1u) != 0u ? b1 : b0;
+                    }
                 }
             }
-            if constexpr (has_min(FMT)) {
 #pragma unroll
-                for (uint32_t e = 0; e < 4u; ++e) {
-                    const float f = FMT == KQ_LAUNCH_Q5_1 ? sm[e] * (g < 2u ? 0x1p-9f : 0x1p-5f)
-                                    : g < 2u              ? sm[e] * 0x1p-5f : 0.0f;
-                    const _Float16 hv = (_Float16)f;
-                    sums[c][e] = half ? (_Float16)(f - (float)hv) : hv;
+            for (uint32_t o = 0; o < G; ++o) sums[c][o] = h4{};
+            if constexpr (has_min(FMT)) {
+                const float scale = FMT == KQ_LAUNCH_Q5_1 ? (g < 2u ? 0x1p-9f : 0x1p-5f)
+                                    : M == kPair || g < 2u ? 0x1p-5f : 0.0f;
+#pragma unroll
+                for (uint32_t e = 0; e < 4u; e += 2u) {
+                    h2 p[4];
+                    split<4>(sm[e] * scale, sm[e + 1u] * scale, p);
+#pragma unroll
+                    for (uint32_t o = 0; o < G; ++o) {
+                        const h2 p0 = p[0], p1 = p[1], p2 = p[2], p3 = p[3];
+                        h2 r;
+                        if constexpr (M == kQuad) {
+                            const h2 even = q1 ? p2 : p0, odd = q1 ? p3 : p1;
+                            r = q0 ? odd : even;
+                        } else if constexpr (M == kEight) {
+                            const h2 big = o == 0u ? p0 : p1, tiny = o == 0u ? p2 : p3;
+                            r = q0 ? tiny : big;
+                        } else {
+                            const h2 a2 = p2 * splat(0x1p-13f), a3 = p3 * splat(0x1p-13f);
+                            r = q0 ? (g < 2u ? p1 : a3) : (g < 2u ? p0 : a2);
+                        }
+                        sums[c][o][e] = r.x;
+                        sums[c][o][e + 1u] = r.y;
+                    }
                 }
-            } else {
-                sums[c] = h4{};
             }
             /* one unit's values, and the next one's on their way */
             __builtin_amdgcn_sched_barrier(0);
         }
     }
+    {
+        const uint64_t any = __ballot(deep);
+        if (lane == 0u) deeps[w] = (uint32_t)(any != 0ull);
+    }
     for (uint32_t t = 1; t < a.pd && t < n_ent; ++t) issue();
 
-    const uint32_t t = threadIdx.x; /* < 128: output column t / 16, row t % 16 */
+    const uint32_t t = threadIdx.x; /* < 16 KC: output column t / 16, row t % 16 */
     float best_v = -__builtin_inff();
     uint32_t best_i = 0xffffffffu;
     bool malformed = false, nonfinite = false;
     f4 acc = {0.f, 0.f, 0.f, 0.f};
     uint32_t slot = 0u, ent = 0u;
-    auto finish = [&](uint32_t tile) {
-        if (t < 128u) {
-            const float *pp = part + (tile & 1u) * nw * 128u + t;
+    auto finish = [&](uint32_t tile, uint32_t parts) {
+        if (t < KC * 16u) {
+            const float *pp = part + (tile & 1u) * nw * (KC * 16u) + t;
             float s = 0.0f;
-            for (uint32_t q = 0; q < nw; ++q) s += pp[q * 128u];
+            for (uint32_t q = 0; q < parts; ++q) s += pp[q * (KC * 16u)];
             const uint32_t row = tile * kT + (t & 15u), col = t >> 4;
             if (row < a.rows && col < a.batch) {
                 nonfinite |= !kq_isfinite(s);
@@ -460,63 +736,120 @@ __global__ __launch_bounds__((max_threads<NC>())) void mv_tiles(MvtArgs a) {
             }
         }
     };
-    for (uint32_t tile = lo; tile < hi; ++tile) {
-#pragma unroll
-        for (uint32_t c = 0; c < NC; ++c, ++ent) {
-            /* this chunk's loads have landed (those of the chunks requested
-             * after it may be in flight): in this wave, then in all */
-            const uint32_t after = n_ent - 1u - ent;
-            wait_after<IPW, kMaxPd - 1u>(after < a.pd - 1u ? after : a.pd - 1u);
-            kq_lds_barrier();
-            if (ent + a.pd < n_ent) issue();
-            if (c == 0u && tile > lo) finish(tile - 1u);
-            const uint32_t u = c * nw + w;
-            if (u < nu) { /* wave-uniform */
-                const uint32_t left = a.cols - kUnit * u;
-                const uint32_t live = PART && left < kUnit ? left / 32u : 8u;
-                const uint32_t at = w * UB + (FMT == KQ_LAUNCH_Q6_K ? (j * a.row_bytes) & 2u : 0u);
-                const uint32_t off = at & 2u;
-                const uint8_t *p = ring + slot * a.slot + j * a.pitch * 16u + at;
-                const f4 v = unit_product<FMT>(p, off, g, live, tile * kT + j < a.rows, A[c],
-                                               sums[c], malformed);
-                const int4 sg = *(const int4 *)(sigs + u * kCols + 4u * (g & 1u));
-                acc[0] += ldexpf(v[0], -sg.x);
-                acc[1] += ldexpf(v[1], -sg.y);
-                acc[2] += ldexpf(v[2], -sg.z);
-                acc[3] += ldexpf(v[3], -sg.w);
-            }
-            slot = slot == a.pd ? 0u : slot + 1u;
-        }
-        /* columns 4g .. 4g + 3 of row j: the hi and the lo product rows */
-        float *pw = part + ((tile & 1u) * nw + w) * 128u;
-#pragma unroll
-        for (uint32_t k = 0; k < 4u; ++k) {
-            const float o = acc[k] + __shfl_xor(acc[k], 32, KQ_WAVE);
-            if (g < 2u) pw[(4u * g + k) * 16u + j] = o;
-            acc[k] = 0.0f;
-        }
-    }
+    /* the first chunk's loads have landed (those of the chunks requested after
+     * it may be in flight): in this wave, then in all */
+    wait_after<IPW, kMaxPd - 1u>(n_ent - 1u < a.pd - 1u ? n_ent - 1u : a.pd - 1u);
     kq_lds_barrier();
-    if (hi > lo) finish(hi - 1u);
+    if (__builtin_expect(__ballot(lane < nw && deeps[lane < nw ? lane : 0u] != 0u) != 0ull, 0)) {
+        /* some value lies too far below its unit's largest for the operand:
+         * the rows in binary32, a wave a row (every workgroup sees the same
+         * values and comes here) */
+        const MvtArgs *b = late_args();
+        for (uint32_t tile = lo; tile < hi; ++tile) {
+            for (uint32_t r = w; r < kT; r += nw) {
+                const uint32_t row = tile * kT + r;
+                if (row >= b->rows) break;
+                const uint8_t *rp = b->W + (size_t)row * b->row_bytes;
+                float sum[KC];
+#pragma unroll
+                for (uint32_t k = 0; k < KC; ++k) sum[k] = 0.0f;
+                for (uint32_t c = 4u * lane; c < b->cols; c += 4u * KQ_WAVE) {
+                    float wt[4];
+                    weights_at<FMT>(rp, c, wt, malformed);
+#pragma unroll
+                    for (uint32_t k = 0; k < KC; ++k) {
+                        if (k >= b->batch) break;
+                        const float4 xv = *(const float4 *)(b->x + (size_t)k * b->cols + c);
+                        sum[k] = fmaf(wt[0], xv.x, sum[k]);
+                        sum[k] = fmaf(wt[1], xv.y, sum[k]);
+                        sum[k] = fmaf(wt[2], xv.z, sum[k]);
+                        sum[k] = fmaf(wt[3], xv.w, sum[k]);
+                        if (k & 1u) __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+#pragma unroll
+                for (uint32_t k = 0; k < KC; ++k) {
+                    float v = sum[k];
+                    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, KQ_WAVE);
+                    if (lane == 0u) part[(tile & 1u) * nw * (KC * 16u) + k * 16u + r] = v;
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            /* the other parity was read before the previous barrier */
+            kq_lds_barrier();
+            finish(tile, 1u);
+        }
+    } else {
+        for (uint32_t tile = lo; tile < hi; ++tile) {
+#pragma unroll
+            for (uint32_t c = 0; c < NC; ++c, ++ent) {
+                if (ent != 0u) {
+                    const uint32_t after = n_ent - 1u - ent;
+                    wait_after<IPW, kMaxPd - 1u>(after < a.pd - 1u ? after : a.pd - 1u);
+                    kq_lds_barrier();
+                }
+                if (ent + a.pd < n_ent) issue();
+                if (c == 0u && tile > lo) finish(tile - 1u, nw);
+                const uint32_t u = c * nw + w;
+                if (u < nu) { /* wave-uniform */
+                    const uint32_t left = a.cols - kUnit * u;
+                    const uint32_t live = PART && left < kUnit ? left / 32u : 8u;
+                    const uint32_t at = w * UB + (FMT == KQ_LAUNCH_Q6_K ? (j * a.row_bytes) & 2u : 0u);
+                    const uint32_t off = at & 2u;
+                    const uint8_t *p = ring + slot * a.slot + j * a.pitch * 16u + at;
+                    const f4 v = unit_product<FMT, M>(p, off, g, live, tile * kT + j < a.rows, A[c],
+                                                      sums[c], malformed);
+                    if constexpr (M == kQuad) {
+                        /* the four parts of column g */
+                        acc[0] += ldexpf(fmaf(0x1p-24f, v[2] + v[3], v[0] + v[1]), -sigs[u * KC + g]);
+                    } else {
+                        const int4 sg = *(const int4 *)(sigs + u * KC + 4u * (g & 1u));
+                        const int at = M == kPair || g < 2u ? 0 : kTiny;
+                        acc[0] += ldexpf(v[0], -sg.x - at);
+                        acc[1] += ldexpf(v[1], -sg.y - at);
+                        acc[2] += ldexpf(v[2], -sg.z - at);
+                        acc[3] += ldexpf(v[3], -sg.w - at);
+                    }
+                }
+                slot = slot == a.pd ? 0u : slot + 1u;
+            }
+            float *pw = part + ((tile & 1u) * nw + w) * (KC * 16u);
+            if constexpr (M == kQuad) {
+                pw[g * 16u + j] = acc[0];
+                acc[0] = 0.0f;
+            } else {
+                /* columns 4g .. 4g + 3 of row j: operand rows 0 .. 7 and 8 .. 15 */
+#pragma unroll
+                for (uint32_t k = 0; k < 4u; ++k) {
+                    const float o = acc[k] + __shfl_xor(acc[k], 32, KQ_WAVE);
+                    if (g < 2u) pw[(4u * g + k) * 16u + j] = o;
+                    acc[k] = 0.0f;
+                }
+            }
+        }
+        kq_lds_barrier();
+        if (hi > lo) finish(hi - 1u, nw);
+    }
     /* no LDS-DMA load may outlive the workgroup */
     wait_vm<0>();
-    if (bad) kq_flag(a.status, KQ_DEV_INPUT);
-    if (malformed) kq_flag(a.status, KQ_DEV_MALFORMED);
-    if (nonfinite) kq_flag(a.status, KQ_DEV_NUMERIC);
-    if (a.part_v != nullptr && t < 128u) {
+    const MvtArgs *b = late_args();
+    if (bad) kq_flag(b->status, KQ_DEV_INPUT);
+    if (malformed) kq_flag(b->status, KQ_DEV_MALFORMED);
+    if (nonfinite) kq_flag(b->status, KQ_DEV_NUMERIC);
+    if (b->part_v != nullptr && t < KC * 16u) {
 #pragma unroll
         for (int o = 8; o > 0; o >>= 1) {
             const float ov = __shfl_xor(best_v, o, KQ_WAVE);
             const uint32_t oi = __shfl_xor(best_i, o, KQ_WAVE);
             argmax_merge(best_v, best_i, ov, oi);
         }
-        if ((t & 15u) == 0u && (t >> 4) < a.batch) {
-            const size_t row = (size_t)(t >> 4) * a.part_stride;
-            a.part_v[row + blockIdx.x] = best_v;
-            a.part_i[row + blockIdx.x] = best_i;
-            for (uint32_t sl = blockIdx.x + gridDim.x; sl < a.part_stride; sl += gridDim.x) {
-                a.part_v[row + sl] = -__builtin_inff();
-                a.part_i[row + sl] = 0xffffffffu;
+        if ((t & 15u) == 0u && (t >> 4) < b->batch) {
+            const size_t row = (size_t)(t >> 4) * b->part_stride;
+            b->part_v[row + blockIdx.x] = best_v;
+            b->part_i[row + blockIdx.x] = best_i;
+            for (uint32_t sl = blockIdx.x + gridDim.x; sl < b->part_stride; sl += gridDim.x) {
+                b->part_v[row + sl] = -__builtin_inff();
+                b->part_i[row + sl] = 0xffffffffu;
             }
         }
     }
@@ -544,22 +877,24 @@ uint32_t device_cus() {
 }
 
 constexpr uint32_t kLdsCu = 160u * 1024u;
+constexpr uint32_t kMaxEight = 2u; /* units per wave with two operands each */
 
-/* The waves of a workgroup: the count (at most 10, 8 with three or more
- * units each) that leaves the fewest idle in a row's last chunk, the larger
- * of equals: one unit a wave where a row has at most 10 (10240 x 2560 Q8_0
- * at 8 columns: 12.9 us with 10 waves of one unit, 22 with 5 of two). Two
- * workgroups per CU where their registers and two chunk slots each fit
- * (151936 x 2048 Q6_K at 4 columns: 61.8 us, 72.4 with one), and as many
- * slots as fit then. */
-bool make_plan(uint32_t type, uint32_t rows, uint32_t cols, Plan &p) {
+/* The waves of a workgroup: the count (at most 10, 8 with more than two
+ * operands of 32 registers each) that leaves the fewest idle in a row's last
+ * chunk, the larger of equals: one unit a wave where a row has at most 10
+ * (10240 x 2560 Q8_0 at 8 columns: 12.9 us with 10 waves of one unit, 22 with
+ * 5 of two). Two workgroups per CU where their registers and two chunk slots
+ * each fit (151936 x 2048 Q6_K at 4 columns: 61.8 us, 72.4 with one), and as
+ * many slots as fit then. */
+bool make_plan(uint32_t type, uint32_t rows, uint32_t cols, uint32_t batch, Plan &p) {
     const uint32_t ub = unit_bytes(type);
     if (ub == 0u || cols == 0u || cols % block_cols(type) != 0u) return false;
-    const uint32_t nu = (cols + kUnit - 1u) / kUnit;
+    const uint32_t nu = (cols + kUnit - 1u) / kUnit, ops = batch > 4u && is_binary32(type) ? 2u : 1u;
+    const uint32_t kc = kCols;
     uint32_t best = 0u, best_idle = 0xffffffffu;
     for (uint32_t nw = 10u; nw >= 2u; --nw) {
         const uint32_t nc = (nu + nw - 1u) / nw;
-        if (nc > 5u || (nc >= kWideNc && nw > 8u) || (nc > 3u && cols % kUnit != 0u)) continue;
+        if (nc * ops > (ops == 2u ? 2u * kMaxEight : 5u) || (nc * ops > kNarrow && nw > 8u) || (nc > 3u && cols % kUnit != 0u)) continue;
         if (nc > 1u && (nw * ub) % 4u != 0u) continue; /* chunks start on dwords */
         const uint32_t idle = nc * nw - nu;
         if (idle < best_idle) {
@@ -573,8 +908,9 @@ bool make_plan(uint32_t type, uint32_t rows, uint32_t cols, Plan &p) {
     const uint32_t units = (best * ub + 2u + 15u) / 16u;
     p.pitch = units | 1u;
     p.slot = (kT * p.pitch + 63u) / 64u * 1024u;
-    const uint32_t fixed = 1024u + 2u * best * 512u + p.nc * best * kCols * 4u;
-    const uint32_t waves = p.nc == 1u ? 20u : p.nc < kWideNc ? 12u : 8u; /* per CU, by registers */
+    const uint32_t fixed = 1024u + 2u * best * kc * 64u + p.nc * best * kc * 4u + best * 4u;
+    /* per CU, by registers */
+    const uint32_t waves = p.nc * ops == 1u ? 20u : p.nc * ops == 2u ? 12u : 8u;
     const uint32_t wgs = 2u * best <= waves && 2u * (2u * p.slot + fixed) <= kLdsCu ? 2u : 1u;
     uint32_t slots = (kLdsCu / wgs - fixed) / p.slot;
     if (slots > kMaxPd + 1u) slots = kMaxPd + 1u;
@@ -592,7 +928,19 @@ uint32_t row_bytes_of(uint32_t type, uint32_t cols) {
 
 template <uint32_t FMT, uint32_t NC, bool PART>
 hipError_t launch_nc(const Plan &p, const MvtArgs &a, hipStream_t s) {
-    hipLaunchKernelGGL((mv_tiles<FMT, NC, PART>), dim3(p.blocks), dim3(p.nw * 64u), p.lds, s, a);
+    constexpr Rows kMany = is_binary32(FMT) ? kEight : kPair;
+    /* five units of four parts take longer to build (4000 x 10240 Q4_K, 2
+     * columns: 18.7 us, kPair 16.4) */
+    constexpr Rows kFew = NC >= 5u && kMany == kPair ? kPair : kQuad;
+    const dim3 grid(p.blocks), block(p.nw * 64u);
+    if (a.batch <= 4u) {
+        hipLaunchKernelGGL((mv_tiles<FMT, NC, PART, kFew>), grid, block, p.lds, s, a);
+    } else {
+        if constexpr (kMany == kEight && NC > kMaxEight)
+            return hipErrorInvalidValue;
+        else
+            hipLaunchKernelGGL((mv_tiles<FMT, NC, PART, kMany>), grid, block, p.lds, s, a);
+    }
     return hipGetLastError();
 }
 
@@ -623,16 +971,17 @@ hipError_t launch_fmt(const Plan &p, const MvtArgs &a, hipStream_t s) {
 extern "C" int kq_launch_mv_tiles_supported(uint32_t type, uint32_t rows, uint32_t cols,
                                             uint32_t batch) {
     Plan p;
-    if (batch < 1u || batch > kCols || !make_plan(type, rows, cols, p)) return 0;
+    if (batch < 1u || batch > kCols || !make_plan(type, rows, cols, batch, p)) return 0;
     /* rows of 34- and 18-byte blocks start on whole dwords (Q6_K ones may
      * not), and the last tile's offsets past the matrix stay within 32 bits */
     const uint64_t rb = row_bytes_of(type, cols);
     return (rb % 4u == 0u || type == KQ_LAUNCH_Q6_K) && rows * rb <= 0xffe00000ull;
 }
 
-extern "C" uint32_t kq_launch_mv_tiles_parts(uint32_t type, uint32_t rows, uint32_t cols) {
+extern "C" uint32_t kq_launch_mv_tiles_parts(uint32_t type, uint32_t rows, uint32_t cols,
+                                             uint32_t batch) {
     Plan p;
-    return make_plan(type, rows, cols, p) ? p.blocks : 0u;
+    return make_plan(type, rows, cols, batch, p) ? p.blocks : 0u;
 }
 
 extern "C" hipError_t kq_launch_mv_tiles(uint32_t type, const void *W, uint32_t rows,
@@ -640,7 +989,7 @@ extern "C" hipError_t kq_launch_mv_tiles(uint32_t type, const void *W, uint32_t 
                                          uint32_t *status, float *part_v, uint32_t *part_i,
                                          uint32_t part_stride, hipStream_t stream) {
     Plan p;
-    if (!kq_launch_mv_tiles_supported(type, rows, cols, batch) || !make_plan(type, rows, cols, p))
+    if (!kq_launch_mv_tiles_supported(type, rows, cols, batch) || !make_plan(type, rows, cols, batch, p))
         return hipErrorInvalidValue;
     MvtArgs a;
     a.W = (const uint8_t *)W;
@@ -658,6 +1007,9 @@ extern "C" hipError_t kq_launch_mv_tiles(uint32_t type, const void *W, uint32_t 
     a.pitch = p.pitch;
     a.slot = p.slot;
     a.pd = p.pd;
+    const uint32_t tiles = (rows + kT - 1u) / kT;
+    a.tiles = tiles / p.blocks;
+    a.more = tiles % p.blocks;
     switch (type) {
     case KQ_LAUNCH_Q4_K: return launch_fmt<KQ_LAUNCH_Q4_K>(p, a, stream);
     case KQ_LAUNCH_Q5_K: return launch_fmt<KQ_LAUNCH_Q5_K>(p, a, stream);

@@ -496,6 +496,95 @@ def test_matvec_tiles(ctx, fmt, rows, cols, batch):
                                    lambda i: ex.scale(i) * inv[np.asarray(i) // rows]))
 
 
+def _zero_weights(fmt, w, rows, cols, column):
+    """Rows of w with the weights of column 3 zero, or of columns 0 .. 31."""
+    b = w.copy().reshape(rows, cols // kq_hip.GEOMETRY[FMTS[fmt]][0], -1)
+    first = b[:, 0]
+    if fmt in ("Q4_K", "Q5_K"):
+        first[:, 8] &= 0xC0  # min of sub-block 0
+        if column:
+            first[:, (48 if fmt == "Q5_K" else 16) + 3] &= 0xF0
+            if fmt == "Q5_K":
+                first[:, 16 + 3] &= 0xFE
+        else:
+            first[:, 4] &= 0xC0
+    elif fmt == "Q6_K":
+        if column:
+            first[:, 3] &= 0xF0  # code 32
+            first[:, 128 + 3] = (first[:, 128 + 3] & 0xFC) | 2
+        else:
+            first[:, 192:194] = 0
+    elif fmt == "Q5_1":
+        first[:, 2:4] = 0
+        if column:
+            first[:, 4] &= 0xF7
+            first[:, 8 + 3] &= 0xF0
+        else:
+            first[:, 0:2] = 0
+    elif column:
+        first[:, 2 + 3] = 0  # Q8_0
+    else:
+        first[:, 0:2] = 0
+    return b.reshape(-1)
+
+
+@pytest.mark.parametrize("k", [18, 24, 33, 45, 100])
+@pytest.mark.parametrize("fmt,rows,cols,batch,column", [
+    (f, r, c, b, col) for f in ALL_FMTS for r, c, b in ((2049, 512, 3), (2050, 2048, 4), (33, 768, 6),
+                                                       (2048, 2816, 4), (40, 4096, 8), (17, 6144, 5))
+    for col in (False, True)
+    # IQ4_NL has no zero code; five and more columns of these have a scale per
+    # 16 columns at most on either path
+    if not (col and (f == "IQ4_NL" or (b > 4 and f in ("Q4_K", "Q6_K", "Q8_0"))))
+] + [("Q8_0", 31, 320, 1, True), ("Q5_1", 30, 2112, 1, True)])
+def test_matvec_values_far_apart(ctx, fmt, rows, cols, batch, column, k):
+    # values 2^k apart in one 256-column unit, the large one against weights
+    # that are zero: the small ones count in full, as in binary32. (The bar is
+    # 8 u S, u = 2^-24, S the sum of the other products' magnitudes; up to 256
+    # of them, in a tree and a few serial sums.)
+    t = FMTS[fmt]
+    key = S.stream_key(S.W_MATVEC_Q6K, 97, rows * 64 + batch, cols // 32)
+    w = _zero_weights(fmt, S.quant_matrix(fmt, key, rows, cols), rows, cols, column)
+    x = np.zeros((batch, cols), np.float32)
+    x[:, :256] = S.normal_f32(key ^ 0x55, batch * 256).reshape(batch, 256)
+    x[:, 3] = 2.0 ** k
+    x[0] *= np.float32(2.0 ** -20)
+    dw, dx, dy = ctx.upload(w), ctx.upload(x), ctx.alloc(rows * batch * 4)
+    ctx.matvec(t, dw, rows, cols, dx, batch, dy)
+    got = ctx.download(dy, np.float32, rows * batch).astype(np.float64)
+    for b in (dw, dx, dy):
+        b.close()
+    ex = exact.matvec(t, w, rows, cols, x)
+    every = np.arange(rows * batch)
+    assert (np.abs(got - ex(every)) <= 2.0 ** -21 * ex.scale(every)).all()
+
+
+@pytest.mark.parametrize("fmt", ALL_FMTS)
+def test_lm_head_values_far_apart(ctx, fmt):
+    # the same with the argmax partials, and the failures of such a call
+    rows, cols, batch, t = 6000, 2560, 6, FMTS[fmt]
+    w = S.quant_matrix(fmt, S.stream_key(S.W_MATVEC_Q6K, 98, t), rows, cols)
+    x = S.normal_f32(S.stream_key(S.W_MATVEC_Q6K, 99, t), batch * cols).reshape(batch, cols)
+    x[2, 256:512] *= np.float32(1e-25)
+    x[2, 300] = 1.0
+    x_bad, w_bad = x.copy(), w.copy().reshape(-1, kq_hip.GEOMETRY[t][1])
+    x_bad[1, 7] = np.inf
+    w_bad[-1, {"Q6_K": slice(208, 210)}.get(fmt, slice(0, 2))] = [0x00, 0x7C]
+    dw, dx, dy, di = ctx.upload(w), ctx.upload(x), ctx.alloc(rows * batch * 4), ctx.alloc(batch * 4)
+    dxb, dwb = ctx.upload(x_bad), ctx.upload(w_bad.reshape(-1))
+    for a, b, name in ((dw, dxb, "NUMERIC_DOMAIN"), (dwb, dx, "MALFORMED_QUANTIZED_DATA")):
+        with pytest.raises(kq_hip.KqError) as e:
+            ctx.lm_head(t, a, rows, cols, b, batch, dy, di)
+        assert e.value.name == name
+    ctx.lm_head(t, dw, rows, cols, dx, batch, dy, di)
+    got = ctx.download(dy, np.float32, rows * batch).reshape(batch, rows)
+    assert_close(got, kq_oracle.matvec(t, w, rows, cols, x, threads=oracle_threads()),
+                 exact=exact.matvec(t, w, rows, cols, x))
+    assert np.array_equal(ctx.download(di, np.uint32, batch), got.argmax(1))
+    for b in (dw, dx, dy, di, dxb, dwb):
+        b.close()
+
+
 @pytest.mark.parametrize("fmt,cols,field", [("Q4_K", 2560, 2), ("Q5_K", 512, 0), ("Q6_K", 768, 208),
                                             ("Q8_0", 640, 0), ("Q5_1", 320, 2), ("IQ4_NL", 2112, 0)])
 def test_matvec_tiles_fails_closed(ctx, fmt, cols, field):
