@@ -736,34 +736,53 @@ static uint32_t row_launches(uint32_t type, uint32_t cols, uint32_t batch) {
 }
 
 /* The row engine or the matrix-core tiles (kq_mvtiles.hip). The tiles take
- * about the same time for 1 to 8 columns; the row engine's grows with them.
- * Measured over 256 .. 40,000 rows of 512 .. 10,240 columns in every format
- * (row engine against tiles, us):
+ * about the same time for 1 to 4 and for 5 to 8 columns; the row engine's
+ * grows with them and in steps of 2,048 rows. Measured over 256 .. 40,000 rows
+ * of 512 .. 10,240 columns in every format (row engine / tiles, us):
  *   - five columns or more are two launches of the row engine: the tiles
- *     win everywhere (1000 x 2048 Q5_1, 5 columns: 9.2 / 6.4; 10000 x 2560
- *     Q8_0, 8 columns: 74.8 / 11.7);
+ *     win (1000 x 2048 Q8_0, 5 columns: 8.4 / 5.9; 10240 x 2560 Q8_0, 8
+ *     columns: 73.8 / 11.5; level in Q5_1 at 1000 x 2048: 8.9 / 9.0);
  *   - so they do where fewer columns take several launches, rows of other
- *     widths than the engine's (4000 x 640 Q8_0, 1 column: 7.6 / 4.8;
- *     10000 x 10240 Q4_K, 2 columns: 43.7 / 24.4), up to 20,000 rows at one
+ *     widths than the engine's (10000 x 640 Q8_0, 1 column: 8.8 / 5.3;
+ *     10000 x 10240 Q4_K, 2 columns: 43.0 / 26.3), up to 20,000 rows at one
  *     column (40000 x 640 Q5_1: 11.8 / 15.2);
- *   - in one launch, 3 and 4 columns from about 2,048 rows (4000 x 2048
- *     Q8_0, 4 columns: 7.6 / 5.8; 300 rows: 4.8 / 5.6), Q6_K 2 columns from
- *     about 4,096 (4000 x 2560: 8.4 / 6.8; 1000 rows: 5.4 / 6.6) up to 4,096
- *     columns (4000 x 6144: 12.1 / 14.4); the other formats at 2 columns and
- *     all at one stay (40000 x 2048, 2 columns: Q8_0 16.1 / 18.6, Q4_K
- *     13.1 / 15.6).
- * The 151936 x 2048 Q6_K head at 2 .. 4 columns is the one place where an
- * earlier kernel, made for 4 columns of that width, was a little faster (whole
- * call 61.3, 60.9, 62.4 against 64.1, 62.2, 64.9; level at 70001 rows, 25.4 ..
- * 35.9 against 22.6 .. 23.0 at 40000): its step held two sub-blocks of 4
- * columns where a tile's holds one of 8. 5 columns took it 106, 8 112; a tile
- * pass takes 63 and 65. */
-static bool use_tiles(uint32_t type, uint32_t rows, uint32_t cols, uint32_t batch) {
-    if (!kq_launch_mv_tiles_supported(type, rows, cols, batch)) return false;
+ *   - in one launch, 3 and 4 columns above 2,048 rows (3000 x 2560 Q4_K, 3
+ *     columns: 8.6 / 6.4; 2048 rows: 5.6 / 6.3; 2048 x 4096: 5.7 / 7.8; level
+ *     at 1,024 columns up to 8,000 rows), of up to 1,024 from there (2048 x 512 Q4_K:
+ *     8.3 / 5.1);
+ *   - but where the engine's rows come in whole widths and there are many of
+ *     them, it stays for the 32-weight formats at 3 columns: 1,024 columns
+ *     above 30,000 rows (40000 Q8_0: 11.2 / 12.9, Q6_K: 14.2 / 12.0), in Q5_1,
+ *     whose tiles decode longest, at 4 columns too, and widths of a power of
+ *     two above 16,000 (20000 x 2048, 3 columns: 11.2 / 12.7; x 2560: 21.6 /
+ *     21.1). Q5_1 at 3 columns also stays from 4,097 rows, where the tiles
+ *     start another round, to 6,000 (4097 x 2560: 10.9 / 13.2; 3000: 9.5 / 7.8;
+ *     8000: 16.8 / 13.6);
+ *   - Q6_K at 2 columns above about 5,000 rows (6000 x 2560: 11.7 / 11.1; 4097:
+ *     9.4 / 10.8) up to 4,096 columns (4000 x 6144: 12.1 / 14.4), but not 1,024
+ *     columns above 30,000 (40000: 10.2 / 11.8); the other formats at 2 columns
+ *     and all at one stay (40000 x 2048, 2 columns: Q8_0 16.1 / 18.6, Q4_K
+ *     13.1 / 15.6). */
+static bool prefer_tiles(uint32_t type, uint32_t rows, uint32_t cols, uint32_t batch) {
     if (batch > 4u) return true;
     if (row_launches(type, cols, batch) > 1u) return batch > 1u || rows <= 20000u;
-    if (batch >= 3u) return rows >= 2048u;
-    return batch == 2u && type == KQ_LAUNCH_Q6_K && rows >= 4096u && cols <= 4096u;
+    const bool many_1024 = cols == 1024u && rows > 30000u;
+    if (batch <= 2u)
+        return batch == 2u && type == KQ_LAUNCH_Q6_K && cols <= 4096u && rows > 5000u && !many_1024;
+    if (type == KQ_LAUNCH_Q5_1) {
+        if (many_1024) return false;
+        if (batch == 3u && ((rows > 4096u && rows < 6000u && cols >= 2048u) ||
+                            (rows > 16000u && cols >= 2048u && (cols & (cols - 1u)) == 0u)))
+            return false;
+    }
+    if (many_1024 && batch == 3u && (type == KQ_LAUNCH_Q8_0 || type == KQ_LAUNCH_IQ4_NL)) return false;
+    return rows > 2048u || (rows == 2048u && cols <= 1024u);
+}
+
+/* (the tiles' plan last: it costs the host more than a small launch shows) */
+static bool use_tiles(uint32_t type, uint32_t rows, uint32_t cols, uint32_t batch) {
+    return prefer_tiles(type, rows, cols, batch) &&
+           kq_launch_mv_tiles_supported(type, rows, cols, batch);
 }
 
 extern "C" uint32_t kq_launch_matvec_columns(uint32_t type, uint32_t rows, uint32_t cols,
