@@ -285,30 +285,24 @@ __global__ __launch_bounds__(64) void router_chain(const float *__restrict__ wt,
  * leave two waves per SIMD, and ran 30% slower at 512 x 512). Rows past the
  * experts read as zeros and are not stored; the shared gate vector is not a
  * row here (its logit only feeds the sigmoid gate, compared by tolerance). */
-constexpr uint32_t kSxTW = 1;
 constexpr uint32_t kSxWaves = 8;
 constexpr uint32_t kSxCols = 64;
 
-__global__ __launch_bounds__(64 * kSxWaves) void router_chain_sx(
-    const float *__restrict__ router, const float *__restrict__ hidden_states, uint32_t tokens,
-    uint32_t experts, uint32_t hidden, float *__restrict__ logits, uint32_t *status) {
+/* the chains of experts e0 .. e0 + 63 for one token a wave: token t (wave
+ * uniform), stored where `store` */
+__device__ __forceinline__ void chain_sx(const float *__restrict__ router,
+                                         const float *__restrict__ hidden_states, uint32_t experts,
+                                         uint32_t hidden, uint32_t e0, uint32_t t, bool store,
+                                         float *__restrict__ logits, uint32_t *status) {
     constexpr uint32_t NQ = kSxCols / 4u;  /* float4 per row per chunk */
     constexpr uint32_t PITCH = 65u;        /* float4 per q line */
     constexpr uint32_t LOADS = 64u * NQ / (64u * kSxWaves); /* float4 per thread per chunk */
     __shared__ float4 tile[2][NQ * PITCH];
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const uint32_t e0 = blockIdx.y * 64u;
-    const uint32_t tb = (blockIdx.x * kSxWaves + wave) * kSxTW;
     /* loader: float4 q = tid % NQ of rows tid / NQ + (64 * kSxWaves / NQ) * k */
     const uint32_t lq = tid % NQ, lr = tid / NQ;
     constexpr uint32_t RSTEP = 64u * kSxWaves / NQ;
-    const float *xr[kSxTW];
-#pragma unroll
-    for (uint32_t b = 0; b < kSxTW; ++b) {
-        const uint32_t t = tb + b < tokens ? tb + b : tokens - 1u;
-        xr[b] = hidden_states + (size_t)__builtin_amdgcn_readfirstlane(t) * hidden;
-    }
+    const float *xr = hidden_states + (size_t)__builtin_amdgcn_readfirstlane(t) * hidden;
     float4 ld[LOADS];
     bool bad = false;
     auto gload = [&](uint32_t c) {
@@ -329,9 +323,7 @@ __global__ __launch_bounds__(64 * kSxWaves) void router_chain_sx(
             tile[buf][lq * PITCH + lr + RSTEP * k] = v;
         }
     };
-    float acc[kSxTW];
-#pragma unroll
-    for (uint32_t b = 0; b < kSxTW; ++b) acc[b] = 0.0f;
+    float acc = 0.0f;
     const uint32_t nc = hidden / kSxCols;
     gload(0u);
     lstore(0u);
@@ -343,15 +335,12 @@ __global__ __launch_bounds__(64 * kSxWaves) void router_chain_sx(
 #pragma unroll
         for (uint32_t q = 0; q < NQ; ++q) {
             const float4 w = tl[q * PITCH];
-#pragma unroll
-            for (uint32_t b = 0; b < kSxTW; ++b) {
-                const float4 xv = *(const float4 *)(xr[b] + c * kSxCols + 4u * q);
-                float p;
-                p = w.x * xv.x; acc[b] = acc[b] + p;
-                p = w.y * xv.y; acc[b] = acc[b] + p;
-                p = w.z * xv.z; acc[b] = acc[b] + p;
-                p = w.w * xv.w; acc[b] = acc[b] + p;
-            }
+            const float4 xv = *(const float4 *)(xr + c * kSxCols + 4u * q);
+            float p;
+            p = w.x * xv.x; acc = acc + p;
+            p = w.y * xv.y; acc = acc + p;
+            p = w.z * xv.z; acc = acc + p;
+            p = w.w * xv.w; acc = acc + p;
         }
         /* the other buffer was last read before the previous barrier */
         if (c + 1u < nc) lstore((c + 1u) & 1u);
@@ -359,11 +348,17 @@ __global__ __launch_bounds__(64 * kSxWaves) void router_chain_sx(
         if (c + 2u < nc) gload(c + 2u);
     }
     const uint32_t e = e0 + lane;
-#pragma unroll
-    for (uint32_t b = 0; b < kSxTW; ++b) {
-        if (tb + b < tokens && e < experts) logits[(size_t)(tb + b) * experts + e] = acc[b];
-    }
+    if (store && e < experts) logits[(size_t)t * experts + e] = acc;
     if (bad) kq_flag(status, KQ_DEV_INPUT);
+}
+
+__global__ __launch_bounds__(64 * kSxWaves) void router_chain_sx(
+    const float *__restrict__ router, const float *__restrict__ hidden_states, uint32_t tokens,
+    uint32_t experts, uint32_t hidden, float *__restrict__ logits, uint32_t *status) {
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t t = blockIdx.x * kSxWaves + wave;
+    chain_sx(router, hidden_states, experts, hidden, blockIdx.y * 64u, t < tokens ? t : tokens - 1u,
+             t < tokens, logits, status);
 }
 
 /* Maximum over the 64 lanes of a wave, returned in every lane: DPP within
@@ -1355,17 +1350,23 @@ __global__ __launch_bounds__(1024) void route_select(RouteArgs a) {
  *      the k-th one's) is out. The others, 11 of 512 on N(0, 1) activations
  *      at k = 10, get the CPU's exact chains, and from those the
  *      exact expf terms: the selection and its order follow where the terms
- *      are equal (ids ascending, as the CPU orders equal probabilities) or
- *      apart by more than the spacing of their quotients by the common sum;
- *      two terms one step apart, equal terms across the selection's edge,
+ *      are equal (ids ascending, as the CPU orders equal probabilities; its
+ *      partial selection's rule where they lie across the selection's edge)
+ *      or apart by more than the spacing of their quotients by the common
+ *      sum. A row of zeros, whose logits are all +0, selects the first ids.
+ *      Two terms one step apart, more than kCandMax candidates,
  *      probabilities that may underflow and anything non-finite do not decide.
- *   4. route_fallback: the tokens left undecided (3e-5 of random ones) run
- *      every chain and the reference's route finish.
+ *   4. route_left_chains, route_left_finish: the tokens left undecided (3e-5
+ *      of random ones) run every chain and the reference's route finish,
+ *      over the whole device as the route without candidates does: where no
+ *      token decides, that route's time comes on top (a layer of 512 tokens
+ *      at 2048 x 512 under an all-zero router: 325 us, 243 by that route
+ *      alone, 981 with a workgroup per token).
  *
- * The four launches against the chains and the route finish, us: 7 tokens x
- * 2560 columns 39 / 64, 201 x 2560 42 / 61, 512 x 2048 45 / 70, 2499 x 2560
- * 92 / 334. A candidate wave is bound by its chain (8 cycles per dependent
- * add, 8.5 us at 2560) and the loads that lead up to it.
+ * The launches against the chains and the route finish, us: 7 tokens x 2560
+ * columns 39 / 64, 201 x 2560 42 / 61, 512 x 2048 45 / 70, 2499 x 2560 92 /
+ * 334. A candidate wave is bound by its chain (8 cycles per dependent add, 8.5
+ * us at 2560) and the loads that lead up to it.
  *
  * The bound. With s = |w| |x| (2-norms), sum |w_i x_i| <= s (Cauchy-Schwarz)
  * and n columns: the CPU's chain errs by at most n u s (1 + n u), u = 2^-24,
@@ -1659,6 +1660,19 @@ __global__ __launch_bounds__(256) void route_candidates(RouteManyArgs a) {
         undecided();
         return;
     }
+    if (xn == 0.0f) { /* every probability 1 / E: the first K ids */
+        const float p = 1.0f / (float)a.experts;
+        float sum = 0.0f;
+        for (uint32_t i = 0; i < K; ++i) sum += p;
+        if (lane < K) {
+            const size_t o = (size_t)t * K + lane;
+            a.ids[o] = lane;
+            a.weights[o] = p / sum;
+            a.order[o] = lane;
+        }
+        if (lane == 0u) a.shared_scale[t] = kq_sigmoid(a.shared_logit[t]);
+        return;
+    }
     top = wave_max(top);
     /* L: the K-th largest lower bound, with multiplicity */
     int kth = kNone;
@@ -1771,19 +1785,49 @@ __global__ __launch_bounds__(256) void route_candidates(RouteManyArgs a) {
         srt_id[w][rank] = id;
     }
     wave_sync();
-    const bool sel = lane < K;
-    const float se = sel ? srt_ex[w][lane] : 0.0f;
-    const uint32_t si = sel ? srt_id[w][lane] : 0xffffffffu;
+    /* the terms from the K-th on up, and those equal to it */
+    float se = have ? srt_ex[w][lane] : -1.0f;
+    uint32_t si = have ? srt_id[w][lane] : 0xffffffffu;
+    const float edge = rdl_f32(se, K - 1u);
+    const bool in = se >= edge;
     const float ne = lane + 1u < n ? srt_ex[w][lane + 1u] : 0.0f;
     /* quotients by one sum differ after rounding when they are a unit in
      * the last place (at most 2^-23 of them) apart */
     const bool apart = lane + 1u >= n || se - ne > 1.02f * 0x1p-23f * se;
-    const bool ok = !sel || (kq_isfinite(srt_l[w][lane]) && srt_l[w][lane] - m > -75.0f &&
-                             (apart || (lane + 1u < K && se == ne)));
+    const bool ok = !in || (kq_isfinite(srt_l[w][lane]) && srt_l[w][lane] - m > -75.0f &&
+                            (apart || se == ne));
     if (__ballot(!ok) != 0ull || __ballot(have && !kq_isfinite(l)) != 0ull) {
         undecided();
         return;
     }
+    const uint64_t in_mask = __ballot(in);
+    const uint32_t n_in = (uint32_t)__popcll(in_mask);
+    if (n_in > K) {
+        /* equal terms across the edge, as route_finish_body: those kept are
+         * the last of the ones that the first K of all these ids hold */
+        uint32_t upto = 0;
+        for (uint32_t i = 0; i < n_in; ++i)
+            upto += (uint32_t)((uint32_t)__builtin_amdgcn_readlane((int)si, (int)i) <= si);
+        const bool above = se > edge;
+        const uint32_t g = (uint32_t)__popcll(__ballot(above)), need = K - g;
+        const bool tie = in && !above && upto <= K;
+        const uint64_t ties = __ballot(tie);
+        const uint32_t nt = (uint32_t)__popcll(ties), drop = nt > need ? nt - need : 0u;
+        if (nt < need) { /* cannot be: the first K ids hold K - g ties or more */
+            undecided();
+            return;
+        }
+        const uint32_t before = bits_below(ties);
+        wave_sync();
+        if (tie && before >= drop) {
+            srt_ex[w][g + before - drop] = se;
+            srt_id[w][g + before - drop] = si;
+        }
+        wave_sync();
+        se = have ? srt_ex[w][lane] : -1.0f;
+        si = have ? srt_id[w][lane] : 0xffffffffu;
+    }
+    const bool sel = lane < K;
     float sum = 0.0f;
     uint32_t by_id = 0;
     for (uint32_t i = 0; i < K; ++i) {
@@ -1799,18 +1843,33 @@ __global__ __launch_bounds__(256) void route_candidates(RouteManyArgs a) {
     if (lane == 0u) a.shared_scale[t] = kq_sigmoid(a.shared_logit[t]);
 }
 
-/* the undecided tokens: every chain, then the reference's route finish */
-template <uint32_t HIDDEN>
-__global__ __launch_bounds__(1024) void route_fallback(RouteManyArgs a) {
+/* the undecided tokens: every chain, eight tokens and 64 experts a workgroup */
+__global__ __launch_bounds__(64 * kSxWaves) void route_left_chains(RouteManyArgs a) {
+    const uint32_t n = *a.n_left;
+    const uint32_t groups = (n + kSxWaves - 1u) / kSxWaves, items = groups * ((a.experts + 63u) / 64u);
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    for (uint32_t i = blockIdx.x; i < items; i += gridDim.x) {
+        const uint32_t k = i % groups * kSxWaves + wave;
+        const uint32_t t = __builtin_amdgcn_readfirstlane(a.left[k < n ? k : n - 1u]);
+        chain_sx(a.router, a.x, a.experts, a.hidden, i / groups * 64u, t, k < n, a.logits, a.status);
+    }
+}
+
+/* and the reference's route finish, a token a workgroup */
+__global__ __launch_bounds__(1024) void route_left_finish(RouteManyArgs a) {
     const uint32_t n = *a.n_left;
     for (uint32_t i = blockIdx.x; i < n; i += gridDim.x) {
         const uint32_t t = a.left[i];
-        exact_all_rows<HIDDEN>(a.router, a.sgw, a.x + (size_t)t * HIDDEN, a.experts,
-                               a.logits + (size_t)t * a.experts, a.shared_logit + t, a.status);
         route_finish_body(t, a.logits, a.shared_logit, a.experts, a.top_k, a.probs, a.ids,
                           a.weights, a.order, a.shared_scale, a.status);
         __syncthreads();
     }
+}
+
+/* threads of a route finish: one per expert, and a wave for the sum */
+uint32_t finish_threads(uint32_t experts) {
+    const uint32_t n = 64u * ((experts + 63u) / 64u + 1u);
+    return n < 1024u ? n : 1024u;
 }
 
 /* 64 x 256 tiles read the fewest bytes a product; with fewer than 40 of them
@@ -1845,15 +1904,12 @@ hipError_t launch_route_many(const RouteManyArgs &a, hipStream_t s) {
         hipLaunchKernelGGL(route_candidates<8>, grid, dim3(256), 0, s, a);
     else
         hipLaunchKernelGGL(route_candidates<16>, grid, dim3(256), 0, s, a);
-    const dim3 fg(a.tokens < 64u ? a.tokens : 64u);
-    switch (a.hidden) {
-    case 256: hipLaunchKernelGGL(route_fallback<256u>, fg, dim3(1024), 0, s, a); break;
-    case 512: hipLaunchKernelGGL(route_fallback<512u>, fg, dim3(1024), 0, s, a); break;
-    case 1024: hipLaunchKernelGGL(route_fallback<1024u>, fg, dim3(1024), 0, s, a); break;
-    case 2048: hipLaunchKernelGGL(route_fallback<2048u>, fg, dim3(1024), 0, s, a); break;
-    case 2560: hipLaunchKernelGGL(route_fallback<2560u>, fg, dim3(1024), 0, s, a); break;
-    default: return hipErrorInvalidValue;
-    }
+    /* as many workgroups as the device holds, when every token is left */
+    const uint32_t items = (a.tokens + kSxWaves - 1u) / kSxWaves * ((a.experts + 63u) / 64u);
+    hipLaunchKernelGGL(route_left_chains, dim3(items < 1024u ? items : 1024u), dim3(64u * kSxWaves), 0,
+                       s, a);
+    hipLaunchKernelGGL(route_left_finish, dim3(a.tokens < 1024u ? a.tokens : 1024u),
+                       dim3(finish_threads(a.experts)), 0, s, a);
     return hipGetLastError();
 }
 
@@ -2589,8 +2645,7 @@ extern "C" hipError_t kq_launch_moe_route(const kq_launch_moe_dims *d, const flo
     const uint32_t ep = pad64(d->experts + 1u);
     const uint32_t groups = (d->experts + 1u + kRtRows - 1u) / kRtRows;
     bool fused = tokens == 1u;
-    uint32_t fin = 64u * ((d->experts + 63u) / 64u + 1u);
-    if (fin > 1024u) fin = 1024u;
+    const uint32_t fin = finish_threads(d->experts);
     /* one token, ids only needed exactly: the bounds, then the selection
      * (certified, refined or exact) in one workgroup */
     if (fused && certify && d->top_k <= kMaxTopK) {
@@ -2644,8 +2699,8 @@ extern "C" hipError_t kq_launch_moe_route(const kq_launch_moe_dims *d, const flo
     }
 #undef KQ_ROUTER_DECODE
     /* several tokens, only the ids exactly, and a gate/up pass that reads the
-     * split activations (KQ_ROUTE_ONE's hidden sizes): by candidates */
-    if (tokens > 1u && certify && stage != nullptr && d->top_k <= kCandMaxK) {
+     * split activations: by candidates (stage_row's and the chunks' widths) */
+    if (tokens > 1u && certify && stage != nullptr && d->top_k <= kCandMaxK && d->hidden % 256u == 0u) {
         RouteManyArgs a;
         a.router = router;
         a.sgw = shared_gate_weight;
@@ -2677,9 +2732,8 @@ extern "C" hipError_t kq_launch_moe_route(const kq_launch_moe_dims *d, const flo
      * finish forms the shared gate's logit */
     const bool in_place = !fused && d->hidden % kSxCols == 0u;
     if (in_place) {
-        const uint32_t per_wg = kSxTW * kSxWaves;
         hipLaunchKernelGGL(router_chain_sx,
-                           dim3((tokens + per_wg - 1u) / per_wg, (d->experts + 63u) / 64u),
+                           dim3((tokens + kSxWaves - 1u) / kSxWaves, (d->experts + 63u) / 64u),
                            dim3(64u * kSxWaves), 0, s, router, hidden, tokens, d->experts,
                            d->hidden, ws->logits, status);
     } else if (!fused) {

@@ -47,15 +47,21 @@ def oracle_ids(H, E, K, router, x):
     return np.stack([kq_oracle.moe_route(dims, (kq_oracle.F32, router), r)[2] for r in x])
 
 
-@pytest.mark.parametrize("pattern", ["random", "duplicates", "zero", "near-tie", "quantised"])
-@pytest.mark.parametrize("H,E,K,T", [(256, 24, 3, 2), (512, 64, 12, 19), (1024, 130, 8, 67),
-                                     (2048, 512, 10, 33), (2560, 512, 10, 201), (256, 1000, 32, 130),
-                                     (512, 600, 10, 900)])
+PATTERNS = ["random", "duplicates", "triples", "zero", "near-tie", "quantised"]
+
+
+@pytest.mark.parametrize("H,E,K,T,pattern", [
+    (*shape, p) for shape in ((256, 24, 3, 2), (512, 64, 12, 19), (1024, 130, 8, 67),
+                              (2048, 512, 10, 33), (2560, 512, 10, 201), (256, 1000, 32, 130),
+                              (512, 600, 10, 900), (1024, 24, 3, 2), (1024, 1000, 32, 130))
+    for p in PATTERNS] + [(2560, 512, 10, 1281, "random"), (1024, 512, 10, 1300, "zero"),
+                          (2048, 600, 10, 900, "triples")])
 def test_ids_exact(ctx, H, E, K, T, pattern):
-    # one and more tokens per tile of the approximate logits (16 x 32 tiles,
-    # and 64 x 64 from 524,288 logits on), expert counts off the tiles and
-    # above 512, up to 32 selected; tokens of zeros, of tiny and of large
-    # activations (whose lower probabilities underflow) among the others
+    # from 1,024 columns on the candidate route: one and more tokens per tile
+    # of the approximate logits (64 x 64, and 64 x 256 from 40 of those on: 900
+    # and 1,281 tokens), expert counts off the tiles and above 512, up to 32
+    # selected; tokens of zeros, of tiny and of large activations (whose lower
+    # probabilities underflow) among the others
     key = S.stream_key(S.W_MOE, 60, H + E, K)
     w = S.moe_weights(S.W_MOE + 60, H, E, I, I)
     router = S.normal_f32(key, E * H, 0.02).reshape(E, H)
@@ -64,6 +70,11 @@ def test_ids_exact(ctx, H, E, K, T, pattern):
     if pattern == "duplicates":
         # equal logits inside and across the selection's edge
         router[rng.integers(0, E, E // 3)] = router[rng.integers(0, E, E // 3)]
+    elif pattern == "triples":
+        # equal logits across the edge of every token, few enough to decide
+        router[1::3] = router[0::3][: len(router[1::3])]
+        router[2::3] = router[0::3][: len(router[2::3])]
+        router = router[rng.permutation(E)]
     elif pattern == "zero":
         router[:] = 0.0
     elif pattern == "quantised":
