@@ -168,14 +168,14 @@ void kq_launch_moe_ws_carve(const kq_launch_moe_dims *d, uint32_t tokens, void *
                             kq_launch_moe_ws *ws);
 int kq_launch_moe_supported(const kq_launch_moe_dims *d, const kq_launch_moe_weights *w);
 /* logits (+ shared gate logit), softmax, partial-selection top-k, weights.
- * certify != 0 (one token, only the ids needed exactly): selects from exact
- * product sums with a proven error bound when the bound separates the
- * selection, from the exact chains of the contenders when that separates
- * it, and from every exact chain otherwise; the logits and probabilities
- * are then not always written and the weights are within fp32 tolerance of
- * the CPU's. ids_out (optional) also receives the ids. stage (optional,
- * several tokens): where the route finish also splits every token's row for
- * the grouped gate/up pass (kq_launch_moe_grouped_stage). */
+ * certify != 0 (only the ids needed exactly): selects from sums with an error
+ * bound when the bound separates the selection, from the exact chains of the
+ * contenders when that separates it, and from every exact chain otherwise; the
+ * logits and probabilities are then not always written and the weights are
+ * within fp32 tolerance of the CPU's. (Several tokens: where stage is given.)
+ * ids_out (optional) also receives the ids. stage (optional, several tokens):
+ * where every token's row is also split for the grouped gate/up pass
+ * (kq_launch_moe_grouped_stage). */
 hipError_t kq_launch_moe_route(const kq_launch_moe_dims *d, const float *router,
                                const float *shared_gate_weight, const float *hidden,
                                uint32_t tokens, const kq_launch_moe_ws *ws, uint32_t *status,

@@ -837,6 +837,15 @@ __device__ __forceinline__ void route_finish_body(
     }
 }
 
+/* token t's ids, written by this workgroup, to the caller's copy (if any) */
+__device__ __forceinline__ void copy_ids(uint32_t t, uint32_t top_k, const uint32_t *ids,
+                                         uint32_t *ids_out) {
+    if (ids_out == nullptr) return;
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < top_k; i += blockDim.x)
+        ids_out[(size_t)t * top_k + i] = ids[(size_t)t * top_k + i];
+}
+
 /* One workgroup per token. With sgw given, the token's shared gate logit
  * is first formed here as sgw . x in any order (it only feeds the sigmoid
  * gate, compared by tolerance); thread 0 stores it and reads it back in
@@ -847,7 +856,7 @@ __global__ __launch_bounds__(1024) void route_finish(
     uint32_t experts, uint32_t top_k, float *__restrict__ probs_all, uint32_t *__restrict__ ids_all,
     float *__restrict__ weights_all, uint32_t *__restrict__ order_all,
     float *__restrict__ shared_scale, uint32_t *status, const float *__restrict__ sgw,
-    const float *__restrict__ hidden_states, uint32_t hidden, void *stage) {
+    const float *__restrict__ hidden_states, uint32_t hidden, void *stage, uint32_t *ids_out) {
     if (stage != nullptr) kq::stage_row(hidden_states, blockIdx.x, gridDim.x, hidden, stage, status);
     if (sgw != nullptr) {
         __shared__ float part[16];
@@ -877,6 +886,7 @@ __global__ __launch_bounds__(1024) void route_finish(
     }
     route_finish_body(blockIdx.x, logits_all, shared_logit, experts, top_k, probs_all, ids_all,
                       weights_all, order_all, shared_scale, status);
+    copy_ids(blockIdx.x, top_k, ids_all, ids_out);
 }
 
 /*
@@ -1389,7 +1399,7 @@ struct RouteManyArgs {
     float *parts;       /* approximate logits' parts from the third on */
     uint32_t splits;
     float *logits, *shared_logit, *probs;
-    uint32_t *ids;
+    uint32_t *ids, *ids_out; /* ids_out: the caller's copy (may be null) */
     float *weights;
     uint32_t *order;    /* order[t K] holds token t's scaled 2-norm until its selection is written */
     float *shared_scale;
@@ -1667,6 +1677,7 @@ __global__ __launch_bounds__(256) void route_candidates(RouteManyArgs a) {
         if (lane < K) {
             const size_t o = (size_t)t * K + lane;
             a.ids[o] = lane;
+            if (a.ids_out != nullptr) a.ids_out[o] = lane;
             a.weights[o] = p / sum;
             a.order[o] = lane;
         }
@@ -1837,6 +1848,7 @@ __global__ __launch_bounds__(256) void route_candidates(RouteManyArgs a) {
     if (sel) {
         const size_t o = (size_t)t * K;
         a.ids[o + lane] = si;
+        if (a.ids_out != nullptr) a.ids_out[o + lane] = si;
         a.weights[o + lane] = se / sum;
         a.order[o + by_id] = lane;
     }
@@ -1862,6 +1874,7 @@ __global__ __launch_bounds__(1024) void route_left_finish(RouteManyArgs a) {
         const uint32_t t = a.left[i];
         route_finish_body(t, a.logits, a.shared_logit, a.experts, a.top_k, a.probs, a.ids,
                           a.weights, a.order, a.shared_scale, a.status);
+        copy_ids(t, a.top_k, a.ids, a.ids_out);
         __syncthreads();
     }
 }
@@ -2720,6 +2733,7 @@ extern "C" hipError_t kq_launch_moe_route(const kq_launch_moe_dims *d, const flo
         a.shared_logit = ws->shared_logit;
         a.probs = ws->probs;
         a.ids = ws->ids;
+        a.ids_out = ids_out;
         a.weights = ws->weights;
         a.order = ws->order;
         a.shared_scale = ws->shared_scale;
@@ -2751,14 +2765,8 @@ extern "C" hipError_t kq_launch_moe_route(const kq_launch_moe_dims *d, const flo
     hipLaunchKernelGGL(route_finish, dim3(tokens), dim3(fin), 0, s, ws->logits, ws->shared_logit,
                        d->experts, d->top_k, ws->probs, ws->ids, ws->weights, ws->order,
                        ws->shared_scale, status, in_place ? shared_gate_weight : nullptr, hidden,
-                       d->hidden, stage);
-    e = hipGetLastError();
-    /* the one-token selection writes the caller's ids itself; here they
-     * are copied (several tokens, or a hidden size without an instance) */
-    if (e == hipSuccess && ids_out != nullptr)
-        e = hipMemcpyAsync(ids_out, ws->ids, (size_t)tokens * d->top_k * 4u,
-                           hipMemcpyDeviceToDevice, s);
-    return e;
+                       d->hidden, stage, ids_out);
+    return hipGetLastError();
 }
 
 extern "C" hipError_t kq_launch_moe_route_finish(const float *logits, const float *shared_logit,
@@ -2772,7 +2780,7 @@ extern "C" hipError_t kq_launch_moe_route_finish(const float *logits, const floa
         return hipErrorInvalidValue;
     hipLaunchKernelGGL(route_finish, dim3(tokens), dim3(fin), 0, s, logits,
                        const_cast<float *>(shared_logit), experts, top_k, probs, ids, weights,
-                       order, shared_scale, status, nullptr, nullptr, 0u, nullptr);
+                       order, shared_scale, status, nullptr, nullptr, 0u, nullptr, nullptr);
     return hipGetLastError();
 }
 

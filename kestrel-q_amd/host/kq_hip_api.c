@@ -1346,18 +1346,15 @@ kq_status kq_hip_moe_execute_quantized(kq_hip_context *c, const kq_hip_moe_confi
     grouped = tokens >= KQ_GROUPED_MIN_TOKENS && kq_launch_moe_grouped_supported(&d, &lw);
     stage = grouped ? kq_launch_moe_grouped_stage(&d, &lw, &ws) : NULL;
     /* the layer needs the CPU's expert ids exactly and its weights to fp32
-     * tolerance: one token may take the certified routing */
+     * tolerance: certified routing; it writes the caller's ids too */
     e = kq_launch_moe_route(&d, w->router, w->shared_gate_weight, hidden, (uint32_t)tokens, &ws,
-                            c->d_status, 1, tokens == 1u ? ids : NULL, stage, c->stream);
+                            c->d_status, 1, ids, stage, c->stream);
     if (e == hipSuccess && grouped)
         e = kq_launch_moe_grouped(&d, &lw, hidden, (uint32_t)tokens, &ws, stage != NULL, out,
                                   c->d_status, c->stream);
     else if (e == hipSuccess)
         e = kq_launch_moe_experts(&d, &lw, hidden, (uint32_t)tokens, &ws, out, c->d_status,
                                   c->stream);
-    /* one token: the route kernel wrote the caller's ids itself */
-    if (e == hipSuccess && ids != NULL && tokens > 1u)
-        e = hipMemcpyAsync(ids, ws.ids, tokens * d.top_k * 4u, hipMemcpyDeviceToDevice, c->stream);
     return finish(c, e, "MoE execute launch", diag);
 }
 
