@@ -57,7 +57,8 @@ PATTERNS = ["random", "duplicates", "triples", "zero", "near-tie", "quantised"]
     for p in PATTERNS] + [(2560, 512, 10, 1281, "random"), (1024, 512, 10, 1300, "zero"),
                           (2048, 600, 10, 900, "triples")])
 def test_ids_exact(ctx, H, E, K, T, pattern):
-    # from 1,024 columns on the candidate route: one and more tokens per tile
+    # from 1,024 columns or 524,288 logits on the candidate route, the chains
+    # of every expert below: one and more tokens per tile
     # of the approximate logits (64 x 64, and 64 x 256 from 40 of those on: 900
     # and 1,281 tokens), expert counts off the tiles and above 512, up to 32
     # selected; tokens of zeros, of tiny and of large activations (whose lower
@@ -96,10 +97,11 @@ def test_ids_exact(ctx, H, E, K, T, pattern):
     assert bad.size == 0, (bad[:5], ids[bad[:2]], want[bad[:2]])
 
 
-def test_output_with_ties(ctx):
-    # the layer's output where some tokens take the whole route: weights and
-    # combine order are those of the ids
-    H, E, K, T = 512, 48, 5, 40
+@pytest.mark.parametrize("H", [512, 1024])
+def test_output_with_ties(ctx, H):
+    # the layer's output where some tokens tie: weights and combine order are
+    # those of the ids
+    E, K, T = 48, 5, 40
     w = S.moe_weights(S.W_MOE + 61, H, E, I, I)
     r = w["router"].reshape(E, H)
     r[7] = r[30]
@@ -113,9 +115,10 @@ def test_output_with_ties(ctx):
     assert_close(out, ref, exact=exact.moe(dims, ROLES, w, x, ids))
 
 
+@pytest.mark.parametrize("H", [512, 1024])
 @pytest.mark.parametrize("where", ["activation", "router", "overflow"])
-def test_fails_closed(ctx, where):
-    H, E, K, T = 512, 64, 6, 21
+def test_fails_closed(ctx, where, H):
+    E, K, T = 64, 6, 21
     w = S.moe_weights(S.W_MOE + 62, H, E, I, I)
     x = S.normal_f32(S.stream_key(S.W_MOE, 62), T * H).reshape(T, H)
     good = run(ctx, w, H, E, K, x)
