@@ -28,9 +28,10 @@
  *     row tile) sequence side by side, so an item's tokens come to its L2
  *     once; the loads run one step ahead across tiles.
  *
- * Measured at 2499 tokens, 512 experts, 10 per token, 2560 x 640: gate/up Q4_K
- * 779 -> 560 us, down Q5_1 592 -> 520 us, the Q8_0 shared expert (as 64-token
- * items of a dense product) 332 -> 124 us. What bounds it: the matrix cores
+ * Measured at 2499 tokens, 512 experts, 10 per token, 2560 x 640, against the
+ * 16-token passes: gate/up Q4_K 779 -> 587 us, down Q5_1 592 -> 510 us, the Q8_0
+ * shared expert (as 64-token items of a dense product) 332 -> 133 us. Error of
+ * the layer against binary64 1.09e-6, as theirs. What bounds it: the matrix cores
  * are busy for 31 % and 18 % of that, the vector ALU (decode, scales) about as
  * long, and with two waves of 250 registers per SIMD the two overlap little;
  * sixteen waves of one tile each (128 registers, spilled) took 771 us for the
@@ -52,6 +53,11 @@ constexpr uint32_t kM = 64;       /* tokens per item */
 constexpr uint32_t kDies = 8;     /* workgroups go round-robin over the dies */
 constexpr uint32_t kShared = 0x80000000u;
 constexpr uint32_t kOut = 0x80000000u; /* an offset past every buffer */
+/* Steps (of 128 columns) whose products a sum takes; the output holds the sum
+ * of the runs before. The shared expert's 2560 columns in one sum err by 3.0e-7
+ * of its output, in four by 2.2e-7, as in dense_q8's parts (two: 2.4e-7); 24
+ * us more of the 2499-token layer. The K formats' few blocks are one sum. */
+constexpr uint32_t kRun = 5;
 
 /* a wave-uniform dword written by an earlier launch */
 __device__ __forceinline__ uint32_t uniform(const uint32_t *p) {
@@ -324,19 +330,20 @@ __global__ __launch_bounds__(NW * 64) void gm_product(GmArgs a) {
     };
 
     /* ---- products ---- */
-    f4 acc[NT][4], macc[NT][4];
+    /* (Q5_1: in 2^-5 of the others' scale, that of the sums the min term adds) */
+    f4 acc[NT][4];
     auto clear = [&]() {
 #pragma unroll
         for (uint32_t m = 0; m < NT; ++m)
 #pragma unroll
-            for (int f = 0; f < 4; ++f) acc[m][f] = macc[m][f] = f4{0.f, 0.f, 0.f, 0.f};
+            for (int f = 0; f < 4; ++f) acc[m][f] = f4{0.f, 0.f, 0.f, 0.f};
     };
     clear();
     bool bad = false, malformed = false;
     /* the 32-column formats' many scales: 0, or NaN once a scale was not finite: one multiply-add a pair of them */
     h2 finite = splat(0.0f);
     auto check = [&](uint32_t pair) { finite = fma2(as_h2(pair), splat(0.0f), finite); };
-    uint32_t c_t = lo, c_tile = lo % nt, c_step = 0u, par = 0u;
+    uint32_t c_t = lo, c_tile = lo % nt, c_step = 0u, c_run = 0u, par = 0u;
     Item cur = item(lo / nt);
     uint4 hd[2], qa[2], qb[2], qh[2] = {};
 
@@ -397,8 +404,7 @@ __global__ __launch_bounds__(NW * 64) void gm_product(GmArgs a) {
                 for (uint32_t f = 0; f < NF; ++f) {
                     const f4 mm = mfma16(*(const h4 *)(p + 512u * f), mins, zero);
 #pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        acc[m][f][e] = fmaf(dm, mm[e], fmaf(dw, t[m][f][e], acc[m][f][e]));
+                    for (int e = 0; e < 4; ++e) acc[m][f][e] += fmaf(dw, t[m][f][e], dm * mm[e]);
                 }
             }
         } else if constexpr (FMT == KQ_LAUNCH_Q6_K) {
@@ -481,7 +487,7 @@ __global__ __launch_bounds__(NW * 64) void gm_product(GmArgs a) {
                         const uint2 qv = *(const uint2 *)(blk + 2u + 2u * (g & 1u));
                         c0 = ((qv.x >> shn) & 0x0f0f0f0fu) | spread4(hbits & 15u);
                         c1 = ((qv.y >> shn) & 0x0f0f0f0fu) | spread4(hbits >> 4);
-                        d[m] = half_bits(dm);
+                        d[m] = half_bits(dm) * 0x1p-5f;
                         mins[m][s] = dm >> 16;
                         check(dm);
                     } else if (s % 2u == 0u) {
@@ -537,13 +543,13 @@ __global__ __launch_bounds__(NW * 64) void gm_product(GmArgs a) {
                                                                     (mins[m][2] | (mins[m][3] << 16)) & on));
 #pragma unroll
                     for (uint32_t f = 0; f < NF; ++f)
-                        macc[m][f] = mfma16(*(const h4 *)(p + 256u * f), mn, macc[m][f]);
+                        acc[m][f] = mfma16(*(const h4 *)(p + 256u * f), mn, acc[m][f]);
                 }
             }
         }
     };
     /* the finished tile: token i = 16 f + 4 g + q, row of this lane */
-    auto store = [&]() {
+    auto store = [&](bool add) {
         const bool sh = (cur.ex & kShared) != 0u;
         const uint32_t pos0 = sh && !a.plain ? a.pairs + cur.first : cur.first;
         const uint32_t col = sh && a.plain ? a.rows : 0u;
@@ -569,9 +575,8 @@ __global__ __launch_bounds__(NW * 64) void gm_product(GmArgs a) {
                     for (uint32_t m = 0; m < NT; ++m) {
                         const uint32_t row = c_tile * TROWS + 16u * NT * w + 16u * m + j;
                         const bool valid = i < cur.count && row < a.rows;
-                        float v = acc[m][f][q];
-                        if constexpr (S::MINS != 0u) v = fmaf(32.0f, macc[m][f][q], v);
-                        v = ldexpf(v, -sg);
+                        float v = ldexpf(acc[m][f][q], (S::MINS != 0u ? 5 : 0) - sg);
+                        if (add && valid) v += o[row];
                         bad |= valid && !kq_isfinite(v);
                         if (valid) o[row] = v;
                     }
@@ -605,10 +610,19 @@ __global__ __launch_bounds__(NW * 64) void gm_product(GmArgs a) {
         case 3u: product(std::integral_constant<uint32_t, 3u>{}, img, slot); break;
         default: product(std::integral_constant<uint32_t, 4u>{}, img, slot); break;
         }
-        if (++c_step == steps) {
-            store();
+        ++c_step;
+        if constexpr (!GU) {
+            if (++c_run == kRun && c_step != steps) {
+                store(c_step != kRun);
+                clear();
+                c_run = 0u;
+            }
+        }
+        if (c_step == steps) {
+            store(!GU && steps > kRun);
             clear();
             c_step = 0u;
+            c_run = 0u;
             c_t += peers;
             c_tile += peers;
             if (c_tile >= nt && k + 1u < n) {

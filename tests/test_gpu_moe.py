@@ -708,6 +708,37 @@ def test_moe_prefill_many_per_expert(ctx, H, E, K, I, T, g, d, sg, sd):
     assert_close(out, ref, exact=ex)
 
 
+def test_moe_prefill_many_shared_sums(ctx):
+    # The shared expert's 2560 columns where 20 and more tokens meet each
+    # expert: its sums err by 2.2e-7 of the output, the three products and the
+    # gate together; 3.0e-7 where a row's 80 blocks are one sum.
+    H, E, K, I, T = 2560, 8, 4, 640, 130
+    seed = S.W_MOE + 7200
+    w = S.moe_weights(seed, H, E, I, I, gate_fmt="Q4_K", down_fmt="Q5_1", shared_gate_fmt="Q8_0",
+                      shared_down_fmt="Q8_0")
+    w["down"].reshape(-1, 24)[:, :4] = 0  # routed experts give zeros
+    x = S.normal_f32(S.stream_key(seed, S.R_HIDDEN), T * H).reshape(T, H)
+    cfg, t = kq_hip.MoeConfig(H, E, K, I, I), kq_hip.TYPE_IDS
+    n = cfg.scratch_bytes(T)
+    bufs = {k: ctx.upload(v) for k, v in w.items()}
+    scratch, dx, dout = ctx.alloc(n), ctx.upload(x), ctx.alloc(T * H * 4)
+    ctx.moe_execute(cfg, kq_hip.moe_weights(bufs, t["Q4_K"], t["Q5_1"], t["Q8_0"], t["Q8_0"]), dx,
+                    T, dout, None, scratch, n)
+    got = ctx.download(dout, np.float32, T * H).reshape(T, H).astype(np.float64)
+    for b in list(bufs.values()) + [scratch, dx, dout]:
+        b.close()
+    cfg.close()
+
+    def mat(role, rows, cols):
+        return kq_oracle.dequantize(t["Q8_0"], w[role]).reshape(rows, cols).astype(np.float64)
+
+    x64 = x.astype(np.float64)
+    gate, up = x64 @ mat("shared_gate", I, H).T, x64 @ mat("shared_up", I, H).T
+    out = (gate / (1.0 + np.exp(-gate)) * up) @ mat("shared_down", H, I).T
+    out *= (1.0 / (1.0 + np.exp(-(x64 @ w["shared_gate_weight"].astype(np.float64)))))[:, None]
+    assert np.linalg.norm(got - out) <= 2.6e-7 * np.linalg.norm(out)
+
+
 def test_moe_reference_model_prefill_512(ctx):
     # The reference model's MoE layer (2560 / 512 experts / top-10 / 640,
     # Q4_K gate/up, Q5_1 down, Q8_0 shared) over 512 tokens: the grouped
