@@ -708,6 +708,59 @@ def test_moe_prefill_many_per_expert(ctx, H, E, K, I, T, g, d, sg, sd):
     assert_close(out, ref, exact=ex)
 
 
+# bytes of a scale in a block of each format
+SCALE_AT = {"Q4_K": (0, 2), "Q5_K": (0, 2), "Q6_K": (208,), "Q8_0": (0,), "Q5_1": (0, 2)}
+
+
+@pytest.mark.parametrize("H,E,K,I,T,g,d,sg,sd", [
+    (2560, 16, 4, 640, 83, "Q4_K", "Q5_1", "Q8_0", "Q8_0"),
+    (512, 8, 4, 640, 67, "Q5_K", "Q8_0", "Q8_0", "Q8_0"),
+    (2048, 16, 4, 512, 180, "Q4_K", "Q6_K", "Q4_K", "Q6_K"),
+], ids=["q4k-q5_1", "q5k-q8_0", "q4k-q6_k"])
+def test_moe_prefill_many_fails_closed(ctx, H, E, K, I, T, g, d, sg, sd):
+    # 20 and more tokens per expert: a non-finite scale in the last block of
+    # each role, a non-finite activation of the last token and products past
+    # binary32 fail the call; a good call after them gives what one gave before
+    seed = S.W_MOE + 7100 + H
+    w = S.moe_weights(seed, H, E, I, I, gate_fmt=g, down_fmt=d, shared_gate_fmt=sg,
+                      shared_down_fmt=sd)
+    x = S.normal_f32(S.stream_key(seed, S.R_HIDDEN), T * H).reshape(T, H)
+    cfg, t = kq_hip.MoeConfig(H, E, K, I, I), kq_hip.TYPE_IDS
+    n = cfg.scratch_bytes(T)
+    bufs = {k: ctx.upload(v) for k, v in w.items()}
+    scratch, dx, dout = ctx.alloc(n), ctx.upload(x), ctx.alloc(T * H * 4)
+
+    def run(b, xin):
+        ctx.moe_execute(cfg, kq_hip.moe_weights(b, t[g], t[d], t[sg], t[sd]), xin, T, dout, None,
+                        scratch, n)
+        return ctx.download(dout, np.uint32, T * H)
+
+    def refused(b, xin, name, what):
+        with pytest.raises(kq_hip.KqError) as e:
+            run(b, xin)
+        assert e.value.name == name, what
+
+    good = run(bufs, dx)
+    fmts = {"gate": g, "up": g, "down": d, "shared_gate": sg, "shared_up": sg, "shared_down": sd}
+    for role, fmt in fmts.items():
+        for at in SCALE_AT[fmt]:
+            bad = w[role].copy().reshape(-1, kq_hip.GEOMETRY[t[fmt]][1])
+            bad[-1, at:at + 2] = [0x00, 0x7E]  # NaN
+            db = ctx.upload(bad.reshape(-1))
+            refused({**bufs, role: db}, dx, "MALFORMED_QUANTIZED_DATA", (role, at))
+            db.close()
+    for value in (np.inf, np.nan, 1e30):
+        xb = x.copy()
+        xb[-1, -1 if value != 1e30 else slice(None)] = value
+        db = ctx.upload(xb)
+        refused(bufs, db, "NUMERIC_DOMAIN", value)
+        db.close()
+    assert np.array_equal(run(bufs, dx), good)
+    for b in list(bufs.values()) + [scratch, dx, dout]:
+        b.close()
+    cfg.close()
+
+
 def test_moe_prefill_many_shared_sums(ctx):
     # The shared expert's 2560 columns where 20 and more tokens meet each
     # expert: its sums err by 2.2e-7 of the output, the three products and the
