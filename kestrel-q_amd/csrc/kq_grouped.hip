@@ -1378,20 +1378,32 @@ static hipError_t launch_combine(const kq_launch_moe_dims *d, const kq_launch_mo
     return hipGetLastError();
 }
 
-/* Tokens per expert on average from which the 64-token products (kq_gemm.hip)
- * are the faster ones. Whole layer, 512 experts, 10 per token, 16-token passes
- * against them: 2560 x 640 Q4_K / Q5_1 at 16 tokens per expert (820 tokens)
- * 805 and 848 us, at 19.5 928 and 885, at 49 1979 and 1417; Q5_K / Q8_0 at 16
- * 872 and 910, at 19.5 1084 and 949. The mixed-tile passes of 2048 x 512 Q4_K /
- * Q6_K keep up for longer: at 27 692 and 780, at 49 1072 and 996, level near
- * 39. */
-static const uint32_t kWideTokens = 20u, kWideTokensMixed = 44u;
+/* Whether the 64-token products (kq_gemm.hip) are the faster ones. Their items
+ * are few and large: with few experts the device is not filled, and what is
+ * left in a last round weighs more. Whole layer, 16-token passes / 64-token
+ * products, us, at tokens per expert:
+ *   2560 x 640, Q4_K / Q5_1 (Q5_K / Q8_0 within 10 % of it):
+ *     512 experts  16: 808 / 861, 20: 1024 / 955, 50: 2105 / 1572
+ *     256          20: 550 / 551, 24: 592 / 570, 50: 1046 / 819
+ *     128          32: 402 / 416, 44: 504 / 461
+ *     64           50: 304 / 328, 64: 378 / 362, 80: 452 / 432
+ *     32           50: 251 / 250, 80: 314 / 316, 120: 440 / 335
+ *     16           80: 231 / 240, 120: 269 / 252;   8  120: 200 / 223
+ *   2048 x 512, Q4_K / Q6_K, whose mixed-tile passes keep up for longer:
+ *     512 experts  32: 783 / 818, 44: 1028 / 968, 120: 2652 / 2149
+ *     256          44: 509 / 512, 80: 871 / 911, 120: 1267 / 1150
+ *     64           80: 235 / 271, 120: 320 / 286;   16  80: 117 / 127, 120: 137 / 130 */
+static bool wide_faster(uint64_t pairs, uint32_t experts, bool mixed) {
+    if (pairs >= UINT64_C(100) * experts && pairs >= 1500u) return true;
+    return mixed ? pairs >= UINT64_C(44) * experts && pairs >= 22000u
+                 : pairs >= UINT64_C(12) * experts + 2900u;
+}
 
 static bool wide_supported(const kq_launch_moe_dims *d, const kq_launch_moe_weights *w,
                            uint32_t tokens, bool lds_shared, bool mixed) {
     const uint32_t npos = tokens * d->top_k + tokens;
     if (!gu_lds_routed(d, w) ||
-        (uint64_t)tokens * d->top_k < (uint64_t)d->experts * (mixed ? kWideTokensMixed : kWideTokens) ||
+        !wide_faster((uint64_t)tokens * d->top_k, d->experts, mixed) ||
         !kq_launch_gm_gate_up_supported(w->gate_type, d->inter, d->hidden, tokens) ||
         !kq_launch_gm_matrix_supported(w->down_type, d->hidden, d->inter, npos))
         return false;

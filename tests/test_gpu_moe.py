@@ -687,20 +687,20 @@ def test_moe_prefill_grouped_formats(ctx, H, E, K, I, T, g, d, sg, sd):
         b.close()
 
 
-# 20 and more tokens per expert on average (44 at 2048 x 512): up to 64 of them against each
-# decoded weight. Items of one to four 16-token fragments, an expert's second
-# item, the last of its tokens alone in one; row tiles that the rows do not
-# fill; every down format; a shared expert in the item list and beside it.
+# 100 and more tokens per expert on average (fewer where there are many experts): up to 64 of
+# them against each decoded weight. Items of one to four 16-token fragments, an
+# expert's second and third item; row tiles that the rows do not fill; every
+# down format; a shared expert in the item list and beside it.
 @pytest.mark.parametrize("H,E,K,I,T,g,d,sg,sd", [
-    (2560, 16, 4, 640, 83, "Q4_K", "Q5_1", "Q8_0", "Q8_0"),
-    (2560, 8, 4, 640, 67, "Q5_K", "Q8_0", "Q8_0", "Q8_0"),
-    (2048, 16, 4, 512, 180, "Q4_K", "Q6_K", "Q4_K", "Q6_K"),
-    (512, 3, 1, 512, 197, "Q4_K", "Q6_K", "Q4_K", "Q6_K"),
-    (256, 5, 2, 640, 129, "Q5_K", "Q5_1", "Q5_K", "Q5_1"),
-    (256, 4, 2, 512, 41, "Q4_K", "Q8_0", "Q4_K", "Q8_0"),
-    (1024, 4, 4, 640, 65, "Q4_K", "Q5_1", "Q4_K", "Q5_1"),
-], ids=["2560-q5_1", "2560-q5k-q8_0", "2048-q6_k", "512-q6_k", "256-q5k-q5_1", "256-q8_0",
-        "all-65"])
+    (2560, 16, 4, 640, 400, "Q4_K", "Q5_1", "Q8_0", "Q8_0"),
+    (1024, 8, 4, 640, 375, "Q5_K", "Q8_0", "Q8_0", "Q8_0"),
+    (2048, 16, 4, 512, 401, "Q4_K", "Q6_K", "Q4_K", "Q6_K"),
+    (512, 3, 1, 512, 1501, "Q4_K", "Q6_K", "Q4_K", "Q6_K"),
+    (256, 5, 2, 640, 751, "Q5_K", "Q5_1", "Q5_K", "Q5_1"),
+    (256, 4, 2, 512, 750, "Q4_K", "Q8_0", "Q4_K", "Q8_0"),
+    (1024, 4, 4, 640, 385, "Q4_K", "Q5_1", "Q4_K", "Q5_1"),
+], ids=["2560-q5_1", "1024-q5k-q8_0", "2048-q6_k", "512-q6_k", "256-q5k-q5_1", "256-q8_0",
+        "all-385"])
 def test_moe_prefill_many_per_expert(ctx, H, E, K, I, T, g, d, sg, sd):
     seed = S.W_MOE + 7000 + H + I + T
     out, ids, ref, tr, ex = run_layer(ctx, H, E, K, I, T, g, d, sg, sd, seed)
@@ -713,12 +713,12 @@ SCALE_AT = {"Q4_K": (0, 2), "Q5_K": (0, 2), "Q6_K": (208,), "Q8_0": (0,), "Q5_1"
 
 
 @pytest.mark.parametrize("H,E,K,I,T,g,d,sg,sd", [
-    (2560, 16, 4, 640, 83, "Q4_K", "Q5_1", "Q8_0", "Q8_0"),
-    (512, 8, 4, 640, 67, "Q5_K", "Q8_0", "Q8_0", "Q8_0"),
-    (2048, 16, 4, 512, 180, "Q4_K", "Q6_K", "Q4_K", "Q6_K"),
+    (2560, 16, 4, 640, 400, "Q4_K", "Q5_1", "Q8_0", "Q8_0"),
+    (512, 8, 4, 640, 375, "Q5_K", "Q8_0", "Q8_0", "Q8_0"),
+    (2048, 16, 4, 512, 400, "Q4_K", "Q6_K", "Q4_K", "Q6_K"),
 ], ids=["q4k-q5_1", "q5k-q8_0", "q4k-q6_k"])
 def test_moe_prefill_many_fails_closed(ctx, H, E, K, I, T, g, d, sg, sd):
-    # 20 and more tokens per expert: a non-finite scale in the last block of
+    # the 64-token products: a non-finite scale in the last block of
     # each role, a non-finite activation of the last token and products past
     # binary32 fail the call; a good call after them gives what one gave before
     seed = S.W_MOE + 7100 + H
@@ -762,10 +762,9 @@ def test_moe_prefill_many_fails_closed(ctx, H, E, K, I, T, g, d, sg, sd):
 
 
 def test_moe_prefill_many_shared_sums(ctx):
-    # The shared expert's 2560 columns where 20 and more tokens meet each
-    # expert: its sums err by 2.2e-7 of the output, the three products and the
+    # The shared expert's 2560 columns in the 64-token products: its sums err by 2.2e-7 of the output, the three products and the
     # gate together; 3.0e-7 where a row's 80 blocks are one sum.
-    H, E, K, I, T = 2560, 8, 4, 640, 130
+    H, E, K, I, T = 2560, 8, 4, 640, 375
     seed = S.W_MOE + 7200
     w = S.moe_weights(seed, H, E, I, I, gate_fmt="Q4_K", down_fmt="Q5_1", shared_gate_fmt="Q8_0",
                       shared_down_fmt="Q8_0")
