@@ -1384,8 +1384,11 @@ __global__ __launch_bounds__(1024) void route_select(RouteArgs a) {
  * rounding errors dw (their 2-norm is formed, a third of the 2^-11 |w| it
  * could be), 2^-21 s for the tokens' split, and by its fp32 accumulation: two
  * steps of 32 products per 32 columns, each at most 32 2^-24 of its own terms
- * and 2^-23 of the running sum off, at most (2^-18 + n 2^-27) s; n 2^-25 s is
- * taken. Together |dw| |x| + (2^-21 + 1.5 n 2^-24) s; B takes 1.02 of that,
+ * and 2^-23 of the running sum off (what binary32 additions in any order, cut or
+ * rounded, allow; no public document states it for the matrix cores, and
+ * test_mfma_step_error and test_mfma_chain_error measure it on worst cases: a
+ * large first term, cancelling ones, one sign), at most (2^-18 + n 2^-27) s; n
+ * 2^-25 s is taken. Together |dw| |x| + (2^-21 + 1.5 n 2^-24) s; B takes 1.02 of that,
  * plus 2^-20 |a| for the binary32 arithmetic on a and B, plus 1e-37 for
  * underflow.
  */

@@ -416,10 +416,9 @@ def test_matvec_fails_closed(ctx):
     (65536, 256, 2, 1.0), (70001, 2048, 3, 1.0), (65537, 4096, 4, 1e-30),
     (66000, 1024, 2, 1e6), (65600, 512, 4, 1.0), (65551, 2048, 4, 1.0)])
 def test_matvec_q6k_batched_mfma(ctx, rows, cols, batch, scale):
-    # Q6_K with 2..4 activation columns on at least 65,536 rows runs on
-    # MFMA (exact fp16 codes, activation columns as fp16 hi + lo after a
-    # power-of-two scaling): ragged last tiles, 1 .. 16 blocks per row, tiny
-    # and large activations (compared relative to their scale)
+    # Q6_K heads of 2..4 activation columns (on the matrix-core tiles but for
+    # 1,024 columns at 2): ragged last tiles, 1 .. 16 blocks per row, tiny and
+    # large activations (compared relative to their scale)
     say(f"q6k mfma {rows}x{cols} batch {batch} scale {scale}")
     key = S.stream_key(S.W_MATVEC_Q6K, rows, cols, batch)
     w = S.quant_matrix("Q6_K", key, rows, cols)
@@ -437,8 +436,7 @@ def test_matvec_q6k_batched_mfma(ctx, rows, cols, batch, scale):
 
 @pytest.mark.parametrize("cols", [256, 2048])
 def test_matvec_q6k_batched_mfma_fails_closed(ctx, cols):
-    # 2,048 columns run on the tile-shared kernel, the other widths on the
-    # per-wave block rings
+    # one unit of 256 columns, and one a wave of eight
     rows = 65536
     w = S.quant_matrix("Q6_K", S.stream_key(S.W_MATVEC_Q6K, 91), rows, cols)
     x = S.normal_f32(S.stream_key(S.W_MATVEC_Q6K, 92), 2 * cols).reshape(2, cols)
@@ -611,6 +609,72 @@ def test_matvec_tiles_fails_closed(ctx, fmt, cols, field):
         b.close()
 
 
+@pytest.mark.parametrize("kind", ["large first", "cancelling", "spread", "one sign"])
+def test_mfma_step_error(ctx, kind):
+    # What the routing of several tokens takes of one 16x16x32 fp16 step (the
+    # bound at route_prep): its 32 products are exact in binary32, and their
+    # sum is off by at most 32 2^-24 of the products' magnitudes, in whatever
+    # order they are added and however the bits below are cut. Seen through
+    # Q8_0 rows with scale 1 on the tiles, where a row's first block is one
+    # step; activations of 11 bits make the other parts of the operand zero.
+    rows, batch, cols = 4096, 4, 64
+    rng = np.random.default_rng(len(kind))
+    q = rng.integers(-127, 128, (rows, 2, 32))
+    x = np.ldexp(rng.integers(1024, 2048, (batch, 2, 32)).astype(np.float64),
+                 0 if kind == "one sign" else rng.integers(-10, 1, (batch, 2, 32)))
+    x *= rng.choice([-1.0, 1.0], x.shape)
+    x[:, 1] = 0.0
+    if kind == "large first":
+        x[:, 0, 0], q[:, 0, 0] = 2047.0, 127
+    elif kind == "cancelling":
+        x[:, 0, 16:], q[:, 0, 16:] = -x[:, 0, :16], q[:, 0, :16]
+        x[:, 0, 31] = 2.0 ** -9
+    elif kind == "one sign":
+        x, q = np.abs(x), np.abs(q)
+    blocks = np.zeros((rows, 2, 34), np.uint8)
+    blocks[:, :, :2] = np.array([1.0], np.float16).view(np.uint8)
+    blocks[:, :, 2:] = q.astype(np.int8).view(np.uint8)
+    xf = x.reshape(batch, cols).astype(np.float32)
+    dw, dx, dy = ctx.upload(blocks.reshape(-1)), ctx.upload(xf), ctx.alloc(rows * batch * 4)
+    ctx.matvec(kq_hip.TYPE_Q8_0, dw, rows, cols, dx, batch, dy)
+    got = ctx.download(dy, np.float32, rows * batch).reshape(batch, rows).astype(np.float64)
+    for b in (dw, dx, dy):
+        b.close()
+    terms = x.reshape(batch, 1, cols) * q.reshape(1, rows, cols)
+    assert (np.abs(got - terms.sum(2)) <= 32 * 2.0 ** -24 * np.abs(terms).sum(2)).all()
+
+
+@pytest.mark.parametrize("kind", ["large first", "spread", "one sign"])
+def test_mfma_chain_error(ctx, kind):
+    # and of a chain of steps: each adds at most 2^-23 of the accumulator to
+    # that. A Q4_K unit is eight steps in one accumulator; scales 1 and mins 0
+    # make its weights the codes (48: 32 of the terms, 2 of at most their
+    # whole sum for each step).
+    rows, batch, cols = 2304, 4, 256
+    rng = np.random.default_rng(len(kind))
+    q = rng.integers(0, 16, (rows, cols))
+    x = np.ldexp(rng.integers(1024, 2048, (batch, cols)).astype(np.float64),
+                 0 if kind == "one sign" else rng.integers(-10, 1, (batch, cols)))
+    if kind != "one sign":
+        x *= rng.choice([-1.0, 1.0], x.shape)
+    if kind == "large first":
+        x[:, ::64], q[:, ::64] = 2047.0, 15
+    blocks = np.zeros((rows, 144), np.uint8)
+    blocks[:, :2] = np.array([1.0], np.float16).view(np.uint8)
+    blocks[:, 4:8] = 1   # scales of sub-blocks 0 .. 3
+    blocks[:, 12:16] = 1  # and 4 .. 7
+    c = q.reshape(rows, 4, 2, 32)
+    blocks[:, 16:] = (c[:, :, 0] | c[:, :, 1] << 4).reshape(rows, 128)
+    dw, dx = ctx.upload(blocks.reshape(-1)), ctx.upload(x.astype(np.float32))
+    dy = ctx.alloc(rows * batch * 4)
+    ctx.matvec(kq_hip.TYPE_Q4_K, dw, rows, cols, dx, batch, dy)
+    got = ctx.download(dy, np.float32, rows * batch).reshape(batch, rows).astype(np.float64)
+    for b in (dw, dx, dy):
+        b.close()
+    terms = x.reshape(batch, 1, cols) * q.reshape(1, rows, cols)
+    assert (np.abs(got - terms.sum(2)) <= 48 * 2.0 ** -24 * np.abs(terms).sum(2)).all()
+
+
 def test_argmax_exact(ctx):
     rng = np.random.default_rng(9)
     v = rng.standard_normal((3, 151936)).astype(np.float32)
@@ -687,22 +751,27 @@ def test_lm_head_q8_0_248320x2560(ctx):
         b.close()
 
 
-@pytest.mark.parametrize("V,batch", [(40000, 5), (40000, 6), (40000, 8), (65600, 5)])
-def test_lm_head_batch_spans_launches(ctx, V, batch):
-    # batches over 4 run as several launches whose wave counts differ (at
-    # 65,600 rows the first four columns run on MFMA, the fifth on the row
-    # engine); the argmax partials of every batch row must still merge to
-    # the first max
-    H = 2048
-    say(f"lm head {V}x{H} batch {batch}")
-    w = S.quant_matrix("Q6_K", S.stream_key(S.W_LM_HEAD, S.R_WEIGHT, 7), V, H)
+@pytest.mark.parametrize("fmt,V,H,batch", [("Q6_K", 40000, 2048, b) for b in (5, 6, 8)] + [
+    ("Q6_K", 65600, 2048, 5), ("Q4_K", 9000, 12288, 5), ("Q6_K", 5001, 12288, 8),
+    ("Q8_0", 40000, 96, 5), ("IQ4_NL", 20001, 32, 8), ("Q5_K", 30000, 6144, 5),
+    ("Q5_1", 9001, 5120, 7)])
+def test_lm_head_batch_spans_launches(ctx, fmt, V, H, batch):
+    # batches over 4 as one launch (Q6_K, 2048 columns), and as several whose
+    # partial counts differ: rows of more than 10,240 columns, or off a dword,
+    # which the matrix-core tiles refuse, on the row engine; four columns on
+    # the tiles and the rest on either where more than four columns of
+    # binary32 operands would not fit (above 4,096 columns). The argmax
+    # partials of every batch row must merge to the first max.
+    say(f"lm head {fmt} {V}x{H} batch {batch}")
+    t = FMTS[fmt]
+    w = S.quant_matrix(fmt, S.stream_key(S.W_LM_HEAD, S.R_WEIGHT, 7), V, H)
     h = S.normal_f32(S.stream_key(S.W_LM_HEAD, S.R_HIDDEN, 70 + batch), batch * H).reshape(batch, H)
     dw, dh = ctx.upload(w), ctx.upload(h)
     dl, di = ctx.alloc(V * batch * 4), ctx.alloc(batch * 4)
-    ctx.lm_head(kq_hip.TYPE_Q6_K, dw, V, H, dh, batch, dl, di)
+    ctx.lm_head(t, dw, V, H, dh, batch, dl, di)
     logits = ctx.download(dl, np.float32, V * batch).reshape(batch, V)
     ids = ctx.download(di, np.uint32, batch)
-    ref = kq_oracle.matvec(kq_oracle.Q6_K, w, V, H, h, threads=oracle_threads())
-    assert_close(logits, ref, exact=exact.matvec(kq_oracle.Q6_K, w, V, H, h))
+    ref = kq_oracle.matvec(t, w, V, H, h, threads=oracle_threads())
+    assert_close(logits, ref, exact=exact.matvec(t, w, V, H, h))
     for b in range(batch):
         assert ids[b] == int(np.argmax(logits[b]))
