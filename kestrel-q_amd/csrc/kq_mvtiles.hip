@@ -130,14 +130,22 @@ constexpr uint32_t columns_of(Rows m) { return m == kQuad ? 4u : 8u; }
 constexpr uint32_t operands_of(Rows m) { return m == kEight ? 2u : 1u; }
 
 /* What the operands take, in the scaled values (largest in [2^14, 2^15)). Four
- * parts hold a value as binary32 does down to least_value(), two the values of
- * 8 columns as a scale per 16 does if one of them reaches least_group(); so do
- * four parts the sums of such columns, which are scaled down again. Anything
- * smaller but zeros goes to the binary32 rows. */
-constexpr float least_value() { return 0x1p-25f; }
+ * parts hold a value as binary32 does down to least_value() (asked of the
+ * formats that the row engine multiplies so). 16 columns are held as a scale of
+ * their own holds them if one reaches least_group(): two parts are off by 2^-25,
+ * four by 2^-49, the scale by 2^-23 of their largest; and the sums of such
+ * columns, which are scaled down again, if one does. Anything smaller but zeros
+ * goes to the binary32 rows. (Asked of single values, the 320 SiLU outputs of a
+ * saturated rank projection went there in most calls: 20 us more on the 68 of a
+ * one-token block.) */
+template <uint32_t FMT, Rows M>
+constexpr float least_value() {
+    return M == kQuad && !is_binary32(FMT) ? 0.0f : 0x1p-25f; /* kPair: not looked at */
+}
 template <uint32_t FMT, Rows M>
 constexpr float least_group() {
-    return M == kPair ? 0x1p-2f : is_k(FMT) ? 0x1p-20f : FMT == KQ_LAUNCH_Q5_1 ? 0x1p-16f : 0.0f;
+    return M == kPair ? 0x1p-2f : is_k(FMT) ? 0x1p-20f : FMT == KQ_LAUNCH_Q5_1 ? 0x1p-16f
+                      : is_binary32(FMT) ? 0.0f : 0x1p-25f;
 }
 
 /* The column of its unit that lane k-group g's element e of operand step s
@@ -551,17 +559,28 @@ __global__ __launch_bounds__((max_threads<NC, M>())) void mv_tiles(MvtArgs a) {
             for (uint32_t k = 0; k < NV; ++k) {
                 const uint32_t mx = mag(v[k].x), my = mag(v[k].y), mz = mag(v[k].z), mw = mag(v[k].w);
                 gm[k] = max(max(mx, my), max(mz, mw));
-                if constexpr (M != kPair) {
+                if constexpr (M != kPair && least_value<FMT, M>() != 0.0f) {
                     value1 = min(min(value1, mx - 1u), my - 1u);
                     value1 = min(min(value1, mz - 1u), mw - 1u);
                 }
             }
             if constexpr (least_group<FMT, M>() != 0.0f) {
-                /* a group: half a step; Q6_K, four elements of two k-groups */
+                /* a group. kQuad: 16 columns, a lane's (K formats), four
+                 * elements of each k-group (Q6_K) or half a step of k-groups g
+                 * and g ^ 1; else 8 of them, half a step or, Q6_K, four elements
+                 * of two k-groups (the other 8 beside them cost registers that
+                 * the widest rows do not have) */
+                constexpr uint32_t N = FMT == KQ_LAUNCH_Q6_K ? 1u : is_k(FMT) ? 4u : 2u;
 #pragma unroll
                 for (uint32_t k = 0; k < NV; ++k) {
                     if constexpr (M == kQuad) {
-                        if (k & 1u) group1 = min(group1, max(gm[k - 1u], gm[k]) - 1u);
+                        if (k % N != 0u) continue;
+                        uint32_t gk = gm[k];
+#pragma unroll
+                        for (uint32_t n = 1; n < N; ++n) gk = max(gk, gm[k + n]);
+                        if constexpr (FMT == KQ_LAUNCH_Q6_K) gk = max_groups(gk);
+                        else if constexpr (!is_k(FMT)) gk = max16(gk);
+                        group1 = min(group1, gk - 1u);
                     } else {
                         gm[k] = FMT == KQ_LAUNCH_Q6_K ? max16(gm[k]) : max(gm[k], ror8(gm[k]));
                         group1 = min(group1, gm[k] - 1u);
@@ -579,7 +598,7 @@ __global__ __launch_bounds__((max_threads<NC, M>())) void mv_tiles(MvtArgs a) {
             bad |= nf;
             const int sig = !nf && m != 0u ? 15 - __builtin_amdgcn_frexp_expf(__uint_as_float(m)) : 0;
             auto below = [&](float scaled) { return max(mag(ldexpf(scaled, -sig)), 1u) - 1u; };
-            deep |= !nf && (value1 < below(least_value()) || group1 < below(least_group<FMT, M>()));
+            deep |= !nf && (value1 < below(least_value<FMT, M>()) || group1 < below(least_group<FMT, M>()));
             if (g == 0u && (M == kQuad ? q == 0u : i < KC)) sigs[(c * nw + w) * KC + col] = sig;
             float run[2] = {0.0f, 0.0f}, by_step[NV]; /* sums over this lane's values */
             uint32_t own[4][4]; /* kQuad: a step's [part][dword] */
