@@ -43,7 +43,7 @@
  *
  * Bound: HBM for matrices that fill the device, the first loads' latency
  * and the operand's build below that. Against the row engine: 10240 x 2560
- * Q8_0 at 8 columns 76.7 -> 11.9 us (2.4 TB/s), the 248320 x 2560 Q8_0 head
+ * Q8_0 at 8 columns 76.7 -> 12.3 us (2.3 TB/s), the 248320 x 2560 Q8_0 head
  * at 5 columns 273 -> 136 us (5.0 TB/s). Two operands keep one workgroup per
  * CU: 40000 x 2048 at 8 columns, Q5_K 23 us (row engine 53), Q5_1 37
  * (46). Error against binary64 sums of normal
