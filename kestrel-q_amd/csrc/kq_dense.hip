@@ -25,28 +25,15 @@
  */
 #include "kq_device.h"
 #include "kq_launch.h"
+#include "kq_mfma.h"
 
 namespace {
 
-typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-typedef float f4 __attribute__((ext_vector_type(4)));
+using namespace kq::mf;
 
 constexpr uint32_t kTile = 16;
 constexpr uint32_t kWaves = 4;
 constexpr int kBadRow = 0x7fffffff;
-constexpr uint32_t kMagic = 0x64646464u; /* fp16 0x64XX = 1024 + XX */
-
-__device__ __forceinline__ h2 as_h2(uint32_t u) { return __builtin_bit_cast(h2, u); }
-__device__ __forceinline__ h2 bytes_lo(uint32_t m) {
-    return as_h2(__builtin_amdgcn_perm(kMagic, m, 0x04010400u));
-}
-__device__ __forceinline__ h2 bytes_hi(uint32_t m) {
-    return as_h2(__builtin_amdgcn_perm(kMagic, m, 0x04030402u));
-}
-__device__ __forceinline__ float f16f(uint32_t h) {
-    return (float)__builtin_bit_cast(_Float16, (unsigned short)(h & 0xffffu));
-}
 
 /* Row t of X [tokens][k] (k a multiple of 4): sig[t] and the scaled row as
  * fp16 hi + lo in xh, xl [tokens][k]; a row with a non-finite value is
@@ -204,7 +191,7 @@ __global__ __launch_bounds__(kWaves * 64) void dense_q8(DenseArgs a) {
                     f4 t = {0.f, 0.f, 0.f, 0.f};
                     t = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bv, t, 0, 0, 0);
                     t = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, bv, t, 0, 0, 0);
-                    const float d = f16f(bb ? s.w[m][i].d[bb] >> 16 : s.w[m][i].d[bb]);
+                    const float d = half_bits(bb ? s.w[m][i].d[bb] >> 16 : s.w[m][i].d[bb]);
                     malformed |= !kq_isfinite(d);
 #pragma unroll
                     for (int q = 0; q < 4; ++q) acc[m][i][q] = fmaf(d, t[q], acc[m][i][q]);

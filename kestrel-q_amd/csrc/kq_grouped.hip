@@ -47,34 +47,15 @@
 #include "kq_stage.h"
 #include "kq_device.h"
 #include "kq_dma.h"
+#include "kq_mfma.h"
 
 namespace {
 
-typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-typedef float f4 __attribute__((ext_vector_type(4)));
+using namespace kq::mf;
 
 constexpr uint32_t kTile = 16;          /* tokens per M-chunk, rows per N-tile */
-constexpr uint32_t kMagic = 0x64646464u; /* fp16 0x64XX = 1024 + XX */
 
-__device__ __forceinline__ h2 as_h2(uint32_t u) { return __builtin_bit_cast(h2, u); }
 __device__ __forceinline__ uint32_t as_u(h2 v) { return __builtin_bit_cast(uint32_t, v); }
-
-/* bytes b0, b1 (sel 0x04010400) or b2, b3 (sel 0x04030402) of m as fp16
- * 1024 + byte */
-__device__ __forceinline__ h2 bytes_lo(uint32_t m) {
-    return as_h2(__builtin_amdgcn_perm(kMagic, m, 0x04010400u));
-}
-__device__ __forceinline__ h2 bytes_hi(uint32_t m) {
-    return as_h2(__builtin_amdgcn_perm(kMagic, m, 0x04030402u));
-}
-
-__device__ __forceinline__ h2 fma2(h2 a, h2 b, h2 c) { return __builtin_elementwise_fma(a, b, c); }
-
-__device__ __forceinline__ float f16f(uint32_t h) {
-    return (float)__builtin_bit_cast(_Float16, (unsigned short)(h & 0xffffu));
-}
 
 __device__ __forceinline__ float wave_max_abs(float v) {
 #pragma unroll
@@ -348,8 +329,8 @@ struct Tile<KQ_LAUNCH_Q4_K, KDIM, NMAT> {
         h4 bm[NMAT];
 #pragma unroll
         for (int m = 0; m < NMAT; ++m) {
-            d[m] = f16f(r[m].hd.x);
-            const float dmin = f16f(r[m].hd.x >> 16);
+            d[m] = half_bits(r[m].hd.x);
+            const float dmin = half_bits(r[m].hd.x >> 16);
             malformed |= !kq_isfinite(d[m]) || !kq_isfinite(dmin);
             dm[m] = dmin * 32.0f; /* the activation sums carry 2^-5 */
             /* scales of sub-blocks 2g and 2g+1 (src/kq_numeric.c:161-174) */
@@ -435,7 +416,7 @@ struct Tile<KQ_LAUNCH_Q6_K, KDIM, NMAT> {
         uint32_t sc[NMAT][4];
 #pragma unroll
         for (int m = 0; m < NMAT; ++m) {
-            d[m] = f16f(r[m].d);
+            d[m] = half_bits(r[m].d);
             malformed |= !kq_isfinite(d[m]);
             const uint32_t sh = r[m].sh ? 2u : 0u;
             sc[m][0] = kq_align2(r[m].sc.y, r[m].sc.x, sh);
@@ -523,7 +504,7 @@ struct Tile<KQ_LAUNCH_Q8_0, KSL, NMAT> {
                 f4 t = {0.f, 0.f, 0.f, 0.f};
                 t = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bw, t, 0, 0, 0);
                 t = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, bw, t, 0, 0, 0);
-                const float d = f16f((bb & 1u) ? r[m].d[bb] >> 16 : r[m].d[bb]);
+                const float d = half_bits((bb & 1u) ? r[m].d[bb] >> 16 : r[m].d[bb]);
                 malformed |= !kq_isfinite(d);
 #pragma unroll
                 for (int k = 0; k < 4; ++k) acc[m][k] = fmaf(d, t[k], acc[m][k]);
@@ -538,11 +519,6 @@ struct Tile<KQ_LAUNCH_Q5_1, KSL, NMAT> {
     using F = Fmt<KQ_LAUNCH_Q5_1>;
     using S = Stage<KQ_LAUNCH_Q5_1, KSL>;
     using Raw = F::Raw;
-
-    /* bit k of x (k < 4) to bit 8k + 4: the fifth bit of four codes */
-    __device__ static __forceinline__ uint32_t spread4(uint32_t x) {
-        return (kq_mul_u24(x, 0x00204081u) & 0x01010101u) << 4;
-    }
 
     /* iteration b: blocks 4b .. 4b + 3 of the slice; codes 0..31 are
      * exact in fp16, d scales the step and m the block's activation sum */
@@ -576,7 +552,7 @@ struct Tile<KQ_LAUNCH_Q5_1, KSL, NMAT> {
                 f4 t = {0.f, 0.f, 0.f, 0.f};
                 t = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bw, t, 0, 0, 0);
                 t = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, bw, t, 0, 0, 0);
-                const float d = f16f(r[m].dm[bb]), mn = f16f(r[m].dm[bb] >> 16);
+                const float d = half_bits(r[m].dm[bb]), mn = half_bits(r[m].dm[bb] >> 16);
                 malformed |= !kq_isfinite(d) || !kq_isfinite(mn);
                 const float m32 = mn * 32.0f; /* the sums carry 2^-5 */
 #pragma unroll

@@ -33,29 +33,17 @@
 #include "kq_launch.h"
 #include "kq_device.h"
 #include "kq_dma.h"
+#include "kq_mfma.h"
 
 namespace {
 
-typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-typedef float f4 __attribute__((ext_vector_type(4)));
+using namespace kq::mf;
+
 typedef kq_i4v i4v;
 
 constexpr uint32_t kT = 16;
 constexpr uint32_t kShared = 0x80000000u; /* item flag: the shared expert */
 constexpr int kBadRow = 0x7fffffff;
-
-__device__ __forceinline__ h2 as_h2(uint32_t u) { return __builtin_bit_cast(h2, u); }
-__device__ __forceinline__ h2 byte_pair_lo(uint32_t m) {
-    return as_h2(__builtin_amdgcn_perm(0x64646464u, m, 0x04010400u));
-}
-__device__ __forceinline__ h2 byte_pair_hi(uint32_t m) {
-    return as_h2(__builtin_amdgcn_perm(0x64646464u, m, 0x04030402u));
-}
-__device__ __forceinline__ float half_bits(uint32_t h) {
-    return (float)__builtin_bit_cast(_Float16, (uint16_t)(h & 0xffffu));
-}
 
 __device__ __forceinline__ uint32_t sload(const uint32_t *p) {
     const uint64_t a = (uint64_t)(uintptr_t)p;
@@ -294,7 +282,7 @@ void dn_q6k(DnArgs a) {
 #pragma unroll
                 for (uint32_t q = 0; q < 4u; ++q) {
                     const uint32_t s = 8u * n + 2u * q + h; /* sub-block */
-                    const h2 w0 = byte_pair_lo(c[q]) + bias, w1 = byte_pair_hi(c[q]) + bias;
+                    const h2 w0 = bytes_lo(c[q]) + bias, w1 = bytes_hi(c[q]) + bias;
                     const h4 bw = h4{w0.x, w0.y, w1.x, w1.y};
                     /* columns 128n + 32q + 16h + 4g .. +3 of block b */
                     const uint32_t ai = (n * 2u + h) * 4u + q;
@@ -594,7 +582,7 @@ void dn_q6k_pair(DnArgs a) {
 #pragma unroll
                 for (uint32_t q = 0; q < 4u; ++q) {
                     const uint32_t s = 8u * n + 2u * q + hh; /* sub-block */
-                    const h2 w0 = byte_pair_lo(c[q]) + bias, w1 = byte_pair_hi(c[q]) + bias;
+                    const h2 w0 = bytes_lo(c[q]) + bias, w1 = bytes_hi(c[q]) + bias;
                     const h4 bw = h4{w0.x, w0.y, w1.x, w1.y};
                     /* columns 128n + 32q + 16hh + 4g .. +3 of block h */
                     const uint32_t ai = (n * 2u + hh) * 4u + q;
@@ -644,11 +632,6 @@ struct DnSmallShape {
     static_assert(RB % 4u == 0u, "rows start 4-byte aligned in the slot");
     static constexpr uint32_t TB = kT * RB;                  /* tile bytes */
 };
-
-/* bits 0..3 of x (x < 16) to bit 4 of bytes 0..3 */
-__device__ __forceinline__ uint32_t spread4(uint32_t x) {
-    return (kq_mul_u24(x, 0x00204081u) & 0x01010101u) << 4;
-}
 
 /* The Q5_1 / Q8_0 down pass on pairs of waves, as dn_q6k_pair: wave h of a
  * pair multiplies blocks h NH .. h NH + NH - 1 of every row (NH = blocks per
@@ -890,8 +873,8 @@ void dn_small_pair(DnArgs a) {
                 }
                 malformed |= !kq_isfinite(d);
             }
-            const h2 w0 = byte_pair_lo(c0) + bias, w1 = byte_pair_hi(c0) + bias;
-            const h2 w2 = byte_pair_lo(c1) + bias, w3 = byte_pair_hi(c1) + bias;
+            const h2 w0 = bytes_lo(c0) + bias, w1 = bytes_hi(c0) + bias;
+            const h2 w2 = bytes_lo(c1) + bias, w3 = bytes_hi(c1) + bias;
             const h8 bw = h8{w0.x, w0.y, w1.x, w1.y, w2.x, w2.y, w3.x, w3.y};
             const h8 ah = __builtin_bit_cast(h8, axh[b]), al = __builtin_bit_cast(h8, axl[b]);
             f4 t = {0.f, 0.f, 0.f, 0.f};

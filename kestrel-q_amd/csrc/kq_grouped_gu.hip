@@ -55,29 +55,15 @@
 #include "kq_stage.h"
 #include "kq_device.h"
 #include "kq_dma.h"
+#include "kq_mfma.h"
 
 namespace {
 
-typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-typedef float f4 __attribute__((ext_vector_type(4)));
+using namespace kq::mf;
+
 typedef kq_i4v i4v;
 
 constexpr uint32_t kT = 16; /* tokens per chunk, rows per tile */
-
-__device__ __forceinline__ h2 as_h2(uint32_t u) { return __builtin_bit_cast(h2, u); }
-/* bytes b0, b1 / b2, b3 of m as fp16 0x64XX = 1024 + XX */
-__device__ __forceinline__ h2 byte_pair_lo(uint32_t m) {
-    return as_h2(__builtin_amdgcn_perm(0x64646464u, m, 0x04010400u));
-}
-__device__ __forceinline__ h2 byte_pair_hi(uint32_t m) {
-    return as_h2(__builtin_amdgcn_perm(0x64646464u, m, 0x04030402u));
-}
-__device__ __forceinline__ h2 fma2(h2 a, h2 b, h2 c) { return __builtin_elementwise_fma(a, b, c); }
-__device__ __forceinline__ float half_bits(uint32_t h) {
-    return (float)__builtin_bit_cast(_Float16, (uint16_t)(h & 0xffffu));
-}
 
 /* ------------------------------------------------------------------ */
 /* per-token activation split */
@@ -398,8 +384,8 @@ __global__ __launch_bounds__(NB * WPB * 64) void gu_kq(GuArgs a) {
                                     ((((hd[m].w >> 4) & 0x0f0f0f0fu) | ((hd[m].z >> 2) & 0x30303030u)) & ~k0);
                 const h2 one = h2{(_Float16)1.0f, (_Float16)1.0f};
                 const h2 neg = h2{(_Float16)-1024.0f, (_Float16)-1024.0f};
-                const uint32_t mlo = __builtin_bit_cast(uint32_t, fma2(byte_pair_lo(mq), one, neg)) & k01;
-                const uint32_t mhi = __builtin_bit_cast(uint32_t, fma2(byte_pair_hi(mq), one, neg)) & k01;
+                const uint32_t mlo = __builtin_bit_cast(uint32_t, fma2(bytes_lo(mq), one, neg)) & k01;
+                const uint32_t mhi = __builtin_bit_cast(uint32_t, fma2(bytes_hi(mq), one, neg)) & k01;
                 bm[m] = __builtin_bit_cast(h4, make_uint2(mlo, mhi));
             }
             f4 qacc[NM];
@@ -428,8 +414,8 @@ __global__ __launch_bounds__(NB * WPB * 64) void gu_kq(GuArgs a) {
                         m1 = s < 4u ? kq_and_0f(raw1) : kq_and_f0(raw1);
                     }
                     const h2 Sc = s < 4u ? S0[m] : S1[m], Cc = s < 4u ? C0[m] : C1[m];
-                    const h2 w0 = fma2(byte_pair_lo(m0), Sc, Cc), w1 = fma2(byte_pair_hi(m0), Sc, Cc);
-                    const h2 w2 = fma2(byte_pair_lo(m1), Sc, Cc), w3 = fma2(byte_pair_hi(m1), Sc, Cc);
+                    const h2 w0 = fma2(bytes_lo(m0), Sc, Cc), w1 = fma2(bytes_hi(m0), Sc, Cc);
+                    const h2 w2 = fma2(bytes_lo(m1), Sc, Cc), w3 = fma2(bytes_hi(m1), Sc, Cc);
                     const h8 bw = h8{w0.x, w0.y, w1.x, w1.y, w2.x, w2.y, w3.x, w3.y};
                     qacc[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[s], bw, qacc[m], 0, 0, 0);
                     qacc[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[s], bw, qacc[m], 0, 0, 0);
@@ -680,8 +666,8 @@ __global__ __launch_bounds__(NB * 64) void gu_mix(GuArgs a) {
                             ((((hd.w >> 4) & 0x0f0f0f0fu) | ((hd.z >> 2) & 0x30303030u)) & ~k0);
         const h2 one = h2{(_Float16)1.0f, (_Float16)1.0f};
         const h2 neg = h2{(_Float16)-1024.0f, (_Float16)-1024.0f};
-        const uint32_t mlo = __builtin_bit_cast(uint32_t, fma2(byte_pair_lo(mq), one, neg)) & k01;
-        const uint32_t mhi = __builtin_bit_cast(uint32_t, fma2(byte_pair_hi(mq), one, neg)) & k01;
+        const uint32_t mlo = __builtin_bit_cast(uint32_t, fma2(bytes_lo(mq), one, neg)) & k01;
+        const uint32_t mhi = __builtin_bit_cast(uint32_t, fma2(bytes_hi(mq), one, neg)) & k01;
         const h4 bm = __builtin_bit_cast(h4, make_uint2(mlo, mhi));
         f4 qacc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -702,8 +688,8 @@ __global__ __launch_bounds__(NB * 64) void gu_mix(GuArgs a) {
                 m1 = s < 4u ? kq_and_0f(raw1) : kq_and_f0(raw1);
             }
             const h2 Sc = s < 4u ? S0 : S1, Cc = s < 4u ? C0 : C1;
-            const h2 w0 = fma2(byte_pair_lo(m0), Sc, Cc), w1 = fma2(byte_pair_hi(m0), Sc, Cc);
-            const h2 w2 = fma2(byte_pair_lo(m1), Sc, Cc), w3 = fma2(byte_pair_hi(m1), Sc, Cc);
+            const h2 w0 = fma2(bytes_lo(m0), Sc, Cc), w1 = fma2(bytes_hi(m0), Sc, Cc);
+            const h2 w2 = fma2(bytes_lo(m1), Sc, Cc), w3 = fma2(bytes_hi(m1), Sc, Cc);
             const h8 bw = h8{w0.x, w0.y, w1.x, w1.y, w2.x, w2.y, w3.x, w3.y};
             qacc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[s], bw, qacc, 0, 0, 0);
             qacc = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[s], bw, qacc, 0, 0, 0);
